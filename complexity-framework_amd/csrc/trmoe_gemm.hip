@@ -9,7 +9,6 @@
 //                      expert rows through `inverse` and applies the route
 //                      weights and branch scales (engine.py:509-531, 578)
 //   k_combine          the epilogue alone, for shared_width == 0
-//   k_pack             weight re-layout into the K-contiguous packed form
 #include "trmoe_common.h"
 #include "trmoe_internal.h"
 #include "trmoe_gemm.h"
@@ -22,56 +21,6 @@
 #include <type_traits>
 
 namespace trmoe {
-
-// ---------------------------------------------------------------------------
-// packing
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_pack(PackArgs p) {
-    const int64_t total = p.groups * p.dst_rows * p.dst_cols;
-    for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total;
-         idx += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t col = idx % p.dst_cols;
-        const int64_t rowg = idx / p.dst_cols;
-        const int64_t row = rowg % p.dst_rows;
-        const int64_t g = rowg / p.dst_rows;
-        int64_t feat;
-        const char* src;
-        const float* ssrc;
-        if (p.interleave) {
-            const int64_t blk = row >> 6, w = row & 63;
-            feat = blk * 32 + (w & 31);
-            src = (w >= 32) ? (const char*)p.b : (const char*)p.a;
-            ssrc = (w >= 32) ? p.sb : p.sa;
-        } else {
-            feat = row;
-            src = (const char*)p.a;
-            ssrc = p.sa;
-        }
-        const bool valid = feat < p.out_features && col < p.in_features;
-        const int64_t s = g * p.s_group + feat * p.s_out + col * p.s_in;
-        char* d = (char*)p.dst + (g * p.dst_group_stride + row * p.dst_ld + col) * p.elem_bytes;
-        if (p.elem_bytes == 1) {
-            *(uint8_t*)d = valid ? ((const uint8_t*)src)[s] : 0;
-        } else if (p.elem_bytes == 2) {
-            *(uint16_t*)d = valid ? ((const uint16_t*)src)[s] : 0;
-        } else {
-            *(uint32_t*)d = valid ? ((const uint32_t*)src)[s] : 0;
-        }
-        if (p.dst_scale != nullptr && col == 0) {
-            const bool fv = feat < p.out_features;
-            p.dst_scale[g * p.dst_scale_group_stride + row] = fv ? ssrc[g * p.scale_group_stride + feat] : 0.0f;
-        }
-    }
-}
-
-int launch_pack(const PackArgs& p, hipStream_t stream) {
-    const int64_t total = p.groups * p.dst_rows * p.dst_cols;
-    int64_t blocks = (total + 255) / 256;
-    if (blocks > 65536) blocks = 65536;
-    if (blocks < 1) blocks = 1;
-    hipLaunchKernelGGL(k_pack, dim3((unsigned)blocks), dim3(256), 0, stream, p);
-    return check_launch("pack_weight");
-}
 
 // ---------------------------------------------------------------------------
 // K2: shared gate|up + SwiGLU
