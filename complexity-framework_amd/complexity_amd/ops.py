@@ -573,6 +573,84 @@ def pack_fragments(w_packed: torch.Tensor, cols: int) -> tuple:
     return dst, int(cols)
 
 
+@dataclass
+class E4M3Decode:
+    """Decode-sized weights of an e4m3 layer: the shared branch and every
+    expert concatenated, fragment-major, with their scales."""
+
+    gate_up: torch.Tensor
+    gate_up_scale: torch.Tensor
+    down: torch.Tensor
+    down_scale: torch.Tensor   # [1 + E, round_up(H, 256)]
+
+
+@_on_tensor_device
+def pack_e4m3_decode(packed: "PackedLayer", hidden: int) -> E4M3Decode:
+    """trmoe_pack_fragments_e4m3 of the layer's gate|up and down packs."""
+    lib = _lib()
+    E, S = packed.num_experts, packed.shared_width
+    s_pad, w_pad = _round_up(S, 128), _round_up(packed.expert_width, 64)
+    dev = packed.expert_gate_up.device
+    k_groups, f_groups = (hidden + 63) // 64, (s_pad + E * w_pad) // 64
+    rows = 2 * (s_pad + E * w_pad)
+    h_rows = _round_up(hidden, DOWN_ALIGN)
+    gu = torch.empty(rows // 16, k_groups, 1024, dtype=torch.uint8, device=dev)
+    # a segment's padding can reach past the groups its columns fill
+    down = torch.zeros(h_rows // 16, f_groups, 1024, dtype=torch.uint8, device=dev)
+    scales = torch.empty(1 + E, h_rows, dtype=torch.float32, device=dev)
+    scales[0] = packed.shared_down_scale if S else 0.0
+    scales[1:] = packed.expert_down_scale
+
+    def put(w, cols, dst, groups, group0):
+        st = lib.trmoe_pack_fragments_e4m3(_p(w), w.shape[0], cols, w.shape[1], _p(dst), groups, group0, _stream(w))
+        N.check(st, "trmoe_pack_fragments_e4m3")
+
+    gu_scales = []
+    if S:
+        put(packed.shared_gate_up, hidden, gu, k_groups, 0)
+        put(packed.shared_down, S, down, f_groups, 0)
+        gu_scales.append(packed.shared_gate_up_scale)
+    experts = packed.expert_gate_up.view(E * 2 * w_pad, -1)
+    put(experts, hidden, gu[2 * s_pad // 16:], k_groups, 0)
+    gu_scales.append(packed.expert_gate_up_scale.reshape(-1))
+    for e in range(E):
+        put(packed.expert_down[e], packed.expert_width, down, f_groups, (s_pad + e * w_pad) // 64)
+    return E4M3Decode(gu, torch.cat(gu_scales), down, scales)
+
+
+def e4m3_decode_layer(x: torch.Tensor, token_ids: torch.Tensor, route_table: torch.Tensor, packed: "PackedLayer",
+                      route_weights: Sequence[float], shared_scale: float, routed_scale: float,
+                      residual: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """layer_forward of an e4m3 layer on at most SKINNY_MAX_TOKENS tokens."""
+    lib = _lib()
+    _require_cuda(x, token_ids, route_table, residual)
+    n, hidden = x.shape
+    E, S, W = packed.num_experts, packed.shared_width, packed.expert_width
+    dw = packed.e4m3_decode(hidden)
+    feats = _round_up(S, 128) + E * _round_up(W, 64)
+    ids = token_ids.reshape(-1)
+    ids = (ids if ids.dtype == torch.int64 else ids.to(torch.int64)).contiguous()
+    table = route_table.contiguous()
+    top_k, vocab = table.shape
+    if ids.numel() != n or table.dtype != torch.int64:
+        raise ValueError("e4m3_decode_layer: one token id per row and an int64 route table")
+    h = torch.empty(n, feats, dtype=x.dtype, device=x.device)
+    out = torch.empty(n, hidden, dtype=x.dtype, device=x.device)
+    rw = _weights_arg(route_weights)
+    st = lib.trmoe_gate_up_e4m3_decode(_p(x), n, hidden, x.stride(0), _p(dw.gate_up), _p(dw.gate_up_scale), S, E, W,
+                                       _p(ids), _p(table), vocab, top_k, ctypes.cast(rw, ctypes.c_void_p),
+                                       float(shared_scale), float(routed_scale), _p(h), feats, _stream(x))
+    N.check(st, "trmoe_gate_up_e4m3_decode")
+    ws_bytes = lib.trmoe_down_e4m3_decode_workspace_bytes(n, hidden, S, E, W)
+    ws = _down_workspace(x.device, ws_bytes)
+    st = lib.trmoe_down_e4m3_decode(_p(h), n, feats, _p(dw.down), _p(dw.down_scale), dw.down_scale.shape[1], S, E, W,
+                                    hidden, _p(ids), _p(table), vocab, top_k, _p(residual),
+                                    residual.stride(0) if residual is not None else 0, _p(out), hidden, _p(ws),
+                                    ws_bytes, _stream(x))
+    N.check(st, "trmoe_down_e4m3_decode")
+    return out
+
+
 def _weights_arg(route_weights: Sequence[float]):
     arr = (ctypes.c_float * 4)(*[float(w) for w in list(route_weights)[:4]])
     return arr
@@ -724,6 +802,13 @@ class PackedLayer:
     # name -> (copy, cols)
     frag: dict = field(default_factory=dict)
 
+    e4m3_frag: Optional[E4M3Decode] = None           # decode copy of an e4m3 layer, built on first use
+
+    def e4m3_decode(self, hidden: int) -> E4M3Decode:
+        if self.e4m3_frag is None:
+            self.e4m3_frag = pack_e4m3_decode(self, hidden)
+        return self.e4m3_frag
+
     @property
     def fp8(self) -> bool:
         """True when any packed weight holds e4m3 codes (inference-only)."""
@@ -763,7 +848,8 @@ def layer_forward(x: torch.Tensor, token_ids: torch.Tensor, route_table: torch.T
     """out[N, H] = shared_scale*shared(x) + routed_scale*routed(x) (+ residual).
 
     grouped: K1 partition, K3 grouped experts, K2 shared gate|up, K4 down with
-    the un-permute in its epilogue.  dense: fused gate|up over shared and
+    the un-permute in its epilogue; e4m3 weights at decode sizes: one gate|up
+    and one down over the shared and every expert's features.  dense: fused gate|up over shared and
     expert features with route-weighted expert outputs, then one down GEMM.
     norm_eps: the layer runs on rmsnorm(x) (the packs must hold the gate/up
     weights times the norm weight); the per-token scales come from the decode
@@ -807,6 +893,8 @@ def layer_forward(x: torch.Tensor, token_ids: torch.Tensor, route_table: torch.T
                                   top_k, route_weights, 1.0, 1.0, residual,
                                   w_frag=packed.fragments("dense_down", packed.dense_features) if decode else None)
         return (out, gu, h) if save else out
+    if decode and rscale is None and x.dtype == torch.bfloat16 and packed.expert_gate_up.dtype == torch.float8_e4m3fn:
+        return e4m3_decode_layer(x, token_ids, route_table, packed, route_weights, shared_scale, routed_scale, residual)
     sorted_idx, inverse, offsets, _ = route_sort(token_ids, route_table, packed.num_experts, order)
     y = routed_experts(x, sorted_idx, offsets, packed.num_experts, top_k, packed.expert_gate_up,
                        packed.expert_gate_up_scale, packed.expert_down, packed.expert_down_scale,

@@ -828,6 +828,121 @@ int trmoe_pack_fragments(int dtype, const void* packed, int64_t rows, int64_t co
                                  as_stream(stream));
 }
 
+int trmoe_pack_fragments_e4m3(const void* packed, int64_t rows, int64_t cols, int64_t ld, void* dst,
+                              int64_t dst_groups, int64_t group0, void* stream) {
+    TRMOE_REQUIRE(rows > 0 && rows % 16 == 0 && cols > 0 && ld >= round_up(cols, 8) && ld % 8 == 0,
+                  "pack_fragments_e4m3: rows must be a positive multiple of 16, ld a multiple of 8, at least "
+                  "round_up(cols, 8)");
+    TRMOE_REQUIRE(group0 >= 0 && dst_groups >= group0 + (cols + 63) / 64,
+                  "pack_fragments_e4m3: the K groups do not fit the destination's");
+    TRMOE_REQUIRE(packed && dst, "pack_fragments_e4m3: null pointer");
+    TRMOE_REQUIRE(reinterpret_cast<uintptr_t>(packed) % 8 == 0 && aligned16(dst),
+                  "pack_fragments_e4m3: packed must be 8-byte, dst 16-byte aligned");
+    TRMOE_REQUIRE(rows * ld < ((int64_t)1 << 40) && rows * dst_groups < ((int64_t)1 << 40),
+                  "pack_fragments_e4m3: too large");
+    return launch_pack_fragments_e4m3(packed, rows, cols, ld, dst, dst_groups, group0, as_stream(stream));
+}
+
+static int e4m3_decode_ok(const char* who, int64_t n_tokens, int64_t hidden, int64_t shared_width, int num_experts,
+                          int64_t expert_width, int64_t vocab_size, int top_k) {
+    const bool ok = n_tokens >= 0 && n_tokens <= kSkinnyMaxTokens && hidden > 0 && hidden < (int64_t)1 << 20 &&
+                    shared_width >= 0 && shared_width < (int64_t)1 << 20 && num_experts >= 1 &&
+                    num_experts <= kMaxExperts && expert_width > 0 && expert_width < (int64_t)1 << 16 &&
+                    vocab_size > 0 && top_k >= 1 && top_k <= kMaxTopK && top_k <= num_experts;
+    if (ok) return TRMOE_OK;
+    std::string m = std::string(who) + ": at most 128 tokens, and positive dimensions within the kernel's limits";
+    return set_error(TRMOE_ERR_INVALID, m.c_str());
+}
+
+int trmoe_gate_up_e4m3_decode(const void* x, int64_t n_tokens, int64_t hidden, int64_t ldx, const void* w_frag,
+                              const float* w_scale, int64_t shared_width, int num_experts, int64_t expert_width,
+                              const int64_t* token_ids, const int64_t* route_table, int64_t vocab_size, int top_k,
+                              const float* route_weights, float shared_scale, float routed_scale, void* h, int64_t ldh,
+                              void* stream) {
+    const int st = e4m3_decode_ok("gate_up_e4m3_decode", n_tokens, hidden, shared_width, num_experts, expert_width,
+                                  vocab_size, top_k);
+    if (st) return st;
+    const int64_t s_pad = round_up(shared_width, 128), w_pad = round_up(expert_width, 64);
+    const int64_t feats = s_pad + num_experts * w_pad;
+    TRMOE_REQUIRE(ldx >= hidden && ldh >= feats, "gate_up_e4m3_decode: row stride too small");
+    if (n_tokens == 0) return TRMOE_OK;
+    TRMOE_REQUIRE(x && w_frag && w_scale && token_ids && route_table && route_weights && h,
+                  "gate_up_e4m3_decode: null pointer");
+    TRMOE_REQUIRE(rows_ok(x, ldx, 2) && rows_ok(h, ldh, 2) && aligned16(w_frag),
+                  "gate_up_e4m3_decode: x, h and w_frag must be 16-byte aligned with row strides that are multiples of "
+                  "16 bytes");
+    GateUpArgs a{};
+    a.x = x;
+    a.ldx = ldx;
+    a.M = n_tokens;
+    a.K = (int)hidden;
+    a.w_frag = w_frag;
+    a.w_scale = w_scale;
+    a.h = h;
+    a.ldh = ldh;
+    a.shared_mult = shared_scale;
+    a.shared_feats = s_pad;
+    a.expert_feats = w_pad;
+    a.ids = token_ids;
+    a.table = route_table;
+    a.vocab = vocab_size;
+    a.top_k = top_k;
+    a.E = num_experts;
+    for (int j = 0; j < 4; ++j) a.rw[j] = j < top_k ? routed_scale * route_weights[j] : 0.f;
+    return launch_gate_up_e4m3_decode(a, 2 * feats, as_stream(stream));
+}
+
+size_t trmoe_down_e4m3_decode_workspace_bytes(int64_t n_tokens, int64_t hidden, int64_t shared_width, int num_experts,
+                                              int64_t expert_width) {
+    if (n_tokens < 1 || n_tokens > kSkinnyMaxTokens || hidden < 1 || shared_width < 0 || num_experts < 1 ||
+        expert_width < 1)
+        return 0;
+    return down_e4m3_workspace_bytes(n_tokens, hidden,
+                                     round_up(shared_width, 128) + num_experts * round_up(expert_width, 64));
+}
+
+int trmoe_down_e4m3_decode(const void* h, int64_t n_tokens, int64_t ldh, const void* w_frag, const float* w_scale,
+                           int64_t scale_ld, int64_t shared_width, int num_experts, int64_t expert_width,
+                           int64_t hidden, const int64_t* token_ids, const int64_t* route_table, int64_t vocab_size,
+                           int top_k, const void* residual, int64_t ldr, void* out, int64_t ldo, void* workspace,
+                           size_t workspace_bytes, void* stream) {
+    const int st = e4m3_decode_ok("down_e4m3_decode", n_tokens, hidden, shared_width, num_experts, expert_width,
+                                  vocab_size, top_k);
+    if (st) return st;
+    const int64_t s_pad = round_up(shared_width, 128), w_pad = round_up(expert_width, 64);
+    TRMOE_REQUIRE(ldh >= s_pad + num_experts * w_pad && ldo >= hidden && (residual == nullptr || ldr >= hidden),
+                  "down_e4m3_decode: row stride too small");
+    TRMOE_REQUIRE(scale_ld >= round_up(hidden, 32), "down_e4m3_decode: scale_ld < round_up(hidden, 32)");
+    if (n_tokens == 0) return TRMOE_OK;
+    TRMOE_REQUIRE(h && w_frag && w_scale && token_ids && route_table && out && workspace,
+                  "down_e4m3_decode: null pointer");
+    TRMOE_REQUIRE(rows_ok(h, ldh, 2) && aligned16(w_frag) && aligned16(workspace),
+                  "down_e4m3_decode: h, w_frag and workspace must be 16-byte aligned, h rows a multiple of 16 bytes");
+    TRMOE_REQUIRE(workspace_bytes >= trmoe_down_e4m3_decode_workspace_bytes(n_tokens, hidden, shared_width, num_experts,
+                                                                            expert_width),
+                  "down_e4m3_decode: workspace smaller than trmoe_down_e4m3_decode_workspace_bytes()");
+    Down8Args a{};
+    a.h = h;
+    a.ldh = ldh;
+    a.M = n_tokens;
+    a.w_frag = w_frag;
+    a.w_scale = w_scale;
+    a.scale_ld = scale_ld;
+    a.seg0 = (int)(s_pad / 64);
+    a.seg1 = (int)(w_pad / 64);
+    a.E = num_experts;
+    a.N = (int)hidden;
+    a.ids = token_ids;
+    a.table = route_table;
+    a.vocab = vocab_size;
+    a.top_k = top_k;
+    a.residual = residual;
+    a.ldr = ldr;
+    a.out = out;
+    a.ldo = ldo;
+    return launch_down_e4m3_decode(a, static_cast<float*>(workspace), as_stream(stream));
+}
+
 // Extras of the *_ex entry points: validated against the call they ride on.
 static int extras_ok(const char* who, const trmoe_call_extras* ex, int act_dtype, int w_dtype, int64_t k,
                      int64_t n_tokens, bool rms_allowed) {

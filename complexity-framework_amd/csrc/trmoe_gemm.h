@@ -121,6 +121,27 @@ struct DownArgs {
     int64_t ldhs;
 };
 
+// Decode down of an e4m3 layer over the concatenated features [shared (seg0
+// spans of 64) | expert 0 (seg1 spans) | ...] (trmoe_decode8.hip).
+struct Down8Args {
+    const void* h;           // bf16 [M, 64 * (seg0 + E * seg1)]
+    int64_t ldh;
+    int64_t M;
+    const void* w_frag;      // fragment-major codes, 16-row blocks of seg0 + E * seg1 spans
+    const float* w_scale;    // [1 + E][scale_ld]: per segment and output column
+    int64_t scale_ld;
+    int seg0, seg1, E;
+    int N;
+    const int64_t* ids;
+    const int64_t* table;
+    int64_t vocab;
+    int top_k;
+    const void* residual;    // may be null
+    int64_t ldr;
+    void* out;
+    int64_t ldo;
+};
+
 struct RoutedArgs {
     const void* x;
     int64_t ldx;
@@ -242,6 +263,11 @@ struct WgradArgs {
 int launch_pack(const PackArgs& p, hipStream_t stream);
 int launch_gate_up_skinny(int act, int wdt, const GateUpArgs& a, int64_t packed_rows, hipStream_t stream);
 size_t down_skinny_workspace_bytes(int64_t M, int64_t N, int64_t K, int act);
+int launch_pack_fragments_e4m3(const void* src, int64_t rows, int64_t cols, int64_t ld, void* dst, int64_t dst_groups,
+                               int64_t group0, hipStream_t stream);
+int launch_gate_up_e4m3_decode(const GateUpArgs& a, int64_t packed_rows, hipStream_t stream);
+size_t down_e4m3_workspace_bytes(int64_t M, int64_t N, int64_t K);
+int launch_down_e4m3_decode(const Down8Args& a, float* part, hipStream_t stream);
 int launch_stream_read(const void* src, int64_t bytes, uint32_t* sink, int blocks, hipStream_t stream);
 int launch_down_skinny(int act, int wdt, const DownArgs& a, void* workspace, hipStream_t stream);
 int launch_gate_up(int act, int wdt, const GateUpArgs& a, int64_t packed_rows, hipStream_t stream);

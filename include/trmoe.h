@@ -407,6 +407,40 @@ size_t trmoe_fragment_bytes(int dtype, int64_t rows, int64_t cols);
 int trmoe_pack_fragments(int dtype, const void* packed, int64_t rows, int64_t cols, int64_t ld, void* dst,
                          void* stream);
 
+/* ---------------------------------------------------------------------------
+ * Decode (n_tokens <= 128) of a layer with e4m3 weights: the shared branch and
+ * every expert in one gate|up and one down over the concatenated features
+ *     [shared (padded to 128) | expert 0 (padded to 64) | expert 1 | ...],
+ * expert features times the token's route weight (zero where it is not routed
+ * to the expert), as the masked loop of engine.py:66-104 defines them.
+ *
+ * trmoe_pack_fragments_e4m3 copies a packed e4m3 weight [rows, ld] (rows % 16
+ * == 0) so that 16 rows x 64 K values are 1 KiB contiguous:
+ *     dst[(((r / 16) * dst_groups + group0 + k / 64) * 64 + ((k % 64) / 16) * 16 + r % 16) * 16 + k % 16]
+ *         = code k of packed row r, zeros past cols.
+ * gate|up: the shared pack's rows, then each expert's, dst_groups =
+ * ceil(hidden / 64), group0 = 0; w_scale the packs' row scales in the same
+ * order.  down: the rows of every segment (round_up(hidden, 256)), dst_groups
+ * = (round_up(shared_width, 128) + E * round_up(expert_width, 64)) / 64, group0
+ * the segment's first (groups no segment column reaches are zero: clear dst
+ * first); w_scale [1 + E][scale_ld] the segments' column scales
+ * (row 0 is not read when shared_width is 0).
+ * ------------------------------------------------------------------------- */
+int trmoe_pack_fragments_e4m3(const void* packed, int64_t rows, int64_t cols, int64_t ld, void* dst,
+                              int64_t dst_groups, int64_t group0, void* stream);
+int trmoe_gate_up_e4m3_decode(const void* x, int64_t n_tokens, int64_t hidden, int64_t ldx, const void* w_frag,
+                              const float* w_scale, int64_t shared_width, int num_experts, int64_t expert_width,
+                              const int64_t* token_ids, const int64_t* route_table, int64_t vocab_size, int top_k,
+                              const float* route_weights, float shared_scale, float routed_scale, void* h, int64_t ldh,
+                              void* stream);
+size_t trmoe_down_e4m3_decode_workspace_bytes(int64_t n_tokens, int64_t hidden, int64_t shared_width, int num_experts,
+                                              int64_t expert_width);
+int trmoe_down_e4m3_decode(const void* h, int64_t n_tokens, int64_t ldh, const void* w_frag, const float* w_scale,
+                           int64_t scale_ld, int64_t shared_width, int num_experts, int64_t expert_width,
+                           int64_t hidden, const int64_t* token_ids, const int64_t* route_table, int64_t vocab_size,
+                           int top_k, const void* residual, int64_t ldr, void* out, int64_t ldo, void* workspace,
+                           size_t workspace_bytes, void* stream);
+
 /*
  * Optional extras of the *_ex entry points (all-zero = the plain call):
  *   row_scale / rms_eps: the fused RMSNorm scales of the *_rms entry points
