@@ -128,6 +128,17 @@ SIGNATURES = {
     ),
     "trmoe_fragment_bytes": (_c_size, [_c_int, _c_i64, _c_i64]),
     "trmoe_pack_fragments": (_c_int, [_c_int, _c_vp, _c_i64, _c_i64, _c_i64, _c_vp, _c_vp]),
+    "trmoe_qk_norm_rope": (
+        _c_int,
+        [_c_vp, _c_i64, _c_i64, _c_int, _c_int, _c_i64, _c_vp, _c_vp, _c_float, _c_vp, _c_vp, _c_i64, _c_i64, _c_vp,
+         _c_vp, _c_vp, _c_vp, _c_i64, _c_vp],
+    ),
+    "trmoe_decode_attention_workspace_bytes": (_c_size, [_c_i64, _c_i64, _c_int, _c_int, _c_i64]),
+    "trmoe_decode_attention": (
+        _c_int,
+        [_c_vp, _c_i64, _c_i64, _c_i64, _c_vp, _c_float, _c_vp, _c_int, _c_int, _c_vp, _c_vp, _c_float, _c_vp, _c_vp,
+         _c_i64, _c_vp, _c_vp, _c_vp, _c_i64, _c_float, _c_vp, _c_vp, _c_size, _c_vp],
+    ),
     "trmoe_pack_fragments_e4m3": (_c_int, [_c_vp, _c_i64, _c_i64, _c_i64, _c_vp, _c_i64, _c_i64, _c_vp]),
     "trmoe_gate_up_e4m3_decode": (
         _c_int,

@@ -21,7 +21,13 @@ cache, ``decode_step`` appends one token per sequence, and ``generate``
 replays a HIP-graph capture of the decode step (the position is a device
 counter, so one capture serves every step).
 
-Decode attention over the static cache: for one new token, GQA is the 14
+On a GPU in bf16 the attention half runs on the HIP kernels too
+(``ops.qk_norm_rope``, ``ops.decode_attention``): a prompt's q/k norm, rotation
+and cache writes are one pass over the projection, and a decode step of up to
+16 sequences is three launches per block (norm + projection; q/k norm,
+rotation, cache write and attention; output projection + residual).
+
+Elsewhere, decode attention over the static cache: for one new token, GQA is the 14
 query heads viewed as 2 groups of 7 rows, one group per key/value head
 (head h uses key/value head h // 7, as ``repeat_interleave`` pairs them), so
 SDPA runs on [B, 2, 7, 64] queries against the cache without copying it;
@@ -42,7 +48,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import ops
-from .tr_hash import TRHashEngine, TRHashEngineConfig
+from .tr_hash import TRHashBackend, TRHashEngine, TRHashEngineConfig
 
 try:   # torch >= 2.3
     from torch.nn.attention import SDPBackend, sdpa_kernel
@@ -221,6 +227,7 @@ class TRGQADecoder(nn.Module):
         self.cache_len = 0
         self._pos: Optional[torch.Tensor] = None   # device int64 [1]: next decode position
         self._rope = None
+        self._rope32 = None
         self._graph = None
 
     # ------------------------------------------------------------------ weights
@@ -257,8 +264,30 @@ class TRGQADecoder(nn.Module):
             self._rope = (cos.to(device=device, dtype=dtype), sin.to(device=device, dtype=dtype))
         return self._rope
 
+    def _rope_tables32(self, positions: int, device):
+        """fp32 cos / sin for the HIP attention kernels."""
+        if self._rope32 is None or self._rope32[0].shape[0] < positions or self._rope32[0].device != device:
+            cos, sin = rope_tables(self.cfg.head_dim, max(positions, self.cfg.max_position_embeddings),
+                                   self.cfg.rope_theta)
+            self._rope32 = (cos.to(device), sin.to(device))
+        return self._rope32
+
+    def _hip_attention(self, device: torch.device) -> bool:
+        """Whether the attention half runs on the HIP kernels: bf16 on a GPU,
+        dimensions they take, and a decoder that is not pinned to PYTORCH."""
+        cfg = self.cfg
+        return (device.type == "cuda" and self.embed_tokens.weight.dtype == torch.bfloat16
+                and self.layers[0].mlp.config.backend is not TRHashBackend.PYTORCH
+                and ops.attention_unsupported(cfg.hidden_size, cfg.num_heads, cfg.num_kv_heads, cfg.head_dim) is None)
+
+    def _norm(self, norm: RMSNorm, h: torch.Tensor, hip: bool) -> torch.Tensor:
+        if not hip:
+            return norm(h)
+        return ops.rmsnorm_forward(h.reshape(-1, h.shape[-1]), norm.weight, norm.eps)[0].view(h.shape)
+
     def logits(self, h: torch.Tensor) -> torch.Tensor:
-        return F.linear(self.norm(h), self.embed_tokens.weight)
+        hip = not torch.is_grad_enabled() and self._hip_attention(h.device)
+        return F.linear(self._norm(self.norm, h, hip), self.embed_tokens.weight)
 
     # ------------------------------------------------------------------ prompt
     @torch.no_grad()
@@ -276,21 +305,35 @@ class TRGQADecoder(nn.Module):
         # static cache rounded to 64 positions (the masked decode kernel wants
         # an aligned mask row; positions past the current one are masked)
         L = (T + max_new_tokens + 63) // 64 * 64
-        self.k_cache = [torch.zeros(B, cfg.num_kv_heads, L, cfg.head_dim, device=dev, dtype=dt)
+        self.k_cache = [torch.empty(B, cfg.num_kv_heads, L, cfg.head_dim, device=dev, dtype=dt)
                         for _ in self.layers]
-        self.v_cache = [torch.zeros_like(c) for c in self.k_cache]
+        self.v_cache = [torch.empty_like(c) for c in self.k_cache]
+        if L > T:   # the prompt fills the rest
+            for c in self.k_cache + self.v_cache:
+                c[:, :, T:].zero_()
         self.cache_len = T
         self._graph = None
-        cos, sin = self._rope_tables(L, dev, dt)
-        cos, sin = cos[:T], sin[:T]
+        hip = self._hip_attention(dev)
+        if hip:
+            cos, sin = self._rope_tables32(L, dev)
+        else:
+            cos, sin = self._rope_tables(L, dev, dt)
+            cos, sin = cos[:T], sin[:T]
         h = self.embed_tokens(input_ids)
         for i, block in enumerate(self.layers):
             ev = _events(timings, "attention")
-            x = block.input_layernorm(h)
-            q, k, v = block.self_attn.project(x, cos, sin)
-            self.k_cache[i][:, :, :T].copy_(k)
-            self.v_cache[i][:, :, :T].copy_(v)
-            h = h + block.self_attn.output(block.self_attn.prefill_attention(q, k, v))
+            attn = block.self_attn
+            x = self._norm(block.input_layernorm, h, hip)
+            if hip:
+                q = ops.qk_norm_rope(F.linear(x, attn.kqv_weight()).view(B * T, -1), B, cfg.num_heads,
+                                     attn.q_norm.weight, attn.k_norm.weight, attn.q_norm.eps, cos, sin,
+                                     self.k_cache[i], self.v_cache[i]).transpose(1, 2)
+                k, v = self.k_cache[i][:, :, :T], self.v_cache[i][:, :, :T]
+            else:
+                q, k, v = attn.project(x, cos, sin)
+                self.k_cache[i][:, :, :T].copy_(k)
+                self.v_cache[i][:, :, :T].copy_(v)
+            h = h + attn.output(attn.prefill_attention(q, k, v))
             _end(ev)
             ev = _events(timings, "mlp")
             h = self._mlp(block, h, input_ids)
@@ -306,8 +349,10 @@ class TRGQADecoder(nn.Module):
         B = ids.shape[0]
         L = self.k_cache[0].shape[2]
         dt = self.embed_tokens.weight.dtype
-        cos_t, sin_t = self._rope_tables(L, ids.device, dt)
         pos = self._pos
+        if B <= ops.DECODE_ATTN_MAX_BATCH and self._hip_attention(ids.device):
+            return self._decode_body_hip(ids, pos, L)
+        cos_t, sin_t = self._rope_tables(L, ids.device, dt)
         cos = cos_t.index_select(0, pos)           # [1, D]
         sin = sin_t.index_select(0, pos)
         span = torch.arange(L, device=ids.device)
@@ -323,6 +368,21 @@ class TRGQADecoder(nn.Module):
             h = h + block.self_attn.output(attn)
             h = self._mlp(block, h, tok)
         return self.logits(h).view(B, -1)
+
+    def _decode_body_hip(self, ids: torch.Tensor, pos: torch.Tensor, L: int) -> torch.Tensor:
+        cfg = self.cfg
+        B = ids.shape[0]
+        cos, sin = self._rope_tables32(L, ids.device)
+        tok = ids.view(B, 1)
+        h = self.embed_tokens(ids)
+        for i, block in enumerate(self.layers):
+            attn, norm = block.self_attn, block.input_layernorm
+            a = ops.decode_attention(h, norm.weight, norm.eps, attn.kqv_weight(), cfg.num_heads, attn.q_norm.weight,
+                                     attn.k_norm.weight, attn.q_norm.eps, cos, sin, pos, self.k_cache[i],
+                                     self.v_cache[i], attn.scale)
+            h = ops.decode_linear(a, attn.o_proj.weight, h)
+            h = self._mlp(block, h.view(B, 1, -1), tok).view(B, -1)
+        return self.logits(h)
 
     @torch.no_grad()
     def decode_step(self, ids: torch.Tensor) -> torch.Tensor:

@@ -545,6 +545,100 @@ def rmsnorm_backward(x: torch.Tensor, weight: torch.Tensor, r: torch.Tensor, dy:
     return dx, dw
 
 
+# ---------------------------------------------------------------------------
+# decoder attention
+# ---------------------------------------------------------------------------
+
+ATTN_HEAD_DIM = 64
+DECODE_ATTN_MAX_BATCH = 16
+_DECODE_ATTN_GROUPS = (1, 2, 4, 7, 8)
+
+
+def attention_unsupported(hidden: int, num_heads: int, num_kv_heads: int, head_dim: int) -> Optional[str]:
+    """Why the decoder attention kernels cannot take these dimensions (None when they can)."""
+    if head_dim != ATTN_HEAD_DIM:
+        return f"heads of {ATTN_HEAD_DIM}, not {head_dim}"
+    if num_heads % num_kv_heads or num_heads // num_kv_heads not in _DECODE_ATTN_GROUPS:
+        return f"{_DECODE_ATTN_GROUPS} query heads per kv head, not {num_heads} / {num_kv_heads}"
+    if hidden % 32 or hidden > RMSNORM_MAX_HIDDEN[torch.bfloat16]:
+        return f"hidden a multiple of 32, at most {RMSNORM_MAX_HIDDEN[torch.bfloat16]}, not {hidden}"
+    return None
+
+
+def _check_attention(kqv_or_x, tables, caches, weights):
+    cos, sin = tables
+    _require_cuda(kqv_or_x, cos, sin, *caches, *weights)
+    if kqv_or_x.dtype != torch.bfloat16 or any(w.dtype != torch.bfloat16 or not w.is_contiguous() for w in weights):
+        raise ValueError("decoder attention: bf16 activations and contiguous bf16 weights")
+    for t in (cos, sin):
+        if t.dtype != torch.float32 or not t.is_contiguous() or t.shape[-1] != ATTN_HEAD_DIM:
+            raise ValueError("decoder attention: contiguous fp32 cos / sin tables [positions, 64]")
+    k, v = caches
+    if k.dtype != torch.bfloat16 or v.dtype != torch.bfloat16 or k.shape != v.shape or k.ndim != 4 \
+            or not (k.is_contiguous() and v.is_contiguous()) or k.shape[3] != ATTN_HEAD_DIM:
+        raise ValueError("decoder attention: contiguous bf16 caches [sequences, kv heads, length, 64]")
+
+
+@_on_tensor_device
+def qk_norm_rope(kqv: torch.Tensor, sequences: int, num_heads: int, q_weight: torch.Tensor, k_weight: torch.Tensor,
+                 eps: float, cos: torch.Tensor, sin: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
+                 first_position: int = 0, position: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """q [sequences, T, num_heads, 64] = rope(rmsnorm(q)) of the fused
+    projection kqv [sequences * T, (num_heads + 2 kv) * 64]; k and v go into
+    the caches at first_position + t (+ the device counter `position`)."""
+    _check_attention(kqv, (cos, sin), (k_cache, v_cache), (q_weight, k_weight))
+    B, kvh, L, D = k_cache.shape
+    kqv = _rows(kqv)
+    rows, width = kqv.shape
+    if B != sequences or rows % sequences or width != (num_heads + 2 * kvh) * D or q_weight.numel() != D \
+            or k_weight.numel() != D or (position is not None and position.dtype != torch.int64):
+        raise ValueError("qk_norm_rope: shapes do not match")
+    T = rows // sequences
+    q = torch.empty(sequences, T, num_heads, D, dtype=kqv.dtype, device=kqv.device)
+    st = _lib().trmoe_qk_norm_rope(_p(kqv), sequences, T, num_heads, kvh, kqv.stride(0), _p(_vec16(q_weight)),
+                                   _p(_vec16(k_weight)), float(eps), _p(cos), _p(sin), cos.shape[0], first_position,
+                                   _p(position), _p(q), _p(k_cache), _p(v_cache), L, _stream(kqv))
+    N.check(st, "trmoe_qk_norm_rope")
+    return q
+
+
+@_on_tensor_device
+def decode_attention(x: torch.Tensor, norm_weight: torch.Tensor, norm_eps: float, w_kqv: torch.Tensor, num_heads: int,
+                     q_weight: torch.Tensor, k_weight: torch.Tensor, qk_eps: float, cos: torch.Tensor,
+                     sin: torch.Tensor, position: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
+                     scale: float) -> torch.Tensor:
+    """Attention output [B, num_heads * 64] of one new token per sequence (x
+    [B, hidden], B <= DECODE_ATTN_MAX_BATCH) at the device counter `position`:
+    input RMSNorm, projection, q / k norm and rotation, cache write, attention."""
+    lib = _lib()
+    norm_weight, q_weight, k_weight = _vec16(norm_weight), _vec16(q_weight), _vec16(k_weight)
+    _check_attention(x, (cos, sin), (k_cache, v_cache), (w_kqv, norm_weight, q_weight, k_weight))
+    B, kvh, L, D = k_cache.shape
+    x = _rows(x)
+    n, hidden = x.shape
+    if n != B or w_kqv.shape != ((num_heads + 2 * kvh) * D, hidden) or norm_weight.numel() != hidden \
+            or q_weight.numel() != D or k_weight.numel() != D or position.dtype != torch.int64:
+        raise ValueError("decode_attention: shapes do not match")
+    attn = torch.empty(n, num_heads * D, dtype=x.dtype, device=x.device)
+    ws_bytes = lib.trmoe_decode_attention_workspace_bytes(n, hidden, num_heads, kvh, L)
+    ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=x.device)
+    st = lib.trmoe_decode_attention(_p(x), n, hidden, x.stride(0), _p(norm_weight), float(norm_eps), _p(w_kqv),
+                                    num_heads, kvh, _p(q_weight), _p(k_weight), float(qk_eps), _p(cos), _p(sin),
+                                    cos.shape[0], _p(position), _p(k_cache), _p(v_cache), L, float(scale), _p(attn),
+                                    _p(ws), ws_bytes, _stream(x))
+    N.check(st, "trmoe_decode_attention")
+    return attn
+
+
+def decode_linear(x: torch.Tensor, weight: torch.Tensor, residual: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """x [n, K] . weight^T (+ residual) for n <= SKINNY_MAX_TOKENS rows and an
+    nn.Linear weight [N, K] with N % 32 == 0, K % 8 == 0, on the decode down kernel."""
+    n, k = x.shape
+    if n > SKINNY_MAX_TOKENS or weight.shape[0] % 32 or k % 8 or not weight.is_contiguous() or weight.shape[1] != k:
+        raise ValueError("decode_linear: at most 128 rows, a contiguous [N, K] weight with N % 32 == 0 and K % 8 == 0")
+    return shared_down_combine(x, k, weight, None, weight.shape[0], None, None, 1, (1.0,), 1.0, 0.0, residual)
+
+
 def _extras(row_scale: Optional[torch.Tensor] = None, rms_eps: float = 0.0, w_frag=None):
     """trmoe_call_extras for the *_ex calls; w_frag = (fragment copy, cols)."""
     e = N.CallExtras()

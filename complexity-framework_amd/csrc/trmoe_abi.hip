@@ -10,6 +10,7 @@
 #include <string>
 #include <utility>
 
+#include "trmoe_attn.h"
 #include "trmoe_common.h"
 #include "trmoe_gemm.h"
 #include "trmoe_internal.h"
@@ -941,6 +942,117 @@ int trmoe_down_e4m3_decode(const void* h, int64_t n_tokens, int64_t ldh, const v
     a.out = out;
     a.ldo = ldo;
     return launch_down_e4m3_decode(a, static_cast<float*>(workspace), as_stream(stream));
+}
+
+int trmoe_qk_norm_rope(const void* kqv, int64_t sequences, int64_t tokens, int num_heads, int num_kv_heads,
+                       int64_t ldkqv, const void* q_weight, const void* k_weight, float eps, const float* cos,
+                       const float* sin, int64_t positions, int64_t first_position, const int64_t* position, void* q,
+                       void* k_cache, void* v_cache, int64_t cache_length, void* stream) {
+    TRMOE_REQUIRE(sequences >= 0 && tokens >= 0 && num_heads > 0 && num_kv_heads > 0 && num_heads <= 1024 &&
+                      num_kv_heads <= 1024,
+                  "qk_norm_rope: bad dimensions");
+    TRMOE_REQUIRE(ldkqv >= (int64_t)(num_heads + 2 * num_kv_heads) * 64, "qk_norm_rope: ldkqv < the projection's width");
+    TRMOE_REQUIRE(cache_length > 0 && positions >= cache_length, "qk_norm_rope: positions < cache_length");
+    TRMOE_REQUIRE(first_position >= 0 && (position != nullptr || first_position + tokens <= cache_length),
+                  "qk_norm_rope: the tokens do not fit the cache");
+    TRMOE_REQUIRE(eps >= 0.0f, "qk_norm_rope: eps must be non-negative");
+    if (sequences == 0 || tokens == 0) return TRMOE_OK;
+    TRMOE_REQUIRE(kqv && q_weight && k_weight && cos && sin && q && k_cache && v_cache, "qk_norm_rope: null pointer");
+    TRMOE_REQUIRE(aligned16(kqv) && ldkqv % 8 == 0 && aligned16(q_weight) && aligned16(k_weight) && aligned16(q) &&
+                      aligned16(k_cache) && aligned16(v_cache),
+                  "qk_norm_rope: operands must be 16-byte aligned, ldkqv a multiple of 8");
+    TRMOE_REQUIRE(sequences * tokens * (num_heads + 2 * num_kv_heads) < (int64_t)1 << 36, "qk_norm_rope: too many rows");
+    RopeArgs a{};
+    a.kqv = static_cast<const bf16_t*>(kqv);
+    a.ldkqv = ldkqv;
+    a.rows = sequences * tokens;
+    a.T = tokens;
+    a.heads = num_heads;
+    a.kvh = num_kv_heads;
+    a.qw = static_cast<const bf16_t*>(q_weight);
+    a.kw = static_cast<const bf16_t*>(k_weight);
+    a.eps = eps;
+    a.cos = cos;
+    a.sin = sin;
+    a.q = static_cast<bf16_t*>(q);
+    a.k = static_cast<bf16_t*>(k_cache);
+    a.v = static_cast<bf16_t*>(v_cache);
+    a.L = cache_length;
+    a.pos0 = first_position;
+    a.pos = position;
+    return launch_qk_rope(a, as_stream(stream));
+}
+
+// Scratch of trmoe_decode_attention: the projection (fp32), the split
+// counters and the split partials, each 256-byte aligned.
+static void decode_attn_scratch(int64_t batch, int heads, int kvh, int64_t L, size_t* qkv, size_t* counters,
+                                size_t* part) {
+    *qkv = ((size_t)batch * (size_t)(heads + 2 * kvh) * 64 * sizeof(float) + 255) / 256 * 256;
+    *counters = ((size_t)batch * (size_t)kvh * sizeof(int) + 255) / 256 * 256;
+    *part = (size_t)batch * (size_t)heads * (size_t)decode_attn_splits(L, (int)batch * kvh) * 66 * sizeof(float);
+}
+
+static bool decode_attn_dims_ok(int64_t batch, int64_t hidden, int heads, int kvh, int64_t L) {
+    if (batch < 1 || batch > 16 || hidden < 32 || hidden % 32 != 0 || hidden >= (int64_t)1 << 20) return false;
+    if (heads < 1 || kvh < 1 || heads > 256 || kvh > 256 || heads % kvh != 0 || L < 1 || L >= (int64_t)1 << 24) return false;
+    const int g = heads / kvh;
+    return g == 1 || g == 2 || g == 4 || g == 7 || g == 8;
+}
+
+size_t trmoe_decode_attention_workspace_bytes(int64_t batch, int64_t hidden, int num_heads, int num_kv_heads,
+                                              int64_t cache_length) {
+    if (!decode_attn_dims_ok(batch, hidden, num_heads, num_kv_heads, cache_length)) return 0;
+    size_t a, b, c;
+    decode_attn_scratch(batch, num_heads, num_kv_heads, cache_length, &a, &b, &c);
+    return a + b + c;
+}
+
+int trmoe_decode_attention(const void* hidden_rows, int64_t batch, int64_t hidden, int64_t ldx, const void* norm_weight,
+                           float norm_eps, const void* w_kqv, int num_heads, int num_kv_heads, const void* q_weight,
+                           const void* k_weight, float qk_eps, const float* cos, const float* sin, int64_t positions,
+                           const int64_t* position, void* k_cache, void* v_cache, int64_t cache_length, float scale,
+                           void* attn, void* workspace, size_t workspace_bytes, void* stream) {
+    TRMOE_REQUIRE(decode_attn_dims_ok(batch, hidden, num_heads, num_kv_heads, cache_length),
+                  "decode_attention: 1 to 16 sequences, hidden a multiple of 32, 1, 2, 4, 7 or 8 query heads per kv "
+                  "head");
+    TRMOE_REQUIRE(positions >= cache_length && ldx >= hidden && ldx % 8 == 0, "decode_attention: bad strides");
+    TRMOE_REQUIRE(hidden_rows && norm_weight && w_kqv && q_weight && k_weight && cos && sin && position && k_cache &&
+                      v_cache && attn && workspace,
+                  "decode_attention: null pointer");
+    TRMOE_REQUIRE(aligned16(hidden_rows) && aligned16(norm_weight) && aligned16(w_kqv) && aligned16(q_weight) &&
+                      aligned16(k_weight) && aligned16(k_cache) && aligned16(v_cache) && aligned16(workspace),
+                  "decode_attention: operands must be 16-byte aligned");
+    TRMOE_REQUIRE(workspace_bytes >= trmoe_decode_attention_workspace_bytes(batch, hidden, num_heads, num_kv_heads,
+                                                                            cache_length),
+                  "decode_attention: workspace smaller than trmoe_decode_attention_workspace_bytes()");
+    size_t qkv_b, cnt_b, part_b;
+    decode_attn_scratch(batch, num_heads, num_kv_heads, cache_length, &qkv_b, &cnt_b, &part_b);
+    DecodeAttnArgs a{};
+    a.x = static_cast<const bf16_t*>(hidden_rows);
+    a.ldx = ldx;
+    a.B = (int)batch;
+    a.H = (int)hidden;
+    a.kvh = num_kv_heads;
+    a.n_qkv = (num_heads + 2 * num_kv_heads) * 64;
+    a.norm_w = static_cast<const bf16_t*>(norm_weight);
+    a.norm_eps = norm_eps;
+    a.w_kqv = static_cast<const bf16_t*>(w_kqv);
+    a.qn_w = static_cast<const bf16_t*>(q_weight);
+    a.kn_w = static_cast<const bf16_t*>(k_weight);
+    a.qk_eps = qk_eps;
+    a.scale = scale;
+    a.cos = cos;
+    a.sin = sin;
+    a.pos = position;
+    a.k_cache = static_cast<bf16_t*>(k_cache);
+    a.v_cache = static_cast<bf16_t*>(v_cache);
+    a.L = cache_length;
+    char* ws = static_cast<char*>(workspace);
+    a.qkv = reinterpret_cast<float*>(ws);
+    a.counters = reinterpret_cast<int*>(ws + qkv_b);
+    a.part = reinterpret_cast<float*>(ws + qkv_b + cnt_b);
+    a.attn = static_cast<bf16_t*>(attn);
+    return launch_decode_attn(a, num_heads / num_kv_heads, as_stream(stream));
 }
 
 // Extras of the *_ex entry points: validated against the call they ride on.

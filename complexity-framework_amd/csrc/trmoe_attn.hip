@@ -1,0 +1,388 @@
+// The attention half of a decoder block around the TR-MoE layer: grouped-query
+// attention with per-head RMSNorm on q and k and rotary embeddings
+// (complexity/core/attention/gqa.py:88-165, rotary.py:17-80) over a static
+// key/value cache.  Heads are 64 wide, bf16.
+//
+//   k_qk_rope     a prompt's fused k|q|v projection rows -> q (normed, rotated)
+//                 in [token, head, 64], k and v into the caches
+//   k_decode_qkv  one token per sequence, up to 16 sequences: RMSNorm of the
+//                 hidden row and the k|q|v projection in one launch
+//   k_decode_attn that token's q and k norm and rotation, the cache write and
+//                 attention over the cache split along the positions; the last
+//                 workgroup of a (sequence, kv head) merges the splits
+//
+// These replace chains of elementwise passes (a norm is 5 launches, a rotation
+// 5, the cache writes 2, the key/value repeat 2): at a prompt of 8 x 2048 they
+// took 7.0 of the 17.2 ms, and a decode step of one sequence was 470 launches.
+#include "trmoe_attn.h"
+
+#include "trmoe_common.h"
+#include "trmoe_internal.h"
+
+#include <algorithm>
+
+namespace trmoe {
+
+namespace {
+
+constexpr int kD = 64;        // head width
+constexpr int kLanes = 8;     // lanes of a head row, 8 elements each
+
+__device__ __forceinline__ void unpack8(u32x4 v, float (&f)[8]) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        f[2 * j] = __builtin_bit_cast(float, (uint32_t)v[j] << 16);
+        f[2 * j + 1] = __builtin_bit_cast(float, (uint32_t)v[j] & 0xffff0000u);
+    }
+}
+__device__ __forceinline__ u32x4 pack8(const float (&f)[8]) {
+    bf16x8 r;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) r[j] = (bf16_t)f[j];
+    return __builtin_bit_cast(u32x4, r);
+}
+__device__ __forceinline__ float sum8(float s) {   // over the 8 lanes of a head row
+    s += __shfl_xor(s, 1);
+    s += __shfl_xor(s, 2);
+    s += __shfl_xor(s, 4);
+    return s;
+}
+
+// x (the lane's 8 of a head row's 64 elements) -> rope(rmsnorm(x) * w) at one
+// position: element d pairs with d +- 32, which the lane 4 away holds.
+__device__ __forceinline__ void norm_rope(float (&x)[8], const bf16_t* w, float eps, const float* cos,
+                                          const float* sin, int c) {
+    float s = 0.f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) s += x[j] * x[j];
+    const float r = rsqrtf(sum8(s) * (1.0f / kD) + eps);
+    float wf[8];
+    unpack8(*reinterpret_cast<const u32x4*>(w + 8 * c), wf);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[j] = x[j] * r * wf[j];
+    const float sign = c < 4 ? -1.0f : 1.0f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const float other = __shfl_xor(x[j], 4);
+        x[j] = x[j] * cos[8 * c + j] + sign * other * sin[8 * c + j];
+    }
+}
+
+// One head row (of k, q or v) per 8 lanes.  Memory-bound: each projection row
+// is read once and written once, 16 bytes per lane.
+__global__ __launch_bounds__(256) void k_qk_rope(RopeArgs a) {
+    const int slots = a.heads + 2 * a.kvh;
+    const int64_t item = ((int64_t)blockIdx.x * 256 + threadIdx.x) / kLanes;
+    if (item >= a.rows * slots) return;   // whole 8-lane groups leave together
+    const int c = threadIdx.x & 7;
+    const int64_t row = item / slots;
+    const int slot = (int)(item - row * slots);
+    const int64_t b = row / a.T, t = row - b * a.T;
+    int64_t pos = a.pos0 + t;
+    if (a.pos != nullptr) pos += *a.pos;
+    if (pos < 0 || pos >= a.L) return;    // a position past the cache is dropped
+    const u32x4 in = *reinterpret_cast<const u32x4*>(a.kqv + row * a.ldkqv + slot * kD + 8 * c);
+    const int vslot = a.heads + a.kvh;
+    if (slot >= vslot) {
+        *reinterpret_cast<u32x4*>(a.v + ((b * a.kvh + slot - vslot) * a.L + pos) * kD + 8 * c) = in;
+        return;
+    }
+    float x[8];
+    unpack8(in, x);
+    const bool is_k = slot < a.kvh;
+    norm_rope(x, is_k ? a.kw : a.qw, a.eps, a.cos + pos * kD, a.sin + pos * kD, c);
+    bf16_t* dst = is_k ? a.k + ((b * a.kvh + slot) * a.L + pos) * kD
+                       : a.q + (row * a.heads + slot - a.kvh) * kD;
+    *reinterpret_cast<u32x4*>(dst + 8 * c) = pack8(x);
+}
+
+// qkv[m][n] (fp32) = rmsnorm(x_m) . W_n for up to 16 rows: 16 output columns
+// per workgroup, the 8 waves split K (groups of 32), one 16x16x32 MFMA each.
+// The norm weight goes onto x before the product, the row's 1/rms onto the
+// sum after it.  Latency-bound (28 KB of weights per workgroup): every load of
+// a wave's first 4 groups is issued before any is used.
+constexpr int kQkvWaves = 8, kQkvBatch = 4;
+__global__ __launch_bounds__(64 * kQkvWaves) void k_decode_qkv(DecodeAttnArgs a) {
+    __shared__ float red[kQkvWaves][4][64];
+    __shared__ float s_ssq[kQkvWaves][16];
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    const int r = lane & 15, q = lane >> 4;
+    const int n0 = (int)blockIdx.x * 16;
+    if (blockIdx.x == 0)
+        for (int i = threadIdx.x; i < a.B * a.kvh; i += 64 * kQkvWaves) a.counters[i] = 0;
+    const int groups = a.H / 32, per = (groups + kQkvWaves - 1) / kQkvWaves;
+    const int g0 = wave * per, g1 = std::min(g0 + per, groups);
+    const bf16_t* xr = a.x + (int64_t)(r < a.B ? r : 0) * a.ldx + 8 * q;
+    const bf16_t* wr = a.w_kqv + (int64_t)(n0 + r) * a.H + 8 * q;
+    const bf16_t* nr = a.norm_w + 8 * q;
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    float ssq = 0.f;
+    for (int gb = g0; gb < g1; gb += kQkvBatch) {
+        u32x4 xv[kQkvBatch], wv[kQkvBatch], nv[kQkvBatch];
+#pragma unroll
+        for (int j = 0; j < kQkvBatch; ++j) {
+            const u32x4 zero = {0u, 0u, 0u, 0u};
+            const bool in = gb + j < g1;
+            wv[j] = in ? *reinterpret_cast<const u32x4*>(wr + 32 * (gb + j)) : zero;
+            xv[j] = in && r < a.B ? *reinterpret_cast<const u32x4*>(xr + 32 * (gb + j)) : zero;
+            nv[j] = in ? *reinterpret_cast<const u32x4*>(nr + 32 * (gb + j)) : zero;
+        }
+#pragma unroll
+        for (int j = 0; j < kQkvBatch; ++j) {
+            float xf[8], nf[8];
+            unpack8(xv[j], xf);
+            unpack8(nv[j], nf);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                ssq += xf[e] * xf[e];
+                xf[e] *= nf[e];
+            }
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, pack8(xf)),
+                                                          __builtin_bit_cast(bf16x8, (u32x4)wv[j]), acc, 0, 0, 0);
+        }
+    }
+    ssq += __shfl_xor(ssq, 16);
+    ssq += __shfl_xor(ssq, 32);
+    if (q == 0) s_ssq[wave][r] = ssq;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) red[wave][i][lane] = acc[i];
+    __syncthreads();
+    if (threadIdx.x < 256) {
+        const int i = threadIdx.x >> 6, m = 4 * q + i;
+        if (m < a.B) {
+            float s = 0.f, ss = 0.f;
+#pragma unroll
+            for (int w = 0; w < kQkvWaves; ++w) {
+                s += red[w][i][lane];
+                ss += s_ssq[w][m];
+            }
+            a.qkv[(int64_t)m * a.n_qkv + n0 + r] = s * rsqrtf(ss / (float)a.H + a.norm_eps);
+        }
+    }
+}
+
+// Device-scope accesses of the split partials: they bypass the XCD's own L2,
+// so a workgroup of another XCD sees them without a cache write-back.
+__device__ __forceinline__ void store_dev(float* p, float v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float load_dev(const float* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Attention of one new token: workgroup (split, kv head, sequence) takes the
+// cache positions [split * chunk, + chunk) below the current one; the split
+// that holds the current position normalises, rotates and stores its k and v
+// and adds it.  Eight lanes hold one position's 64 elements (so each K and V
+// row is one 128-byte read) for all G query heads of the group, with a
+// running maximum and sum per head; 32 positions are in flight per workgroup
+// and kUnroll loads per lane.  A CU moves its K/V bytes at the vector ALU's
+// pace, so the positions are split until about every CU has a workgroup.
+constexpr int kUnroll = 4;
+template <int G>
+__global__ __launch_bounds__(256) void k_decode_attn(DecodeAttnArgs a, int chunk, int splits) {
+    __shared__ float s_ml[4][G][2];
+    __shared__ float s_acc[4][G][kD];
+    __shared__ int s_last;
+    const int split = (int)blockIdx.x, kvh = (int)blockIdx.y, b = (int)blockIdx.z;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int c = lane & 7, grp = threadIdx.x >> 3;
+    int64_t pos64 = *a.pos;
+    pos64 = pos64 < 0 ? 0 : (pos64 >= a.L ? a.L - 1 : pos64);
+    const int pos = (int)pos64;
+    const int p0 = split * chunk, p1 = std::min(p0 + chunk, pos);
+    const bool own = pos >= p0 && pos < p0 + chunk;
+    const float* row = a.qkv + (int64_t)b * a.n_qkv;
+    const float* cosp = a.cos + (int64_t)pos * kD;
+    const float* sinp = a.sin + (int64_t)pos * kD;
+    const int64_t head_off = ((int64_t)b * a.kvh + kvh) * a.L * kD;
+    const bf16_t* kc = a.k_cache + head_off + 8 * c;
+    const bf16_t* vc = a.v_cache + head_off + 8 * c;
+
+    float q[G][8];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        const float* src = row + (a.kvh + kvh * G + g) * kD + 8 * c;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) q[g][j] = src[j];
+        norm_rope(q[g], a.qn_w, a.qk_eps, cosp, sinp, c);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) q[g][j] *= a.scale * 1.4426950408889634f;   // exp2 below
+    }
+    float m[G], l[G], acc[G][8];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        m[g] = -1e30f;
+        l[g] = 0.f;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) acc[g][j] = 0.f;
+    }
+    auto attend = [&](const float (&kf)[8], const float (&vf)[8]) {
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            float s = 0.f;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) s += q[g][j] * kf[j];
+            s = sum8(s);
+            const float mn = fmaxf(m[g], s);
+            const float f = __builtin_amdgcn_exp2f(m[g] - mn), p = __builtin_amdgcn_exp2f(s - mn);
+            m[g] = mn;
+            l[g] = l[g] * f + p;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) acc[g][j] = acc[g][j] * f + p * vf[j];
+        }
+    };
+    for (int p = p0 + grp; p < p1; p += 32 * kUnroll) {
+        u32x4 kv[kUnroll], vv[kUnroll];
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u) {
+            const int pp = std::min(p + 32 * u, p1 - 1);
+            kv[u] = *reinterpret_cast<const u32x4*>(kc + (int64_t)pp * kD);
+            vv[u] = *reinterpret_cast<const u32x4*>(vc + (int64_t)pp * kD);
+        }
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u) {
+            if (p + 32 * u < p1) {   // uniform over the position's 8 lanes
+                float kf[8], vf[8];
+                unpack8(kv[u], kf);
+                unpack8(vv[u], vf);
+                attend(kf, vf);
+            }
+        }
+    }
+    if (own && threadIdx.x < kLanes) {
+        float kf[8], vf[8];
+        const float* ks = row + kvh * kD + 8 * c;
+        const float* vs = row + (a.kvh + a.kvh * G + kvh) * kD + 8 * c;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            kf[j] = ks[j];
+            vf[j] = vs[j];
+        }
+        norm_rope(kf, a.kn_w, a.qk_eps, cosp, sinp, c);
+        const u32x4 kb = pack8(kf), vb = pack8(vf);
+        *reinterpret_cast<u32x4*>(a.k_cache + head_off + (int64_t)pos * kD + 8 * c) = kb;
+        *reinterpret_cast<u32x4*>(a.v_cache + head_off + (int64_t)pos * kD + 8 * c) = vb;
+        unpack8(kb, kf);   // what later steps will read
+        unpack8(vb, vf);
+        attend(kf, vf);
+    }
+    // merge the wave's 8 positions, then the 4 waves
+#pragma unroll
+    for (int off = 8; off < 64; off <<= 1) {
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            const float mo = __shfl_xor(m[g], off), lo = __shfl_xor(l[g], off);
+            const float mn = fmaxf(m[g], mo);
+            const float f = __builtin_amdgcn_exp2f(m[g] - mn), fo = __builtin_amdgcn_exp2f(mo - mn);
+            m[g] = mn;
+            l[g] = l[g] * f + lo * fo;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) acc[g][j] = acc[g][j] * f + __shfl_xor(acc[g][j], off) * fo;
+        }
+    }
+    if (lane < kLanes) {
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) s_acc[wave][g][8 * c + j] = acc[g][j];
+            if (c == 0) {
+                s_ml[wave][g][0] = m[g];
+                s_ml[wave][g][1] = l[g];
+            }
+        }
+    }
+    __syncthreads();
+    bf16_t* out = a.attn + (int64_t)b * (a.kvh * G * kD) + kvh * G * kD;
+    constexpr int kPart = kD + 2;   // 64 sums, the maximum, the weight
+    float* part = a.part + ((int64_t)(b * a.kvh + kvh) * splits) * (G * kPart);
+    for (int i = threadIdx.x; i < G * kD; i += 256) {
+        const int g = i / kD, d = i % kD;
+        float mn = s_ml[0][g][0];
+#pragma unroll
+        for (int w = 1; w < 4; ++w) mn = fmaxf(mn, s_ml[w][g][0]);
+        float lt = 0.f, v = 0.f;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            const float f = __builtin_amdgcn_exp2f(s_ml[w][g][0] - mn);
+            lt += s_ml[w][g][1] * f;
+            v += s_acc[w][g][d] * f;
+        }
+        if (splits == 1) {
+            out[i] = (bf16_t)(v / lt);
+        } else {
+            float* dst = part + ((int64_t)split * G + g) * kPart;
+            store_dev(dst + d, v);
+            if (d == 0) {
+                store_dev(dst + kD, mn);
+                store_dev(dst + kD + 1, lt);
+            }
+        }
+    }
+    if (splits == 1) return;
+    // this wave's partials have reached memory before the count that says so
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0)
+        s_last = __hip_atomic_fetch_add(a.counters + b * a.kvh + kvh, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+                 splits - 1;
+    __syncthreads();
+    if (!s_last) return;
+    for (int i = threadIdx.x; i < G * kD; i += 256) {
+        const int g = i / kD, d = i % kD;
+        float mn = -1e30f, lt = 0.f, v = 0.f;
+        for (int s = 0; s < splits; ++s) {
+            const float* src = part + ((int64_t)s * G + g) * kPart;
+            const float ms = load_dev(src + kD), ls = load_dev(src + kD + 1), vs = load_dev(src + d);
+            const float m2 = fmaxf(mn, ms);
+            const float f = __builtin_amdgcn_exp2f(mn - m2), fs = __builtin_amdgcn_exp2f(ms - m2);
+            mn = m2;
+            lt = lt * f + ls * fs;
+            v = v * f + vs * fs;
+        }
+        out[i] = (bf16_t)(v / lt);
+    }
+}
+
+}  // namespace
+
+int launch_qk_rope(const RopeArgs& a, hipStream_t stream) {
+    const int64_t lanes = a.rows * (a.heads + 2 * a.kvh) * kLanes;
+    hipLaunchKernelGGL(k_qk_rope, dim3((unsigned)((lanes + 255) / 256)), dim3(256), 0, stream, a);
+    return check_launch("qk_norm_rope");
+}
+
+// Positions per split: at least 128 (4 per lane group), more when the
+// (sequence, kv head) pairs alone fill the CUs.
+static int decode_chunk(int64_t L, int pairs) {
+    int splits = std::max(1, 256 / std::max(1, pairs));
+    const int most = (int)((L + 127) / 128);
+    splits = std::min(splits, most);
+    int chunk = (int)((L + splits - 1) / splits);
+    return (chunk + 31) / 32 * 32;
+}
+
+int64_t decode_attn_splits(int64_t L, int pairs) {
+    const int chunk = decode_chunk(L, pairs);
+    return (L + chunk - 1) / chunk;
+}
+
+int launch_decode_attn(const DecodeAttnArgs& a, int group, hipStream_t stream) {
+    hipLaunchKernelGGL(k_decode_qkv, dim3((unsigned)(a.n_qkv / 16)), dim3(64 * kQkvWaves), 0, stream, a);
+    int st = check_launch("decode_attention (qkv)");
+    if (st) return st;
+    const int chunk = decode_chunk(a.L, a.B * a.kvh);
+    const int splits = (int)decode_attn_splits(a.L, a.B * a.kvh);
+    const dim3 grid((unsigned)splits, (unsigned)a.kvh, (unsigned)a.B);
+    auto kern = group == 1   ? k_decode_attn<1>
+                : group == 2 ? k_decode_attn<2>
+                : group == 4 ? k_decode_attn<4>
+                : group == 7 ? k_decode_attn<7>
+                : group == 8 ? k_decode_attn<8>
+                             : nullptr;
+    if (kern == nullptr) return set_error(TRMOE_ERR_UNSUPPORTED, "decode_attention: 1, 2, 4, 7 or 8 query heads per kv head");
+    hipLaunchKernelGGL(kern, grid, dim3(256), 0, stream, a, chunk, splits);
+    return check_launch("decode_attention");
+}
+
+}  // namespace trmoe

@@ -408,6 +408,37 @@ int trmoe_pack_fragments(int dtype, const void* packed, int64_t rows, int64_t co
                          void* stream);
 
 /* ---------------------------------------------------------------------------
+ * The attention half of a decoder block (gqa.py:88-165, rotary.py:17-80), bf16,
+ * heads of 64.  kqv rows hold the fused projection: num_kv_heads k heads,
+ * num_heads q heads, num_kv_heads v heads.  cos / sin are fp32 [positions, 64]
+ * (both halves of a row alike); the caches are [sequence, kv head,
+ * cache_length, 64].
+ *
+ * trmoe_qk_norm_rope: q = rope(rmsnorm(q) * q_weight) into q [sequence, token,
+ * num_heads, 64], k likewise and v into the caches, token t at position
+ * first_position + t (+ *position, a device counter, when given; a position
+ * past the cache is dropped).
+ *
+ * trmoe_decode_attention: one token per sequence (batch <= 16) at the device
+ * position *position: the projection of rmsnorm(hidden) * norm_weight through
+ * w_kqv [(num_heads + 2 num_kv_heads) * 64, hidden], q and k normed and
+ * rotated, k and v stored at the position, and softmax(scale q K^T) V over
+ * positions 0 .. *position into attn [batch, num_heads * 64]; query head h
+ * reads kv head h / (num_heads / num_kv_heads).
+ * ------------------------------------------------------------------------- */
+int trmoe_qk_norm_rope(const void* kqv, int64_t sequences, int64_t tokens, int num_heads, int num_kv_heads,
+                       int64_t ldkqv, const void* q_weight, const void* k_weight, float eps, const float* cos,
+                       const float* sin, int64_t positions, int64_t first_position, const int64_t* position, void* q,
+                       void* k_cache, void* v_cache, int64_t cache_length, void* stream);
+size_t trmoe_decode_attention_workspace_bytes(int64_t batch, int64_t hidden, int num_heads, int num_kv_heads,
+                                              int64_t cache_length);
+int trmoe_decode_attention(const void* hidden_rows, int64_t batch, int64_t hidden, int64_t ldx, const void* norm_weight,
+                           float norm_eps, const void* w_kqv, int num_heads, int num_kv_heads, const void* q_weight,
+                           const void* k_weight, float qk_eps, const float* cos, const float* sin, int64_t positions,
+                           const int64_t* position, void* k_cache, void* v_cache, int64_t cache_length, float scale,
+                           void* attn, void* workspace, size_t workspace_bytes, void* stream);
+
+/* ---------------------------------------------------------------------------
  * Decode (n_tokens <= 128) of a layer with e4m3 weights: the shared branch and
  * every expert in one gate|up and one down over the concatenated features
  *     [shared (padded to 128) | expert 0 (padded to 64) | expert 1 | ...],
