@@ -161,8 +161,12 @@ class GQAttention(nn.Module):
         return q, k, v
 
     def prefill_attention(self, q, k, v) -> torch.Tensor:
-        """Causal SDPA over the prompt, key/value heads repeated (gqa.py:150-152, 229-266)."""
+        """Causal SDPA over the prompt; each key/value head serves kv_groups
+        query heads (gqa.py:150-152, 229-266).  The reduced-precision kernels
+        take the grouped heads as they are, without a repeated copy."""
         g = self.cfg.kv_groups
+        if q.device.type == "cuda" and q.dtype != torch.float32 and sdpa_kernel is not None:
+            return _sdpa(q, k, v, None, causal=True, scale=self.scale, grouped=g > 1)
         k = k.repeat_interleave(g, dim=1)
         v = v.repeat_interleave(g, dim=1)
         return _sdpa(q, k, v, None, causal=True, scale=self.scale)
@@ -181,12 +185,15 @@ class GQAttention(nn.Module):
         return self.o_proj(attn.transpose(1, 2).reshape(B, T, -1))
 
 
-def _sdpa(q, k, v, mask, *, causal: bool, scale: float) -> torch.Tensor:
+def _sdpa(q, k, v, mask, *, causal: bool, scale: float, grouped: bool = False) -> torch.Tensor:
     """SDPA on the flash / memory-efficient kernels for reduced precision (the
     math kernel raises instead of running); any kernel for fp32."""
     if q.dtype == torch.float32 or sdpa_kernel is None:
         return F.scaled_dot_product_attention(q, k, v, attn_mask=mask, is_causal=causal, scale=scale)
     with sdpa_kernel([SDPBackend.FLASH_ATTENTION, SDPBackend.EFFICIENT_ATTENTION]):
+        if grouped:
+            return F.scaled_dot_product_attention(q, k, v, attn_mask=mask, is_causal=causal, scale=scale,
+                                                  enable_gqa=True)
         return F.scaled_dot_product_attention(q, k, v, attn_mask=mask, is_causal=causal, scale=scale)
 
 

@@ -41,12 +41,21 @@ __device__ __forceinline__ u32x4 pack8(const float (&f)[8]) {
     for (int j = 0; j < 8; ++j) r[j] = (bf16_t)f[j];
     return __builtin_bit_cast(u32x4, r);
 }
-__device__ __forceinline__ float sum8(float s) {   // over the 8 lanes of a head row
-    s += __shfl_xor(s, 1);
-    s += __shfl_xor(s, 2);
-    s += __shfl_xor(s, 4);
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+}
+constexpr int kQuadXor1 = 0xB1, kQuadXor2 = 0x4E, kQuadXor3 = 0x1B, kHalfMirror = 0x141, kRor8 = 0x128;
+// Over the 8 lanes of a head row, on the vector ALU alone (the mirror reaches
+// the other quad, whose lanes all hold its sum).
+__device__ __forceinline__ float sum8(float s) {
+    s += dpp<kQuadXor1>(s);
+    s += dpp<kQuadXor2>(s);
+    s += dpp<kHalfMirror>(s);
     return s;
 }
+// The value of the lane 4 away in its 8: i ^ 7, then ^ 3.
+__device__ __forceinline__ float xor4(float v) { return dpp<kQuadXor3>(dpp<kHalfMirror>(v)); }
 
 // x (the lane's 8 of a head row's 64 elements) -> rope(rmsnorm(x) * w) at one
 // position: element d pairs with d +- 32, which the lane 4 away holds.
@@ -63,7 +72,7 @@ __device__ __forceinline__ void norm_rope(float (&x)[8], const bf16_t* w, float 
     const float sign = c < 4 ? -1.0f : 1.0f;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-        const float other = __shfl_xor(x[j], 4);
+        const float other = xor4(x[j]);
         x[j] = x[j] * cos[8 * c + j] + sign * other * sin[8 * c + j];
     }
 }
@@ -173,84 +182,106 @@ __device__ __forceinline__ float load_dev(const float* p) {
 // Attention of one new token: workgroup (split, kv head, sequence) takes the
 // cache positions [split * chunk, + chunk) below the current one; the split
 // that holds the current position normalises, rotates and stores its k and v
-// and adds it.  Eight lanes hold one position's 64 elements (so each K and V
-// row is one 128-byte read) for all G query heads of the group, with a
-// running maximum and sum per head; 32 positions are in flight per workgroup
-// and kUnroll loads per lane.  A CU moves its K/V bytes at the vector ALU's
-// pace, so the positions are split until about every CU has a workgroup.
+// and adds it.  Eight lanes hold one position's 64 elements, so each K and V
+// row is one 128-byte read, with a running maximum and sum per query head.
+// The G heads of the group are spread over the waves (HPW each), so that a
+// wave normalises and merges only its own; with few heads several waves share
+// them and split the positions (PW).  A step of one sequence has little
+// else to hide latency behind: the first K/V rows are requested before the
+// position is known, and reductions stay on the vector ALU.  Against all heads
+// in every wave and one 128-position split: 14.2 us at 213 positions before.
 constexpr int kUnroll = 4;
+constexpr int kMaxSplits = 64;
+constexpr int kPart = kD + 2;   // 64 sums, the maximum, the weight
+template <int G>
+struct HeadSplit {
+    static constexpr int HW = G >= 4 ? 4 : G;          // waves over heads
+    static constexpr int PW = 4 / HW;                  // waves over positions
+    static constexpr int HPW = (G + HW - 1) / HW;      // heads per wave
+};
+
 template <int G>
 __global__ __launch_bounds__(256) void k_decode_attn(DecodeAttnArgs a, int chunk, int splits) {
-    __shared__ float s_ml[4][G][2];
-    __shared__ float s_acc[4][G][kD];
+    using HS = HeadSplit<G>;
+    constexpr int HPW = HS::HPW, PW = HS::PW;
+    __shared__ float s_ml[PW][G][2];
+    __shared__ float s_acc[PW][G][kD];
+    __shared__ float s_f[G][kMaxSplits + 1];
     __shared__ int s_last;
     const int split = (int)blockIdx.x, kvh = (int)blockIdx.y, b = (int)blockIdx.z;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int c = lane & 7, grp = threadIdx.x >> 3;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    const int hw = wave / PW, pw = wave % PW;
+    const int c = lane & 7, grp = pw * 8 + (lane >> 3);
+    constexpr int kStep = 8 * PW;
+    const int p0 = split * chunk;
+    const int64_t head_off = ((int64_t)b * a.kvh + kvh) * a.L * kD;
+    const bf16_t* kc = a.k_cache + head_off + 8 * c;
+    const bf16_t* vc = a.v_cache + head_off + 8 * c;
+    u32x4 kv[kUnroll], vv[kUnroll];
+    auto load = [&](int p) {   // rows at or past the current position are read (inside the cache) and not used
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u) {
+            const int64_t pp = std::min<int64_t>(p + kStep * u, a.L - 1);
+            kv[u] = *reinterpret_cast<const u32x4*>(kc + pp * kD);
+            vv[u] = *reinterpret_cast<const u32x4*>(vc + pp * kD);
+        }
+    };
+    load(p0 + grp);
     int64_t pos64 = *a.pos;
     pos64 = pos64 < 0 ? 0 : (pos64 >= a.L ? a.L - 1 : pos64);
     const int pos = (int)pos64;
-    const int p0 = split * chunk, p1 = std::min(p0 + chunk, pos);
+    const int p1 = std::min(p0 + chunk, pos);
     const bool own = pos >= p0 && pos < p0 + chunk;
     const float* row = a.qkv + (int64_t)b * a.n_qkv;
     const float* cosp = a.cos + (int64_t)pos * kD;
     const float* sinp = a.sin + (int64_t)pos * kD;
-    const int64_t head_off = ((int64_t)b * a.kvh + kvh) * a.L * kD;
-    const bf16_t* kc = a.k_cache + head_off + 8 * c;
-    const bf16_t* vc = a.v_cache + head_off + 8 * c;
 
-    float q[G][8];
+    float q[HPW][8], m[HPW], l[HPW], acc[HPW][8];
 #pragma unroll
-    for (int g = 0; g < G; ++g) {
+    for (int i = 0; i < HPW; ++i) {
+        const int g = std::min(hw * HPW + i, G - 1);   // the last wave may repeat a head and drop it
         const float* src = row + (a.kvh + kvh * G + g) * kD + 8 * c;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) q[g][j] = src[j];
-        norm_rope(q[g], a.qn_w, a.qk_eps, cosp, sinp, c);
+        for (int j = 0; j < 8; ++j) q[i][j] = src[j];
+        norm_rope(q[i], a.qn_w, a.qk_eps, cosp, sinp, c);
+        m[i] = -1e30f;
+        l[i] = 0.f;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) q[g][j] *= a.scale * 1.4426950408889634f;   // exp2 below
-    }
-    float m[G], l[G], acc[G][8];
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-        m[g] = -1e30f;
-        l[g] = 0.f;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) acc[g][j] = 0.f;
+        for (int j = 0; j < 8; ++j) {
+            q[i][j] *= a.scale * 1.4426950408889634f;   // exp2 below
+            acc[i][j] = 0.f;
+        }
     }
     auto attend = [&](const float (&kf)[8], const float (&vf)[8]) {
 #pragma unroll
-        for (int g = 0; g < G; ++g) {
+        for (int i = 0; i < HPW; ++i) {
             float s = 0.f;
 #pragma unroll
-            for (int j = 0; j < 8; ++j) s += q[g][j] * kf[j];
+            for (int j = 0; j < 8; ++j) s += q[i][j] * kf[j];
             s = sum8(s);
-            const float mn = fmaxf(m[g], s);
-            const float f = __builtin_amdgcn_exp2f(m[g] - mn), p = __builtin_amdgcn_exp2f(s - mn);
-            m[g] = mn;
-            l[g] = l[g] * f + p;
+            const float mn = fmaxf(m[i], s);
+            const float f = __builtin_amdgcn_exp2f(m[i] - mn), p = __builtin_amdgcn_exp2f(s - mn);
+            m[i] = mn;
+            l[i] = l[i] * f + p;
 #pragma unroll
-            for (int j = 0; j < 8; ++j) acc[g][j] = acc[g][j] * f + p * vf[j];
+            for (int j = 0; j < 8; ++j) acc[i][j] = acc[i][j] * f + p * vf[j];
         }
     };
-    for (int p = p0 + grp; p < p1; p += 32 * kUnroll) {
-        u32x4 kv[kUnroll], vv[kUnroll];
+    for (int p = p0 + grp;;) {
 #pragma unroll
         for (int u = 0; u < kUnroll; ++u) {
-            const int pp = std::min(p + 32 * u, p1 - 1);
-            kv[u] = *reinterpret_cast<const u32x4*>(kc + (int64_t)pp * kD);
-            vv[u] = *reinterpret_cast<const u32x4*>(vc + (int64_t)pp * kD);
-        }
-#pragma unroll
-        for (int u = 0; u < kUnroll; ++u) {
-            if (p + 32 * u < p1) {   // uniform over the position's 8 lanes
+            if (p + kStep * u < p1) {   // uniform over the position's 8 lanes
                 float kf[8], vf[8];
                 unpack8(kv[u], kf);
                 unpack8(vv[u], vf);
                 attend(kf, vf);
             }
         }
+        p += kStep * kUnroll;
+        if (p >= p1) break;
+        load(p);
     }
-    if (own && threadIdx.x < kLanes) {
+    if (own && pw == 0 && lane < kLanes) {
         float kf[8], vf[8];
         const float* ks = row + kvh * kD + 8 * c;
         const float* vs = row + (a.kvh + a.kvh * G + kvh) * kD + 8 * c;
@@ -261,49 +292,50 @@ __global__ __launch_bounds__(256) void k_decode_attn(DecodeAttnArgs a, int chunk
         }
         norm_rope(kf, a.kn_w, a.qk_eps, cosp, sinp, c);
         const u32x4 kb = pack8(kf), vb = pack8(vf);
-        *reinterpret_cast<u32x4*>(a.k_cache + head_off + (int64_t)pos * kD + 8 * c) = kb;
-        *reinterpret_cast<u32x4*>(a.v_cache + head_off + (int64_t)pos * kD + 8 * c) = vb;
+        if (hw == 0) {
+            *reinterpret_cast<u32x4*>(a.k_cache + head_off + (int64_t)pos * kD + 8 * c) = kb;
+            *reinterpret_cast<u32x4*>(a.v_cache + head_off + (int64_t)pos * kD + 8 * c) = vb;
+        }
         unpack8(kb, kf);   // what later steps will read
         unpack8(vb, vf);
         attend(kf, vf);
     }
-    // merge the wave's 8 positions, then the 4 waves
+    // merge the wave's 8 positions
 #pragma unroll
-    for (int off = 8; off < 64; off <<= 1) {
+    for (int i = 0; i < HPW; ++i) {
+        auto merge = [&](auto other) {
+            const float mo = other(m[i]), lo = other(l[i]);
+            const float mn = fmaxf(m[i], mo);
+            const float f = __builtin_amdgcn_exp2f(m[i] - mn), fo = __builtin_amdgcn_exp2f(mo - mn);
+            m[i] = mn;
+            l[i] = l[i] * f + lo * fo;
 #pragma unroll
-        for (int g = 0; g < G; ++g) {
-            const float mo = __shfl_xor(m[g], off), lo = __shfl_xor(l[g], off);
-            const float mn = fmaxf(m[g], mo);
-            const float f = __builtin_amdgcn_exp2f(m[g] - mn), fo = __builtin_amdgcn_exp2f(mo - mn);
-            m[g] = mn;
-            l[g] = l[g] * f + lo * fo;
+            for (int j = 0; j < 8; ++j) acc[i][j] = acc[i][j] * f + other(acc[i][j]) * fo;
+        };
+        merge([](float v) { return dpp<kRor8>(v); });
+        merge([](float v) { return __shfl_xor(v, 16); });
+        merge([](float v) { return __shfl_xor(v, 32); });
+        const int g = hw * HPW + i;
+        if (lane < kLanes && g < G) {
 #pragma unroll
-            for (int j = 0; j < 8; ++j) acc[g][j] = acc[g][j] * f + __shfl_xor(acc[g][j], off) * fo;
-        }
-    }
-    if (lane < kLanes) {
-#pragma unroll
-        for (int g = 0; g < G; ++g) {
-#pragma unroll
-            for (int j = 0; j < 8; ++j) s_acc[wave][g][8 * c + j] = acc[g][j];
+            for (int j = 0; j < 8; ++j) s_acc[pw][g][8 * c + j] = acc[i][j];
             if (c == 0) {
-                s_ml[wave][g][0] = m[g];
-                s_ml[wave][g][1] = l[g];
+                s_ml[pw][g][0] = m[i];
+                s_ml[pw][g][1] = l[i];
             }
         }
     }
     __syncthreads();
     bf16_t* out = a.attn + (int64_t)b * (a.kvh * G * kD) + kvh * G * kD;
-    constexpr int kPart = kD + 2;   // 64 sums, the maximum, the weight
     float* part = a.part + ((int64_t)(b * a.kvh + kvh) * splits) * (G * kPart);
     for (int i = threadIdx.x; i < G * kD; i += 256) {
         const int g = i / kD, d = i % kD;
         float mn = s_ml[0][g][0];
 #pragma unroll
-        for (int w = 1; w < 4; ++w) mn = fmaxf(mn, s_ml[w][g][0]);
+        for (int w = 1; w < PW; ++w) mn = fmaxf(mn, s_ml[w][g][0]);
         float lt = 0.f, v = 0.f;
 #pragma unroll
-        for (int w = 0; w < 4; ++w) {
+        for (int w = 0; w < PW; ++w) {
             const float f = __builtin_amdgcn_exp2f(s_ml[w][g][0] - mn);
             lt += s_ml[w][g][1] * f;
             v += s_acc[w][g][d] * f;
@@ -328,19 +360,32 @@ __global__ __launch_bounds__(256) void k_decode_attn(DecodeAttnArgs a, int chunk
                  splits - 1;
     __syncthreads();
     if (!s_last) return;
+    // the splits' factors, one lane per split, then the weighted sums
+    for (int g = wave; g < G; g += 4) {
+        const float* src = part + ((int64_t)lane * G + g) * kPart + kD;
+        const float ms = lane < splits ? load_dev(src) : -1e30f, ls = lane < splits ? load_dev(src + 1) : 0.f;
+        float mx = ms;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
+        const float f = __builtin_amdgcn_exp2f(ms - mx);
+        float lt = ls * f;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) lt += __shfl_xor(lt, off);
+        s_f[g][lane] = f / lt;
+    }
+    __syncthreads();
     for (int i = threadIdx.x; i < G * kD; i += 256) {
         const int g = i / kD, d = i % kD;
-        float mn = -1e30f, lt = 0.f, v = 0.f;
-        for (int s = 0; s < splits; ++s) {
-            const float* src = part + ((int64_t)s * G + g) * kPart;
-            const float ms = load_dev(src + kD), ls = load_dev(src + kD + 1), vs = load_dev(src + d);
-            const float m2 = fmaxf(mn, ms);
-            const float f = __builtin_amdgcn_exp2f(mn - m2), fs = __builtin_amdgcn_exp2f(ms - m2);
-            mn = m2;
-            lt = lt * f + ls * fs;
-            v = v * f + vs * fs;
+        const float* src = part + (int64_t)g * kPart + d;
+        float v = 0.f;
+        for (int s = 0; s < splits; s += 8) {
+            float t[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) t[u] = load_dev(src + (int64_t)std::min(s + u, splits - 1) * (G * kPart));
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v += s + u < splits ? t[u] * s_f[g][s + u] : 0.f;
         }
-        out[i] = (bf16_t)(v / lt);
+        out[i] = (bf16_t)v;
     }
 }
 
@@ -352,14 +397,13 @@ int launch_qk_rope(const RopeArgs& a, hipStream_t stream) {
     return check_launch("qk_norm_rope");
 }
 
-// Positions per split: at least 128 (4 per lane group), more when the
-// (sequence, kv head) pairs alone fill the CUs.
+// Positions per split: at least 64 (two batches of a lane group's loads), more
+// when the (sequence, kv head) pairs fill the CUs twice over or the splits
+// would pass one lane each in the merge.
 static int decode_chunk(int64_t L, int pairs) {
-    int splits = std::max(1, 256 / std::max(1, pairs));
-    const int most = (int)((L + 127) / 128);
-    splits = std::min(splits, most);
-    int chunk = (int)((L + splits - 1) / splits);
-    return (chunk + 31) / 32 * 32;
+    int64_t splits = std::max(1, 512 / std::max(1, pairs));
+    splits = std::min<int64_t>({splits, (L + 63) / 64, kMaxSplits});
+    return (int)(((L + splits - 1) / splits + 31) / 32 * 32);
 }
 
 int64_t decode_attn_splits(int64_t L, int pairs) {
