@@ -43,6 +43,29 @@ class CallExtras(ctypes.Structure):
 
 _c_extras = ctypes.POINTER(CallExtras)
 
+
+class DecoderDims(ctypes.Structure):
+    """trmoe_decoder_dims (include/trmoe.h)."""
+
+    _fields_ = [
+        *((n, ctypes.c_int64) for n in ("layers", "hidden", "cache_length", "vocab_size", "shared_width",
+                                        "expert_width")),
+        *((n, ctypes.c_int32) for n in ("num_heads", "num_kv_heads", "num_experts", "top_k")),
+        *((n, ctypes.c_float) for n in ("norm_eps", "qk_eps", "attn_scale", "shared_scale", "routed_scale")),
+        ("route_weights", ctypes.c_float * 4),
+    ]
+
+
+class DecoderLayer(ctypes.Structure):
+    """trmoe_decoder_layer (include/trmoe.h)."""
+
+    _fields_ = [(n, ctypes.c_void_p) for n in (
+        "input_norm", "w_kqv", "q_norm", "k_norm", "w_o", "k_cache", "v_cache", "w_gate_up", "w_gate_up_frag",
+        "w_down", "w_down_frag", "route_table")]
+
+
+_c_dims = ctypes.POINTER(DecoderDims)
+
 SIGNATURES = {
     "trmoe_abi_version": (_c_int, []),
     "trmoe_last_error": (ctypes.c_char_p, []),
@@ -138,6 +161,11 @@ SIGNATURES = {
         _c_int,
         [_c_vp, _c_i64, _c_i64, _c_i64, _c_vp, _c_float, _c_vp, _c_int, _c_int, _c_vp, _c_vp, _c_float, _c_vp, _c_vp,
          _c_i64, _c_vp, _c_vp, _c_vp, _c_i64, _c_float, _c_vp, _c_vp, _c_size, _c_vp],
+    ),
+    "trmoe_decoder_step_workspace_bytes": (_c_size, [_c_dims, _c_i64]),
+    "trmoe_decoder_step": (
+        _c_int,
+        [_c_dims, _c_vp, _c_vp, _c_i64, _c_vp, _c_vp, _c_vp, _c_vp, _c_i64, _c_vp, _c_size, _c_vp],
     ),
     "trmoe_pack_fragments_e4m3": (_c_int, [_c_vp, _c_i64, _c_i64, _c_i64, _c_vp, _c_i64, _c_i64, _c_vp]),
     "trmoe_gate_up_e4m3_decode": (

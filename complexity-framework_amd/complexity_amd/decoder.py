@@ -213,6 +213,120 @@ class TRGQABlock(nn.Module):
         self.layer_index = layer_index
 
 
+def _plain(mod: nn.Module, cls: type) -> bool:
+    """A module of exactly `cls` (so not parametrized or replaced) without
+    hooks or bias, its weight in bf16: what a kernel may stand in for."""
+    if type(mod) is not cls or mod._forward_hooks or mod._forward_pre_hooks:
+        return False
+    w = mod._parameters.get("weight")
+    return w is not None and w.dtype is torch.bfloat16 and w.is_contiguous() and mod._parameters.get("bias") is None
+
+
+class _StepPlan:
+    """The layers of a decode step as one native call takes them
+    (``trmoe_decoder_step``): the pointers of every block's weights, packs and
+    caches, with what they were read from.  ``current`` looks at all of it
+    again before each step: module and parameter objects, in-place versions,
+    storage, packs, routing.  Without it a step spends about 100 us per layer
+    in Python, against 30 us of kernels."""
+
+    def __init__(self):
+        self.dims = ops.N.DecoderDims()
+        self.layers = None
+        self.engines = []   # (engine, config, strategy, E, W, pack entry, route table)
+        self.members = []   # (owner's dict, name, object)
+        self.tensors = []   # (owner's dict, name, tensor, version, pointer)
+        self.keep = []      # what the pointers point into
+
+    def _watch(self, owner: nn.Module, name: str) -> nn.Module:
+        mod = owner._modules[name]
+        self.members.append((owner._modules, name, mod))
+        return mod
+
+    def _weight(self, owner: nn.Module, name: str) -> torch.Tensor:
+        t = owner._parameters[name]
+        self.tensors.append((owner._parameters, name, t, t._version, t.data_ptr()))
+        return t
+
+    @classmethod
+    def build(cls, dec: "TRGQADecoder", device: torch.device) -> Optional["_StepPlan"]:
+        """None when a block needs the general path: a replaced MLP half,
+        adapted or e4m3 weights, grouped experts, layers that differ in shape."""
+        if dec.mlp_fn is not None:
+            return None
+        plan = cls()
+        cfg, rows, shapes = dec.cfg, [], set()
+        for i, (name, block) in enumerate(dec.layers._modules.items()):
+            plan.members.append((dec.layers._modules, name, block))
+            attn, mlp = plan._watch(block, "self_attn"), plan._watch(block, "mlp")
+            norm_in, norm_post = plan._watch(block, "input_layernorm"), plan._watch(block, "post_attention_layernorm")
+            if not _plain(norm_post, RMSNorm) or type(mlp) is not TRHashEngine or mlp._fp8:
+                return None
+            for n in ("shared_gate", "shared_up", "shared_down"):
+                mod = mlp._modules.get(n)
+                plan.members.append((mlp._modules, n, mod))
+                if mod is not None:
+                    if type(mod) is not nn.Linear:
+                        return None
+                    plan._weight(mod, "weight")
+            if any(n not in mlp._parameters for n in ("expert_gate", "expert_up", "expert_down")):
+                return None   # parametrized
+            for n in ("expert_gate", "expert_up", "expert_down"):
+                plan._weight(mlp, n)
+            decision = mlp._decide(plan._weight(norm_post, "weight"))
+            if decision.selected is not TRHashBackend.HIP:
+                return None
+            packed = mlp._hip_packed(norm_post.weight)
+            if packed.strategy != ops.STRATEGY_DENSE or packed.act_dtype is not torch.bfloat16:
+                return None
+            c, table = mlp.config, mlp._active_route_table
+            if table.dtype is not torch.int64 or not table.is_contiguous():
+                return None
+            shapes.add((packed.shared_width, packed.num_experts, packed.expert_width, tuple(table.shape),
+                        tuple(c.route_weights), c.shared_output_scale, c.routed_output_scale, norm_in.eps,
+                        norm_post.eps, attn.q_norm.eps, attn.k_norm.eps, attn.scale))
+            for n in ("k_proj", "q_proj", "v_proj"):
+                plan._weight(plan._watch(attn, n), "weight")
+            kqv = attn.kqv_weight()
+            gu = packed.fragments("dense_gate_up", cfg.hidden_size)[0]
+            dn = packed.fragments("dense_down", packed.dense_features)[0]
+            ptrs = (plan._weight(norm_in, "weight"), kqv, plan._weight(plan._watch(attn, "q_norm"), "weight"),
+                    plan._weight(plan._watch(attn, "k_norm"), "weight"),
+                    plan._weight(plan._watch(attn, "o_proj"), "weight"), dec.k_cache[i], dec.v_cache[i],
+                    packed.dense_gate_up, gu, packed.dense_down, dn, table)
+            if any(t.data_ptr() % 16 for t in ptrs) or kqv.dtype is not torch.bfloat16:
+                return None
+            plan.keep.append(ptrs)
+            rows.append(ops.N.DecoderLayer(*(t.data_ptr() for t in ptrs)))
+            plan.engines.append((mlp, c, mlp.routed_strategy, mlp._active_num_experts, mlp._active_expert_width,
+                                 mlp._packed_norm, table))
+            mlp.last_backend, mlp.last_norm = decision, "fused"
+        if len(shapes) != 1:
+            return None
+        S, E, W, (top_k, vocab), rw, ss, rs, e_in, e_post, e_q, e_k, scale = shapes.pop()
+        if e_in != e_post or e_q != e_k or e_in <= 0.0:
+            return None
+        d = plan.dims
+        d.layers, d.hidden, d.cache_length, d.vocab_size = len(rows), cfg.hidden_size, dec.k_cache[0].shape[2], vocab
+        d.shared_width, d.expert_width, d.num_experts, d.top_k = S, W, E, top_k
+        d.num_heads, d.num_kv_heads = cfg.num_heads, cfg.num_kv_heads
+        d.norm_eps, d.qk_eps, d.attn_scale, d.shared_scale, d.routed_scale = e_in, e_q, scale, ss, rs
+        d.route_weights[:] = (list(rw) + [0.0] * 4)[:4]
+        plan.layers = (ops.N.DecoderLayer * len(rows))(*rows)
+        return plan
+
+    def current(self, dec: "TRGQADecoder") -> bool:
+        if dec.mlp_fn is not None or len(dec.layers) != len(self.engines):
+            return False
+        for eng, cfg, strategy, E, W, entry, table in self.engines:
+            if (eng._packed_norm is not entry or eng.config is not cfg or eng.routed_strategy != strategy
+                    or eng._active_num_experts != E or eng._active_expert_width != W
+                    or eng._active_route_table is not table or eng._fp8):
+                return False
+        return (all(d.get(n) is m for d, n, m in self.members)
+                and all(d.get(n) is t and t._version == v and t.data_ptr() == p for d, n, t, v, p in self.tensors))
+
+
 # Replaces a block's MLP half (tests compare against a decoder whose MLPs run
 # another definition): (layer index, h [B, T, H], token ids [B, T], block)
 # -> h + mlp(post_attention_layernorm(h)).
@@ -235,6 +349,7 @@ class TRGQADecoder(nn.Module):
         self._pos: Optional[torch.Tensor] = None   # device int64 [1]: next decode position
         self._rope = None
         self._rope32 = None
+        self._step_plan: Optional[_StepPlan] = None
         self._graph = None
 
     # ------------------------------------------------------------------ weights
@@ -281,11 +396,22 @@ class TRGQADecoder(nn.Module):
 
     def _hip_attention(self, device: torch.device) -> bool:
         """Whether the attention half runs on the HIP kernels: bf16 on a GPU,
-        dimensions they take, and a decoder that is not pinned to PYTORCH."""
+        dimensions they take, a decoder that is not pinned to PYTORCH, and
+        modules as built here (a replaced, adapted or hooked one is called)."""
         cfg = self.cfg
-        return (device.type == "cuda" and self.embed_tokens.weight.dtype == torch.bfloat16
-                and self.layers[0].mlp.config.backend is not TRHashBackend.PYTORCH
-                and ops.attention_unsupported(cfg.hidden_size, cfg.num_heads, cfg.num_kv_heads, cfg.head_dim) is None)
+        if (device.type != "cuda" or self.embed_tokens.weight.dtype is not torch.bfloat16
+                or ops.attention_unsupported(cfg.hidden_size, cfg.num_heads, cfg.num_kv_heads, cfg.head_dim)):
+            return False
+        for block in self.layers:
+            m = block._modules
+            attn = m["self_attn"]
+            if type(attn) is not GQAttention or m["mlp"].config.backend is TRHashBackend.PYTORCH:
+                return False
+            a = attn._modules
+            if not (_plain(m["input_layernorm"], RMSNorm) and _plain(a["q_norm"], RMSNorm)
+                    and _plain(a["k_norm"], RMSNorm) and _plain(a["o_proj"], nn.Linear)):
+                return False
+        return True
 
     def _norm(self, norm: RMSNorm, h: torch.Tensor, hip: bool) -> torch.Tensor:
         if not hip:
@@ -293,7 +419,9 @@ class TRGQADecoder(nn.Module):
         return ops.rmsnorm_forward(h.reshape(-1, h.shape[-1]), norm.weight, norm.eps)[0].view(h.shape)
 
     def logits(self, h: torch.Tensor) -> torch.Tensor:
-        hip = not torch.is_grad_enabled() and self._hip_attention(h.device)
+        hip = (not torch.is_grad_enabled() and h.device.type == "cuda" and h.dtype is torch.bfloat16
+               and _plain(self.norm, RMSNorm) and ops.rmsnorm_unsupported(h, self.norm.weight) is None
+               and self.layers[0].mlp.config.backend is not TRHashBackend.PYTORCH)
         return F.linear(self._norm(self.norm, h, hip), self.embed_tokens.weight)
 
     # ------------------------------------------------------------------ prompt
@@ -320,6 +448,7 @@ class TRGQADecoder(nn.Module):
                 c[:, :, T:].zero_()
         self.cache_len = T
         self._graph = None
+        self._step_plan = None
         hip = self._hip_attention(dev)
         if hip:
             cos, sin = self._rope_tables32(L, dev)
@@ -382,6 +511,11 @@ class TRGQADecoder(nn.Module):
         cos, sin = self._rope_tables32(L, ids.device)
         tok = ids.view(B, 1)
         h = self.embed_tokens(ids)
+        if self._step_plan is None or not self._step_plan.current(self):
+            self._step_plan = _StepPlan.build(self, ids.device)
+        if self._step_plan is not None and h.is_contiguous():
+            ops.decoder_step(h, self._step_plan.dims, self._step_plan.layers, ids.contiguous(), pos, cos, sin)
+            return self.logits(h)
         for i, block in enumerate(self.layers):
             attn, norm = block.self_attn, block.input_layernorm
             a = ops.decode_attention(h, norm.weight, norm.eps, attn.kqv_weight(), cfg.num_heads, attn.q_norm.weight,

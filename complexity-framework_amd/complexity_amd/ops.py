@@ -639,6 +639,25 @@ def decode_linear(x: torch.Tensor, weight: torch.Tensor, residual: Optional[torc
     return shared_down_combine(x, k, weight, None, weight.shape[0], None, None, 1, (1.0,), 1.0, 0.0, residual)
 
 
+@_on_tensor_device
+def decoder_step(h: torch.Tensor, dims: N.DecoderDims, layers, token_ids: torch.Tensor, position: torch.Tensor,
+                 cos: torch.Tensor, sin: torch.Tensor) -> None:
+    """trmoe_decoder_step: h [B, hidden] (contiguous, bf16) goes through every
+    layer of `layers` (an array of N.DecoderLayer) in place."""
+    lib = _lib()
+    _require_cuda(h, token_ids, position, cos, sin)
+    if h.dtype != torch.bfloat16 or not h.is_contiguous() or h.shape[1] != dims.hidden or len(layers) != dims.layers \
+            or token_ids.dtype != torch.int64 or token_ids.numel() != h.shape[0] or not token_ids.is_contiguous() \
+            or position.dtype != torch.int64:
+        raise ValueError("decoder_step: shapes or dtypes do not match")
+    n = h.shape[0]
+    ws_bytes = lib.trmoe_decoder_step_workspace_bytes(ctypes.byref(dims), n)
+    ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=h.device)
+    st = lib.trmoe_decoder_step(ctypes.byref(dims), ctypes.cast(layers, ctypes.c_void_p), _p(h), n, _p(token_ids),
+                                _p(position), _p(cos), _p(sin), cos.shape[0], _p(ws), ws_bytes, _stream(h))
+    N.check(st, "trmoe_decoder_step")
+
+
 def _extras(row_scale: Optional[torch.Tensor] = None, rms_eps: float = 0.0, w_frag=None):
     """trmoe_call_extras for the *_ex calls; w_frag = (fragment copy, cols)."""
     e = N.CallExtras()

@@ -1055,6 +1055,89 @@ int trmoe_decode_attention(const void* hidden_rows, int64_t batch, int64_t hidde
     return launch_decode_attn(a, num_heads / num_kv_heads, as_stream(stream));
 }
 
+// Scratch of trmoe_decoder_step: two hidden buffers, the attention output, the
+// SwiGLU features, then the split partials of the down kernels and the
+// attention's own scratch (used at different times, kept apart).
+struct StepScratch {
+    size_t h, attn, feats, down, attn_ws, total;
+};
+
+static bool step_dims(const trmoe_decoder_dims* d, int64_t batch, StepScratch* s) {
+    if (d == nullptr || !decode_attn_dims_ok(batch, d->hidden, d->num_heads, d->num_kv_heads, d->cache_length)) return false;
+    if (d->shared_width < 0 || d->num_experts < 1 || d->num_experts > kMaxExperts || d->expert_width < 1 ||
+        d->vocab_size < 1 || d->top_k < 1 || d->top_k > kMaxTopK || d->top_k > d->num_experts || d->layers < 1)
+        return false;
+    const int64_t feats = trmoe_dense_routed_features(d->shared_width, d->num_experts, d->expert_width);
+    const int64_t qd = (int64_t)d->num_heads * 64;
+    auto up = [](size_t v) { return (v + 255) / 256 * 256; };
+    s->h = up((size_t)batch * (size_t)d->hidden * 2);
+    s->attn = up((size_t)batch * (size_t)qd * 2);
+    s->feats = up((size_t)batch * (size_t)feats * 2);
+    const size_t down_o = down_skinny_workspace_bytes(batch, d->hidden, qd, TRMOE_BF16);
+    const size_t down_m = down_skinny_workspace_bytes(batch, d->hidden, feats, TRMOE_BF16);
+    s->down = up(down_o > down_m ? down_o : down_m);
+    s->attn_ws = up(trmoe_decode_attention_workspace_bytes(batch, d->hidden, d->num_heads, d->num_kv_heads,
+                                                           d->cache_length));
+    s->total = s->h + s->attn + s->feats + s->down + s->attn_ws;
+    return true;
+}
+
+size_t trmoe_decoder_step_workspace_bytes(const trmoe_decoder_dims* dims, int64_t batch) {
+    StepScratch s;
+    return step_dims(dims, batch, &s) ? s.total : 0;
+}
+
+int trmoe_decoder_step(const trmoe_decoder_dims* d, const trmoe_decoder_layer* layers, void* hidden_rows, int64_t batch,
+                       const int64_t* token_ids, const int64_t* position, const float* cos, const float* sin,
+                       int64_t positions, void* workspace, size_t workspace_bytes, void* stream) {
+    StepScratch s;
+    TRMOE_REQUIRE(step_dims(d, batch, &s), "decoder_step: dimensions outside trmoe_decode_attention's or the layer's");
+    TRMOE_REQUIRE(layers && hidden_rows && token_ids && position && cos && sin && workspace,
+                  "decoder_step: null pointer");
+    TRMOE_REQUIRE(d->hidden % 32 == 0 && aligned16(hidden_rows) && aligned16(workspace),
+                  "decoder_step: hidden rows and workspace must be 16-byte aligned");
+    TRMOE_REQUIRE(workspace_bytes >= s.total, "decoder_step: workspace smaller than trmoe_decoder_step_workspace_bytes()");
+    char* p = static_cast<char*>(workspace);
+    void* mid = p;
+    void* attn = p + s.h;
+    void* feats = p + s.h + s.attn;
+    void* down = p + s.h + s.attn + s.feats;
+    void* attn_ws = p + s.h + s.attn + s.feats + s.down;
+    const int64_t H = d->hidden, qd = (int64_t)d->num_heads * 64;
+    const int64_t F = trmoe_dense_routed_features(d->shared_width, d->num_experts, d->expert_width);
+    for (int64_t i = 0; i < d->layers; ++i) {
+        const trmoe_decoder_layer& l = layers[i];
+        TRMOE_REQUIRE(l.w_o && l.w_gate_up && l.w_gate_up_frag && l.w_down && l.w_down_frag,
+                      "decoder_step: null pointer in a layer");
+        int st = trmoe_decode_attention(hidden_rows, batch, H, H, l.input_norm, d->norm_eps, l.w_kqv, d->num_heads,
+                                        d->num_kv_heads, l.q_norm, l.k_norm, d->qk_eps, cos, sin, positions, position,
+                                        l.k_cache, l.v_cache, d->cache_length, d->attn_scale, attn, attn_ws, s.attn_ws,
+                                        stream);
+        if (st) return st;
+        const float one[4] = {1.f, 0.f, 0.f, 0.f};
+        st = trmoe_shared_down_combine(TRMOE_BF16, TRMOE_BF16, attn, batch, qd, qd, l.w_o, nullptr, H, nullptr, H,
+                                       nullptr, 1, one, 1.0f, 0.0f, hidden_rows, H, mid, H, down, s.down, stream);
+        if (st) return st;
+        trmoe_call_extras ex{};
+        ex.rms_eps = d->norm_eps;
+        ex.w_frag = l.w_gate_up_frag;
+        ex.w_frag_cols = H;
+        st = trmoe_dense_routed_gate_up_ex(TRMOE_BF16, TRMOE_BF16, mid, batch, H, H, l.w_gate_up, nullptr,
+                                           d->shared_width, d->num_experts, d->expert_width, token_ids, l.route_table,
+                                           d->vocab_size, d->top_k, d->route_weights, d->shared_scale, d->routed_scale,
+                                           feats, F, &ex, stream);
+        if (st) return st;
+        ex = trmoe_call_extras{};
+        ex.w_frag = l.w_down_frag;
+        ex.w_frag_cols = F;
+        st = trmoe_shared_down_combine_ex(TRMOE_BF16, TRMOE_BF16, feats, batch, F, F, l.w_down, nullptr, H, nullptr, H,
+                                          nullptr, 1, one, 1.0f, 1.0f, mid, H, hidden_rows, H, down, s.down, &ex,
+                                          stream);
+        if (st) return st;
+    }
+    return TRMOE_OK;
+}
+
 // Extras of the *_ex entry points: validated against the call they ride on.
 static int extras_ok(const char* who, const trmoe_call_extras* ex, int act_dtype, int w_dtype, int64_t k,
                      int64_t n_tokens, bool rms_allowed) {

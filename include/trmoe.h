@@ -503,6 +503,41 @@ int trmoe_shared_down_combine_ex(int act_dtype, int w_dtype, const void* h, int6
                                  int64_t ldo, void* workspace, size_t workspace_bytes,
                                  const trmoe_call_extras* extras, void* stream);
 
+/*
+ * One decode step of a whole decoder (bf16, dense-routed layers, batch <= 16):
+ * for every layer trmoe_decode_attention, the output projection with its
+ * residual, and the MLP half with its RMSNorm and residual, queued by one call
+ * (the host's share of a step is then the launches alone).  hidden_rows
+ * [batch, hidden] holds the embedded tokens on entry and the last layer's
+ * output when the work completes.
+ */
+typedef struct trmoe_decoder_dims {
+    int64_t layers, hidden, cache_length, vocab_size, shared_width, expert_width;
+    int32_t num_heads, num_kv_heads, num_experts, top_k;
+    float norm_eps, qk_eps, attn_scale, shared_scale, routed_scale;
+    float route_weights[4];
+} trmoe_decoder_dims;
+
+typedef struct trmoe_decoder_layer {
+    const void* input_norm;      /* [hidden] */
+    const void* w_kqv;           /* [(num_heads + 2 num_kv_heads) * 64, hidden] */
+    const void* q_norm;          /* [64] */
+    const void* k_norm;
+    const void* w_o;             /* [hidden, num_heads * 64] */
+    void* k_cache;               /* [batch, num_kv_heads, cache_length, 64] */
+    void* v_cache;
+    const void* w_gate_up;       /* the layer's dense-routed packs, its RMSNorm weight folded in, */
+    const void* w_gate_up_frag;  /* and their fragment-major copies */
+    const void* w_down;
+    const void* w_down_frag;
+    const int64_t* route_table;  /* [top_k, vocab_size] */
+} trmoe_decoder_layer;
+
+size_t trmoe_decoder_step_workspace_bytes(const trmoe_decoder_dims* dims, int64_t batch);
+int trmoe_decoder_step(const trmoe_decoder_dims* dims, const trmoe_decoder_layer* layers, void* hidden_rows,
+                       int64_t batch, const int64_t* token_ids, const int64_t* position, const float* cos,
+                       const float* sin, int64_t positions, void* workspace, size_t workspace_bytes, void* stream);
+
 /* ---------------------------------------------------------------------------
  * Backward (bf16 / f32 weights; fp8 weights are inference-only).
  *
