@@ -202,9 +202,11 @@ __device__ __forceinline__ void init_dense_rows(Prov& p, const void* base, int64
 // the tile main loop
 // ---------------------------------------------------------------------------
 // Block tile BM x BN, 4 waves as WAVES_M x WAVES_N, each wave TM x TN MFMA
-// tiles of 32x32.  Two LDS stages; one barrier per K stage.  `lds` holds
-// 2 * (BM + BN) * 128 bytes.
-template <int BM_, int BN_, int WAVES_M_, int WAVES_N_, int PGR_ = 1>
+// tiles of 32x32.  STAGES LDS stages; `lds` holds STAGES * (BM + BN) * 128
+// bytes (e4m3 B rows: 64).
+// KS groups of WAVES_M x WAVES_N waves compute the same tile, each every KS-th
+// K stage on LDS stages of its own; reduce_groups adds their accumulators.
+template <int BM_, int BN_, int WAVES_M_, int WAVES_N_, int PGR_ = 1, int STAGES_ = 2, int KS_ = 1>
 struct TileShape {
     // 1: register-staged loads, one stage ahead (tile_loop_pgr1);
     // 4: direct buffer->LDS loads (tile_loop_dma, bf16/f32 operands only);
@@ -213,18 +215,24 @@ struct TileShape {
     static constexpr int BN = BN_;
     static constexpr int WAVES_M = WAVES_M_;
     static constexpr int WAVES_N = WAVES_N_;
-    static constexpr int NT = 64 * WAVES_M * WAVES_N;   // threads per workgroup
+    static constexpr int KS = KS_;
+    static constexpr int NTG = 64 * WAVES_M * WAVES_N;   // threads of a group
+    static constexpr int NT = NTG * KS;                  // threads per workgroup
     static constexpr int WM = BM / WAVES_M;
     static constexpr int WN = BN / WAVES_N;
     static constexpr int TM = WM / 32;
     static constexpr int TN = WN / 32;
     // 6: direct loads, bf16 A rows of 128 bytes + e4m3 B rows of 64 bytes per
     //    64-element K stage, expanded to bf16 at the fragment read
-    static constexpr int kStages = 2;
+    // More than two stages or groups (direct loads only): tile_loop_ring
+    static constexpr int kStages = STAGES_;
+    static constexpr bool kRing = STAGES_ > 2 || KS_ > 1;
+    static_assert(!kRing || PGR >= 4, "only direct loads run on a ring of stages");
     static constexpr int kStageBytes = PGR == 6 ? BM * kRowBytes + BN * 64 : (BM + BN) * kRowBytes;
-    static constexpr int kLdsBytes = kStages * kStageBytes;
+    static constexpr int kLdsBytes = KS * kStages * kStageBytes;
+    static_assert((KS - 1) * BM * BN * 4 <= kLdsBytes || KS == 1, "the groups' sums pass through the stages' LDS");
     static_assert(WM % 32 == 0 && WN % 32 == 0, "wave tile must be a multiple of 32");
-    static_assert((BM * 8) % NT == 0 && (BN * 8) % NT == 0, "tile rows must split evenly over threads");
+    static_assert((BM * 8) % NTG == 0 && (BN * 8) % NTG == 0, "tile rows must split evenly over threads");
 };
 
 template <class Kind, int TM, int TN>
@@ -366,7 +374,7 @@ struct DmaRows {
         const int64_t nrows = avail < ROWS ? avail : ROWS;
         rsrc = make_rsrc(static_cast<const char*>(base) + row0 * ld_bytes, (uint32_t)(nrows * ld_bytes));
         kbytes = kbytes_;
-        wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+        wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) % kWaves;
         const int lane = threadIdx.x & 63;
 #pragma unroll
         for (int j = 0; j < kInstr; ++j) {
@@ -438,7 +446,7 @@ struct DmaRows64 {
         const int64_t nrows = avail < ROWS ? avail : ROWS;
         rsrc = make_rsrc(static_cast<const char*>(base) + row0 * ld_bytes, (uint32_t)(nrows * ld_bytes));
         kbytes = kbytes_;
-        wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+        wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) % kWaves;
         const int lane = threadIdx.x & 63;
 #pragma unroll
         for (int j = 0; j < kInstr; ++j) {
@@ -484,10 +492,89 @@ __device__ __forceinline__ void tile_loop_dma(const AP& ap, const BP& bp, int K,
     __syncthreads();
 }
 
+// The K loop on a ring of S = Shape::kStages LDS stages per group, S - 1 of
+// them in flight: stage kt + S - 1 is requested as soon as every wave has read
+// stage kt - 1, whose buffer it takes, so a load has S - 2 stages of MFMA work
+// to land and each stage costs one barrier.  For launches with about one
+// workgroup per CU, where a stage of a small tile is a chain of latencies (load,
+// barrier, LDS read, MFMA): groups run KS such chains side by side.  Group g
+// takes stages g, g + KS, ...; requests past the last stage read zeros, and
+// the final barrier drains them before the caller reuses LDS.
+template <class Kind, class Shape, class AP, class BP>
+__device__ __forceinline__ void tile_loop_ring(const AP& ap, const BP& bp, int K, char* lds, int wm0, int wn0,
+                                               f32x16 (&acc)[Shape::TM][Shape::TN]) {
+    constexpr int S = Shape::kStages, KS = Shape::KS;
+    constexpr int kABytes = Shape::BM * kRowBytes;
+    constexpr int kPer = AP::kInstr + BP::kInstr;
+    const int stages = (K + Kind::kStageElems - 1) / Kind::kStageElems;
+    const int nk = (stages + KS - 1) / KS;
+    const int g = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / Shape::NTG);
+    lds += g * S * Shape::kStageBytes;
+#pragma unroll
+    for (int s = 0; s < S - 1; ++s) {
+        ap.issue(s * KS + g, lds + s * Shape::kStageBytes);
+        bp.issue(s * KS + g, lds + s * Shape::kStageBytes + kABytes);
+    }
+    int cur = 0, nxt = S - 1;
+    for (int kt = 0; kt < nk; ++kt) {
+        wait_vmcnt<kPer * (S - 2)>();   // this wave's loads of stage kt have landed
+        wait_lgkmcnt0();                // and its reads of stage kt - 1 are complete
+        lds_barrier();                  // ... and every other wave's
+        char* st = lds + cur * Shape::kStageBytes;
+        char* to = lds + nxt * Shape::kStageBytes;
+        ap.issue((kt + S - 1) * KS + g, to);
+        bp.issue((kt + S - 1) * KS + g, to + kABytes);
+        if constexpr (Shape::PGR == 6)
+            mma_stage_f8<Shape::TM, Shape::TN>(st, st + kABytes, wm0, wn0, acc);
+        else
+            mma_stage<Kind, Shape::TM, Shape::TN>(st, st + kABytes, wm0, wn0, acc);
+        cur = cur + 1 == S ? 0 : cur + 1;
+        nxt = nxt + 1 == S ? 0 : nxt + 1;
+    }
+    __syncthreads();
+}
+
+// Adds the other groups' accumulators to group 0's, in group order, through
+// LDS (free after the loop's last barrier, and again on return).  True for the
+// waves of group 0, which hold the tile.
+template <class Shape>
+__device__ __forceinline__ bool reduce_groups(char* lds, f32x16 (&acc)[Shape::TM][Shape::TN]) {
+    if constexpr (Shape::KS == 1) return true;
+    const int g = __builtin_amdgcn_readfirstlane((int)threadIdx.x / Shape::NTG);
+    const int t = (int)threadIdx.x % Shape::NTG;
+    constexpr int kVals = Shape::TM * Shape::TN * 16;
+    float* red = reinterpret_cast<float*>(lds);
+    if (g > 0) {
+#pragma unroll
+        for (int tm = 0; tm < Shape::TM; ++tm)
+#pragma unroll
+            for (int tn = 0; tn < Shape::TN; ++tn)
+#pragma unroll
+                for (int i = 0; i < 16; ++i)
+                    red[((g - 1) * kVals + (tm * Shape::TN + tn) * 16 + i) * Shape::NTG + t] = acc[tm][tn][i];
+    }
+    __syncthreads();
+    if (g == 0) {
+#pragma unroll
+        for (int o = 0; o < Shape::KS - 1; ++o)
+#pragma unroll
+            for (int tm = 0; tm < Shape::TM; ++tm)
+#pragma unroll
+                for (int tn = 0; tn < Shape::TN; ++tn)
+#pragma unroll
+                    for (int i = 0; i < 16; ++i)
+                        acc[tm][tn][i] += red[(o * kVals + (tm * Shape::TN + tn) * 16 + i) * Shape::NTG + t];
+    }
+    __syncthreads();
+    return g == 0;
+}
+
 template <class Kind, class Shape, class AProv, class BProv>
 __device__ __forceinline__ void tile_loop(const AProv& ap, const BProv& bp, int K, char* lds, int wm0, int wn0,
                                           f32x16 (&acc)[Shape::TM][Shape::TN]) {
-    if constexpr (Shape::PGR == 4 || Shape::PGR == 6)
+    if constexpr (Shape::kRing)
+        tile_loop_ring<Kind, Shape>(ap, bp, K, lds, wm0, wn0, acc);
+    else if constexpr (Shape::PGR == 4 || Shape::PGR == 6)
         tile_loop_dma<Kind, Shape>(ap, bp, K, lds, wm0, wn0, acc);
     else
         tile_loop_pgr1<Kind, Shape>(ap, bp, K, lds, wm0, wn0, acc);

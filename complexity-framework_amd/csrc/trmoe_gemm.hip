@@ -145,8 +145,8 @@ template <class Kind, class Shape, bool ROUTED = true>
 __device__ __forceinline__ void gate_up_epilogue(const GateUpArgs& a, f32x16 (&acc)[Shape::TM][Shape::TN],
                                                  int64_t m0, int64_t n0, char* lds,
                                                  const int (*s_route)[kMaxTopK],
-                                                 const float* s_rscale = nullptr) {
-    gate_up_epi_tile<Kind, Shape, ROUTED>(a, acc, n0, lds, s_route, s_rscale);
+                                                 const float* s_rscale = nullptr, bool holder = true) {
+    if (holder) gate_up_epi_tile<Kind, Shape, ROUTED>(a, acc, n0, lds, s_route, s_rscale);
     wait_lgkmcnt0();   // LDS tile complete; outstanding global loads (a next tile's operands) keep flying
     lds_barrier();
     gate_up_epi_store<Kind, Shape>(a, m0, n0, lds);
@@ -197,7 +197,7 @@ template <class Kind, bool FP8, class Shape, bool GROUPED = false, bool ROUTED =
 __global__ __launch_bounds__(Shape::NT) void k_gate_up_swiglu(GateUpArgs a) {
     using T = typename Kind::T;
     extern __shared__ __align__(16) char lds[];
-    const int wave = threadIdx.x >> 6;
+    const int wave = (threadIdx.x >> 6) % (Shape::NTG / 64);
     const int wm0 = (wave / Shape::WAVES_N) * Shape::WM;
     const int wn0 = (wave % Shape::WAVES_N) * Shape::WN;
     int64_t m0 = (int64_t)blockIdx.x * Shape::BM;
@@ -243,9 +243,12 @@ __global__ __launch_bounds__(Shape::NT) void k_gate_up_swiglu(GateUpArgs a) {
     f32x16 acc[Shape::TM][Shape::TN];
     zero_acc<Kind>(acc);
     tile_loop<Kind, Shape>(ap, bp, a.K, lds, wm0, wn0, acc);
-    if constexpr (SAVE) gate_up_save<Kind, Shape>(a, acc, m0, n0, a.n_base + (int64_t)gridDim.y * Shape::BN);
-    gate_up_epilogue<Kind, Shape, ROUTED>(a, acc, m0, n0, lds, s_route,
-                                          a.row_scale != nullptr ? s_rscale : nullptr);
+    const bool holder = reduce_groups<Shape>(lds, acc);
+    if constexpr (SAVE) {
+        if (holder) gate_up_save<Kind, Shape>(a, acc, m0, n0, a.n_base + (int64_t)gridDim.y * Shape::BN);
+    }
+    gate_up_epilogue<Kind, Shape, ROUTED>(a, acc, m0, n0, lds, s_route, a.row_scale != nullptr ? s_rscale : nullptr,
+                                          holder);
 }
 
 // SwiGLU of one finished tile straight from the accumulators of the calling
@@ -598,7 +601,7 @@ template <class Kind, bool FP8, class Shape, bool GROUPED = false>
 __global__ __launch_bounds__(Shape::NT) void k_down_combine(DownArgs a) {
     using T = typename Kind::T;
     extern __shared__ __align__(16) char lds[];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int wave = (threadIdx.x >> 6) % (Shape::NTG / 64), lane = threadIdx.x & 63;
     const int wm0 = (wave / Shape::WAVES_N) * Shape::WM;
     const int wn0 = (wave % Shape::WAVES_N) * Shape::WN;
     int64_t m0 = (int64_t)blockIdx.x * Shape::BM;
@@ -634,6 +637,7 @@ __global__ __launch_bounds__(Shape::NT) void k_down_combine(DownArgs a) {
     f32x16 acc[Shape::TM][Shape::TN];
     zero_acc<Kind>(acc);
     tile_loop<Kind, Shape>(ap, bp, a.K, lds, wm0, wn0, acc);
+    const bool holder = reduce_groups<Shape>(lds, acc);
 
     const int r = lane & 31;
     float cscale[Shape::TN];
@@ -650,16 +654,18 @@ __global__ __launch_bounds__(Shape::NT) void k_down_combine(DownArgs a) {
         // padded by 16 bytes); the routed gather, residual and store then run
         // over 16-byte chunks of 8 columns.
         constexpr int kORowBytes = Shape::BN * 2 + 16;
+        if (holder) {
 #pragma unroll
-        for (int tm = 0; tm < Shape::TM; ++tm)
+            for (int tm = 0; tm < Shape::TM; ++tm)
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const int rl = wm0 + tm * 32 + acc_row(lane, i);
+                for (int i = 0; i < 16; ++i) {
+                    const int rl = wm0 + tm * 32 + acc_row(lane, i);
 #pragma unroll
-                for (int tn = 0; tn < Shape::TN; ++tn)
-                    *reinterpret_cast<T*>(lds + rl * kORowBytes + (wn0 + tn * 32 + r) * 2) =
-                        from_f32<T>(acc[tm][tn][i] * cscale[tn]);
-            }
+                    for (int tn = 0; tn < Shape::TN; ++tn)
+                        *reinterpret_cast<T*>(lds + rl * kORowBytes + (wn0 + tn * 32 + r) * 2) =
+                            from_f32<T>(acc[tm][tn][i] * cscale[tn]);
+                }
+        }
         __syncthreads();
         constexpr int kChunksPerRow = Shape::BN / 8;
         for (int q = threadIdx.x; q < Shape::BM * kChunksPerRow; q += Shape::NT) {
@@ -709,6 +715,7 @@ __global__ __launch_bounds__(Shape::NT) void k_down_combine(DownArgs a) {
         }
     } else {
         // f32: the tile would not fit in LDS; combine straight from registers
+        if (!holder) return;
 #pragma unroll
         for (int tm = 0; tm < Shape::TM; ++tm) {
 #pragma unroll
@@ -1301,6 +1308,59 @@ static int launch_gate_up_dma_balanced(const GateUpArgs& a, int64_t packed_rows,
     return launch_gate_up_shape<Kind, false, ShapeTallDma>(t, packed_rows, stream);
 }
 
+static int64_t tiles_of(int64_t m, int64_t bm, int64_t n, int64_t bn) { return ((m + bm - 1) / bm) * ((n + bn - 1) / bn); }
+
+template <class Kind, bool FP8, class Shape, bool ROUTED, bool SAVE>
+static int launch_gate_up_ring_shape(const GateUpArgs& a, int64_t rows, hipStream_t stream) {
+    const dim3 grid((unsigned)((a.M + Shape::BM - 1) / Shape::BM), (unsigned)(rows / Shape::BN));
+    constexpr int kEpi = Shape::BM * (Shape::BN / 2 * (int)sizeof(typename Kind::T) + 16);
+    constexpr int kLds = kEpi > Shape::kLdsBytes ? kEpi : Shape::kLdsBytes;
+    auto kern = k_gate_up_swiglu<Kind, FP8, Shape, false, ROUTED, SAVE>;
+    const int st = ensure_lds(kern, kLds);
+    if (st) return st;
+    hipLaunchKernelGGL(kern, grid, dim3(Shape::NT), kLds, stream, a);
+    return check_launch(ROUTED ? "dense_routed_gate_up" : "shared_gate_up");
+}
+
+// Launches of at most one round of workgroups (shared and expert columns
+// together): the smallest tile whose grid still fits the CUs once, because a
+// workgroup's time is its K stages and does not shrink with fewer of them.
+// Gate|up of the 200M layer (hidden 896, 6656 packed rows), us before -> now:
+// 130 tokens 9.7 -> 9.2, 512 17.2 -> 12.4, 777 21.0 -> 19.1 (its expert columns
+// were a second launch, 11.8 more), 1024 21.4 -> 19.9; with e4m3 weights at
+// hidden 2048, 11264 rows: 130 tokens 25.6 -> 20.6, 512 39.2 -> 31.4.  At the
+// next size up the 256-row ping-pong tiles are as fast (777 tokens of that
+// layer: 46.9 against 60.4 on 128x256).  f32 takes 64x128 throughout: its
+// MFMAs bound the stage (2048 tokens 252 -> 216 with the merged launch).
+// Returns whether it took the launch.
+template <class Kind, bool FP8, bool SAVE>
+static bool launch_gate_up_ring(const GateUpArgs& a, int64_t packed_rows, hipStream_t stream, int& st) {
+    const int64_t rows = packed_rows - a.n_base, cus = device_cus();
+    if (rows <= 0 || rows % 128 != 0 || (FP8 && (a.ids != nullptr || a.K % 64 != 0 || a.ldw % 16 != 0))) return false;
+    auto run = [&](auto shape) {
+        using Shape = decltype(shape);
+        if constexpr (!FP8) {
+            if (a.ids != nullptr) return launch_gate_up_ring_shape<Kind, FP8, Shape, true, SAVE>(a, rows, stream);
+        }
+        return launch_gate_up_ring_shape<Kind, FP8, Shape, false, SAVE>(a, rows, stream);
+    };
+    if constexpr (std::is_same_v<Kind, KindF32>) {
+        if (tiles_of(a.M, 256, rows, 256) >= kBigTileMinBlocks) return false;
+        st = run(RingGateUp64<false>{});
+        return true;
+    } else {
+        if (tiles_of(a.M, 64, rows, 128) <= cus)
+            st = run(RingGateUp64<FP8>{});
+        else if (tiles_of(a.M, 128, rows, 128) <= cus)
+            st = run(RingGateUp128<FP8>{});
+        else if (rows % 256 == 0 && tiles_of(a.M, 128, rows, 256) <= cus)
+            st = run(Ring128x256<FP8>{});
+        else
+            return false;
+        return true;
+    }
+}
+
 template <class Kind, bool FP8>
 static int launch_gate_up_kind(const GateUpArgs& a, int64_t packed_rows, hipStream_t stream) {
     const int64_t big_blocks = ((a.M + 255) / 256) * (packed_rows / 256);
@@ -1534,6 +1594,9 @@ static int launch_gate_up_pp(const GateUpArgs& a, int64_t packed_rows, hipStream
 
 int launch_gate_up(int act, int wdt, const GateUpArgs& a, int64_t packed_rows, hipStream_t stream) {
     if (a.gu != nullptr) {
+        int st = TRMOE_OK;
+        if (act == TRMOE_BF16 && wdt == TRMOE_BF16 && launch_gate_up_ring<KindBF16, false, true>(a, packed_rows, stream, st))
+            return st;
         if (pp_eligible(act, wdt, a, packed_rows))
             return a.ids != nullptr ? launch_gate_up_pp<true, true>(a, packed_rows, stream)
                                     : launch_gate_up_pp<false, true>(a, packed_rows, stream);
@@ -1543,6 +1606,16 @@ int launch_gate_up(int act, int wdt, const GateUpArgs& a, int64_t packed_rows, h
         return launch_gate_up_skinny(act, wdt, a, packed_rows, stream);
     if (a.row_scale == nullptr && a.rms_eps > 0.0f)
         return set_error(TRMOE_ERR_INVALID, "gate_up: in-kernel RMSNorm scales need the decode kernels (n <= 128)");
+    {
+        int st = TRMOE_OK;
+        const bool taken =
+            act == TRMOE_F32 && wdt == TRMOE_F32     ? launch_gate_up_ring<KindF32, false, false>(a, packed_rows, stream, st)
+            : act == TRMOE_BF16 && wdt == TRMOE_BF16 ? launch_gate_up_ring<KindBF16, false, false>(a, packed_rows, stream, st)
+            : act == TRMOE_BF16 && wdt == TRMOE_FP8_E4M3
+                ? launch_gate_up_ring<KindBF16, true, false>(a, packed_rows, stream, st)
+                : false;
+        if (taken) return st;
+    }
     if (pp_eligible(act, wdt, a, packed_rows)) {
         if (wdt == TRMOE_FP8_E4M3)
             return a.ids != nullptr ? launch_gate_up_pp<true, false, true>(a, packed_rows, stream)
@@ -1586,8 +1659,7 @@ static int launch_down_shape(const DownArgs& a, hipStream_t stream) {
     return check_launch("shared_down_combine");
 }
 
-// bf16 down GEMMs with at least a full round of 256x256 tiles run on the
-// ping-pong main loop.
+// 256x256 down tiles on the ping-pong main loop.
 template <bool FP8, bool A8 = false>
 static int launch_down_pp(const DownArgs& a, hipStream_t stream) {
     const dim3 grid((unsigned)(((a.M + 255) / 256) * ((a.N + 255) / 256)));
@@ -1608,11 +1680,32 @@ int launch_down_combine_a8(const DownArgs& a, hipStream_t stream) {
 
 // The packed down weights have round_up(N, 256) rows, so every tile choice
 // below reads only packed rows.
+//
+// bf16 and e4m3 weights: the smallest tile whose grid fits the CUs once, as
+// for the gate|up, then the 256x256 ping-pong tiles.  us before -> now, bf16
+// K = 3328, N = 896: 512 tokens 19.0 -> 13.6, 777 19.7 -> 17.8, 2048 21.9 ->
+// 20.7, 3001 43.8 -> 28.6, 4096 42.5 -> 31.4, 8192 59.7 -> 52.7 (256x128: N is
+// half a 256-column tile over), 10000 118 -> 62.6; bf16 K = 5632, N = 2048:
+// 3001 tokens 95 -> 83, 4096 104 -> 92, 5000 146 -> 103; e4m3 there: 130 tokens
+// 48.5 -> 19.1, 512 51.6 -> 20.5, 1024 51.9 -> 32.7, 4096 95.8 -> 72.4.
+// f32 up to one round: 512 tokens 76 -> 61 (K = 3328, N = 896).
 template <class Kind, bool FP8>
 static int launch_down_kind(const DownArgs& a, hipStream_t stream) {
-    const int64_t mt = (a.M + 255) / 256;
+    const int64_t mt = (a.M + 255) / 256, cus = device_cus();
     if constexpr (std::is_same_v<Kind, KindBF16>) {
-        if (a.K > 0 && a.K % 64 == 0 && mt * ((a.N + 255) / 256) >= 256) return launch_down_pp<FP8>(a, stream);
+        if (a.K > 0 && a.K % 64 == 0 && (!FP8 || a.ldw % 16 == 0)) {
+            if (tiles_of(a.M, 64, a.N, 64) <= cus) return launch_down_shape<Kind, FP8, RingDown64<FP8>>(a, stream);
+            if (tiles_of(a.M, 128, a.N, 64) <= cus) return launch_down_shape<Kind, FP8, RingDown128x64<FP8>>(a, stream);
+            if (tiles_of(a.M, 128, a.N, 128) <= cus) return launch_down_shape<Kind, FP8, RingDown128<FP8>>(a, stream);
+            if constexpr (!FP8) {
+                if (a.N % 256 != 0 && tiles_of(a.M, 256, a.N, 128) <= cus)
+                    return launch_down_shape<Kind, FP8, RingDown256x128>(a, stream);
+            }
+            if (tiles_of(a.M, 128, a.N, 256) <= cus) return launch_down_shape<Kind, FP8, Ring128x256<FP8>>(a, stream);
+            return launch_down_pp<FP8>(a, stream);
+        }
+    } else {
+        if (tiles_of(a.M, 64, a.N, 64) <= cus) return launch_down_shape<Kind, FP8, RingDown64F32>(a, stream);
     }
     const bool fits224 = a.N % ShapeDown224::BN == 0;
     if constexpr (FP8) {

@@ -34,7 +34,7 @@ __device__ __forceinline__ void init_bprov(typename BProvSel<Kind, FP8, ROWS, NT
 // register-staged loads otherwise (and always for e4m3 weights, which are
 // expanded to bf16 on the way into LDS).
 template <class Shape, int ROWS>
-using DmaProv = DmaRows<ROWS, Shape::NT>;
+using DmaProv = DmaRows<ROWS, Shape::NTG>;
 template <class Shape>
 struct AProvOf {
     using type = std::conditional_t<(Shape::PGR >= 4), DmaProv<Shape, Shape::BM>, BufRows<Shape::BM, Shape::NT>>;
@@ -45,7 +45,7 @@ struct BProvOf {
     static_assert(!(!FP8 && Shape::PGR == 6), "PGR 6 is the e4m3 weight layout");
     // PGR 6: e4m3 rows of 64 bytes per K stage, the 64-byte-row DMA layout
     using type = std::conditional_t<
-        Shape::PGR == 6, DmaRows64<Shape::BN, Shape::NT>,
+        Shape::PGR == 6, DmaRows64<Shape::BN, Shape::NTG>,
         std::conditional_t<(Shape::PGR >= 4), DmaProv<Shape, Shape::BN>,
                            typename BProvSel<Kind, FP8, Shape::BN, Shape::NT>::type>>;
 };
@@ -82,6 +82,20 @@ using ShapeTallDma = TileShape<128, 256, 1, 4, 4>;          // 128x256: 4 waves 
 // direct loads, or the register path that expands e4m3 weights.
 template <bool FP8, int BN>
 using SmallShape = std::conditional_t<FP8, TileShape<64, BN, 2, 2>, TileShape<64, BN, 2, 2, 4>>;
+
+// Tiles of launches with at most one round of workgroups, on rings of LDS
+// stages (PGR 4 or, with e4m3 weights, 6).  The 64-row tiles run one stage's
+// chain of latencies per 128 or 64 columns, so the down's narrow ones split K
+// over two groups of waves (four in f32, whose MFMAs are 16 times as long).
+template <bool FP8> constexpr int kRingPgr = FP8 ? 6 : 4;
+template <bool FP8> using RingGateUp64 = TileShape<64, 128, 2, 2, kRingPgr<FP8>, 3>;
+template <bool FP8> using RingGateUp128 = TileShape<128, 128, 4, 2, kRingPgr<FP8>, 4>;
+template <bool FP8> using RingDown64 = TileShape<64, 64, 2, 2, kRingPgr<FP8>, 3, 2>;
+template <bool FP8> using RingDown128x64 = TileShape<128, 64, 2, 2, kRingPgr<FP8>, 3, 2>;
+template <bool FP8> using RingDown128 = TileShape<128, 128, 2, 4, kRingPgr<FP8>, 4>;
+template <bool FP8> using Ring128x256 = TileShape<128, 256, 2, 4, kRingPgr<FP8>, 3>;
+using RingDown256x128 = TileShape<256, 128, 4, 2, 4, 3>;
+using RingDown64F32 = TileShape<64, 64, 2, 2, 4, 2, 4>;
 
 // ---------------------------------------------------------------------------
 // expert-grouped tiles
@@ -120,7 +134,7 @@ __device__ __forceinline__ void init_gather_rows(Prov& p, const void* base, cons
     p.rsrc = make_rsrc(base, (uint32_t)(mod * ld_bytes));
     p.kbytes = kbytes;
     if constexpr (requires_wave_field<Prov>::value) {
-        p.wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+        p.wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) % Prov::kWaves;
         const int lane = threadIdx.x & 63;
         constexpr int kRowsPerInstr = Prov::kRowsPerInstr;
 #pragma unroll
