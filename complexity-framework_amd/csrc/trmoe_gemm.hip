@@ -528,12 +528,15 @@ __device__ __forceinline__ void gate_up_save_direct(const GateUpArgs& a, const f
 // stages load and multiply.  SAVE: also the raw gate|up outputs (a.gu).
 // A8 (with FP8): e4m3 activations too, a.x holding the codes (row stride
 // a.ldx bytes) and a.row_scale their per-token scales: 128 K values per
-// stage on the e4m3 MFMA (W8A8).  MXH (with A8): transposed accumulator
+// stage on the e4m3 MFMA (W8A8).  RS: a.row_scale holds the fused RMSNorm's
+// per-token scales (16384 tokens of the 200M layer: 192 us in one-tile
+// workgroups with the scales in LDS).  MXH (with A8): transposed accumulator
 // blocks, and h leaves as block-scaled e4m3 (gate_up_epi_mx).
-template <int TMW, bool SAVE, bool FP8, bool A8 = false, bool MXH = false>
+template <int TMW, bool SAVE, bool FP8, bool A8 = false, bool MXH = false, bool RS = false>
 __global__ __launch_bounds__(512, 1) void k_gate_up_pps(GateUpArgs a, int64_t tiles_m, int64_t n_tiles) {
     static_assert(!A8 || (FP8 && !SAVE), "W8A8 is the inference form of the e4m3 weights");
     static_assert(!MXH || A8, "block-scaled h is written by the W8A8 kernel");
+    static_assert(!RS || (!FP8 && !SAVE), "the fused RMSNorm is the bf16 inference form");
     constexpr int BM = 64 * TMW;
     extern __shared__ __align__(16) char lds[];
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -590,7 +593,7 @@ __global__ __launch_bounds__(512, 1) void k_gate_up_pps(GateUpArgs a, int64_t ti
             else if constexpr (A8)
                 gate_up_epi_direct<TMW, true, true>(a, c, tm0, tn0, wm0, wn0);
             else
-                gate_up_epi_direct<TMW, !FP8>(a, c, tm0, tn0, wm0, wn0);
+                gate_up_epi_direct<TMW, !FP8, RS>(a, c, tm0, tn0, wm0, wn0);
         });
 }
 
@@ -1531,7 +1534,7 @@ static int launch_gate_up_pp_shape(const GateUpArgs& a, int64_t packed_rows, hip
 
 // Persistent 256-row tiles over packed rows [a.n_base, packed_rows): one
 // workgroup per CU (fewer when there are fewer tiles).
-template <bool SAVE, bool FP8>
+template <bool SAVE, bool FP8, bool RS = false>
 static int launch_gate_up_pps(const GateUpArgs& a, int64_t packed_rows, hipStream_t stream) {
     const int64_t tiles_m = (a.M + 255) / 256;
     const int64_t n_tiles = tiles_m * ((packed_rows - a.n_base) / 256);
@@ -1539,7 +1542,7 @@ static int launch_gate_up_pps(const GateUpArgs& a, int64_t packed_rows, hipStrea
     const int64_t grid = n_tiles < cus ? n_tiles : cus;
     using Lay = std::conditional_t<FP8, PPLayoutF8<4>, PPLayoutK<4>>;
     constexpr int kLds = 2 * Lay::kStage;
-    auto kern = k_gate_up_pps<4, SAVE, FP8>;
+    auto kern = k_gate_up_pps<4, SAVE, FP8, false, false, RS>;
     const int st = ensure_lds(kern, kLds);
     if (st) return st;
     if (grid <= 0) return TRMOE_OK;
@@ -1564,32 +1567,47 @@ int launch_gate_up_a8(const GateUpArgs& a, int64_t packed_rows, hipStream_t stre
     return check_launch("shared_gate_up_a8");
 }
 
-// 256-row tiles; when their last round would leave at least half of the CUs
-// idle, the fewest trailing columns whose removal leaves whole rounds run as
-// a second launch of 128-row tiles (C2: 64 x 24 tiles, then 128 x 2 half
-// tiles: seven rounds become six and a round of half tiles).  Launches whose
+// 256x256 tiles in whole rounds, and the trailing columns that would open a
+// round of their own as a second launch of ring tiles, when that is estimated
+// shorter: a launch of at most one round of ring tiles takes about 0.65 of a
+// ping-pong round on 128x256 tiles (19 us against 29 at K = 896, 34 against 57
+// at K = 2048), 0.4 on 64x128.  C2's 64 x 26 tiles: six rounds and 256 ring
+// tiles (26 -> 19 us for the tail); 12 x 44 tiles (3001 tokens of the scaled
+// layer): two rounds and 188 ring tiles instead of three.  Launches whose
 // first columns hold no expert features leave the routing code out.
 template <bool ROUTED, bool SAVE, bool FP8 = false>
 static int launch_gate_up_pp(const GateUpArgs& a, int64_t packed_rows, hipStream_t stream) {
     const int64_t tiles_m = (a.M + 255) / 256;
     const int64_t cols = (packed_rows - a.n_base) / 256;
     const int64_t cus = device_cus();
+    const bool ring = !FP8 || (a.ids == nullptr && a.K % 64 == 0 && a.ldw % 16 == 0);
+    auto rounds = [&](int64_t n) { return (n + cus - 1) / cus; };
     int64_t tail = 0;
-    if ((tiles_m * cols) % cus != 0)
-        for (int64_t k = 1; k < cols; ++k)
-            if ((tiles_m * (cols - k)) % cus == 0 && tiles_m * k * 2 <= cus) {
-                tail = k;
-                break;
-            }
+    double best = (double)rounds(tiles_m * cols);
+    for (int64_t k = 1; ring && k < cols && tiles_of(a.M, 128, k * 256, 256) <= cus; ++k) {
+        const double cost = (double)rounds(tiles_m * (cols - k)) + (tiles_of(a.M, 64, k * 256, 128) <= cus ? 0.4 : 0.65);
+        if (cost < best) {
+            best = cost;
+            tail = k;
+        }
+    }
     const int64_t split = a.n_base + (cols - tail) * 256;
     const bool head_routed = ROUTED && a.ids != nullptr && split > 2 * a.shared_feats;
-    int st = head_routed            ? launch_gate_up_pp_shape<ROUTED, 4, SAVE, FP8>(a, split, stream)
-             : a.row_scale != nullptr ? launch_gate_up_pp_shape<false, 4, SAVE, FP8>(a, split, stream)
-                                      : launch_gate_up_pps<SAVE, FP8>(a, split, stream);
+    int st;
+    if (head_routed)
+        st = launch_gate_up_pp_shape<ROUTED, 4, SAVE, FP8>(a, split, stream);
+    else if (a.row_scale == nullptr)
+        st = launch_gate_up_pps<SAVE, FP8>(a, split, stream);
+    else if constexpr (!FP8 && !SAVE)
+        st = launch_gate_up_pps<false, false, true>(a, split, stream);
+    else
+        st = launch_gate_up_pp_shape<false, 4, SAVE, FP8>(a, split, stream);
     if (st || tail == 0) return st;
     GateUpArgs t = a;
     t.n_base = split;
-    return launch_gate_up_pp_shape<ROUTED, 2, SAVE, FP8>(t, packed_rows, stream);
+    if (!launch_gate_up_ring<KindBF16, FP8, SAVE && !FP8>(t, packed_rows, stream, st))
+        return set_error(TRMOE_ERR_INVALID, "gate_up: the tail columns fit no tile");
+    return st;
 }
 
 int launch_gate_up(int act, int wdt, const GateUpArgs& a, int64_t packed_rows, hipStream_t stream) {
