@@ -60,8 +60,8 @@ class DecoderLayer(ctypes.Structure):
     """trmoe_decoder_layer (include/trmoe.h)."""
 
     _fields_ = [(n, ctypes.c_void_p) for n in (
-        "input_norm", "w_kqv", "q_norm", "k_norm", "w_o", "k_cache", "v_cache", "w_gate_up", "w_gate_up_frag",
-        "w_down", "w_down_frag", "route_table")]
+        "input_norm", "w_kqv", "q_norm", "k_norm", "w_o", "k_cache", "v_cache", "w_gate_up_frag",
+        "w_down_frag", "route_table")]
 
 
 _c_dims = ctypes.POINTER(DecoderDims)
@@ -161,6 +161,12 @@ SIGNATURES = {
         _c_int,
         [_c_vp, _c_i64, _c_i64, _c_i64, _c_vp, _c_float, _c_vp, _c_int, _c_int, _c_vp, _c_vp, _c_float, _c_vp, _c_vp,
          _c_i64, _c_vp, _c_vp, _c_vp, _c_i64, _c_float, _c_vp, _c_vp, _c_size, _c_vp],
+    ),
+    "trmoe_dense_decode_workspace_bytes": (_c_size, [_c_int, _c_i64, _c_i64, _c_i64, _c_int, _c_i64]),
+    "trmoe_dense_decode": (
+        _c_int,
+        [_c_int, _c_vp, _c_i64, _c_i64, _c_i64, _c_vp, _c_vp, _c_i64, _c_int, _c_i64, _c_vp, _c_vp, _c_i64, _c_int,
+         _c_vp, _c_float, _c_float, _c_vp, _c_float, _c_vp, _c_i64, _c_vp, _c_i64, _c_vp, _c_size, _c_vp],
     ),
     "trmoe_decoder_step_workspace_bytes": (_c_size, [_c_dims, _c_i64]),
     "trmoe_decoder_step": (

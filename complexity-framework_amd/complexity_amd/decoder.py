@@ -293,7 +293,7 @@ class _StepPlan:
             ptrs = (plan._weight(norm_in, "weight"), kqv, plan._weight(plan._watch(attn, "q_norm"), "weight"),
                     plan._weight(plan._watch(attn, "k_norm"), "weight"),
                     plan._weight(plan._watch(attn, "o_proj"), "weight"), dec.k_cache[i], dec.v_cache[i],
-                    packed.dense_gate_up, gu, packed.dense_down, dn, table)
+                    gu, dn, table)
             if any(t.data_ptr() % 16 for t in ptrs) or kqv.dtype is not torch.bfloat16:
                 return None
             plan.keep.append(ptrs)

@@ -843,6 +843,40 @@ def shared_down_combine(h: torch.Tensor, shared_width: int, w_down: torch.Tensor
     return out
 
 
+def dense_decode(x: torch.Tensor, token_ids: torch.Tensor, route_table: torch.Tensor, packed: "PackedLayer",
+                 route_weights: Sequence[float], shared_scale: float, routed_scale: float,
+                 residual: Optional[torch.Tensor] = None, row_scale: Optional[torch.Tensor] = None,
+                 rms_eps: float = 0.0) -> torch.Tensor:
+    """A dense-routed layer on at most SKINNY_MAX_TOKENS tokens (trmoe_dense_decode)."""
+    lib = _lib()
+    _require_cuda(x, token_ids, route_table, residual)
+    n, hidden = x.shape
+    F = packed.dense_features
+    gu, dn = packed.fragments("dense_gate_up", hidden)[0], packed.fragments("dense_down", F)[0]
+    ids = token_ids.reshape(-1)
+    ids = (ids if ids.dtype == torch.int64 else ids.to(torch.int64)).contiguous()
+    table = route_table.contiguous()
+    top_k, vocab = table.shape
+    if x.dtype != packed.act_dtype or ids.numel() != n or table.dtype != torch.int64:
+        raise ValueError("dense_decode: the layer's activation dtype, one token id per row and an int64 route table")
+    code = dtype_code(x.dtype)
+    out = torch.empty(n, hidden, dtype=x.dtype, device=x.device)
+    ws_bytes = lib.trmoe_dense_decode_workspace_bytes(code, n, hidden, packed.shared_width, packed.num_experts,
+                                                      packed.expert_width)
+    # not the shared scratch: it holds the layer's features, and every graph
+    # that records the call needs its own
+    ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=x.device)
+    rw = _weights_arg(route_weights)
+    st = lib.trmoe_dense_decode(code, _p(x), n, hidden, x.stride(0), _p(gu), _p(dn), packed.shared_width,
+                                packed.num_experts, packed.expert_width, _p(ids), _p(table), vocab, top_k,
+                                ctypes.cast(rw, ctypes.c_void_p), float(shared_scale), float(routed_scale),
+                                _p(row_scale), float(rms_eps), _p(residual),
+                                residual.stride(0) if residual is not None else 0, _p(out), hidden, _p(ws), ws_bytes,
+                                _stream(x))
+    N.check(st, "trmoe_dense_decode")
+    return out
+
+
 def stream_read(src: torch.Tensor, sink: torch.Tensor) -> None:
     """One launch that reads src's bytes once (trmoe_stream_read): the
     single-launch streaming floor the decode kernels are compared with.
@@ -996,15 +1030,18 @@ def layer_forward(x: torch.Tensor, token_ids: torch.Tensor, route_table: torch.T
     # decode sizes read the weights through their fragment-major copies
     decode = n <= SKINNY_MAX_TOKENS and not save
     if packed.strategy == STRATEGY_DENSE:
+        if decode:
+            frags = packed.fragments("dense_gate_up", hidden), packed.fragments("dense_down", packed.dense_features)
+            if None not in frags:
+                return dense_decode(x, token_ids, route_table, packed, route_weights, shared_scale, routed_scale,
+                                    residual, rscale, eps_in)
         h = dense_routed_gate_up(x, packed.dense_gate_up, packed.shared_width, packed.num_experts,
                                  packed.expert_width, token_ids, route_table, route_weights, shared_scale,
-                                 routed_scale, save=save, row_scale=rscale, rms_eps=eps_in,
-                                 w_frag=packed.fragments("dense_gate_up", hidden) if decode else None)
+                                 routed_scale, save=save, row_scale=rscale, rms_eps=eps_in)
         if save:
             h, gu = h
         out = shared_down_combine(h, packed.dense_features, packed.dense_down, None, hidden, None, None,
-                                  top_k, route_weights, 1.0, 1.0, residual,
-                                  w_frag=packed.fragments("dense_down", packed.dense_features) if decode else None)
+                                  top_k, route_weights, 1.0, 1.0, residual)
         return (out, gu, h) if save else out
     if decode and rscale is None and x.dtype == torch.bfloat16 and packed.expert_gate_up.dtype == torch.float8_e4m3fn:
         return e4m3_decode_layer(x, token_ids, route_table, packed, route_weights, shared_scale, routed_scale, residual)

@@ -1055,11 +1055,102 @@ int trmoe_decode_attention(const void* hidden_rows, int64_t batch, int64_t hidde
     return launch_decode_attn(a, num_heads / num_kv_heads, as_stream(stream));
 }
 
-// Scratch of trmoe_decoder_step: two hidden buffers, the attention output, the
-// SwiGLU features, then the split partials of the down kernels and the
-// attention's own scratch (used at different times, kept apart).
+// Scratch of trmoe_dense_decode: the SwiGLU features, the down's split
+// partials, its counters.
+struct DenseDecodeScratch {
+    size_t feats, part, counters, total;
+};
+
+static DenseDecodeScratch dense_decode_scratch(int act_dtype, int64_t n, int64_t hidden, int64_t feats) {
+    auto up = [](size_t v) { return (v + 255) / 256 * 256; };
+    DenseDecodeScratch s;
+    s.feats = up((size_t)n * (size_t)feats * (size_t)elem_bytes(act_dtype));
+    s.part = up(down_skinny_workspace_bytes(n, hidden, feats, act_dtype));
+    s.counters = up((size_t)dense_decode_counters(hidden) * sizeof(int));
+    s.total = s.feats + s.part + s.counters;
+    return s;
+}
+
+static bool dense_decode_dims_ok(int act_dtype, int64_t n, int64_t hidden, int64_t shared_width, int num_experts,
+                                 int64_t expert_width) {
+    return (act_dtype == TRMOE_F32 || act_dtype == TRMOE_BF16) && n >= 1 && n <= kSkinnyMaxTokens && hidden > 0 &&
+           hidden < (int64_t)1 << 24 && shared_width >= 0 && shared_width < (int64_t)1 << 24 && num_experts >= 1 &&
+           num_experts <= kMaxExperts && expert_width > 0 && expert_width < (int64_t)1 << 20;
+}
+
+size_t trmoe_dense_decode_workspace_bytes(int act_dtype, int64_t n_tokens, int64_t hidden, int64_t shared_width,
+                                          int num_experts, int64_t expert_width) {
+    if (!dense_decode_dims_ok(act_dtype, n_tokens, hidden, shared_width, num_experts, expert_width)) return 0;
+    return dense_decode_scratch(act_dtype, n_tokens, hidden,
+                                trmoe_dense_routed_features(shared_width, num_experts, expert_width))
+        .total;
+}
+
+int trmoe_dense_decode(int act_dtype, const void* x, int64_t n_tokens, int64_t hidden, int64_t ldx,
+                       const void* w_gate_up_frag, const void* w_down_frag, int64_t shared_width, int num_experts,
+                       int64_t expert_width, const int64_t* token_ids, const int64_t* route_table, int64_t vocab_size,
+                       int top_k, const float* route_weights, float shared_scale, float routed_scale,
+                       const float* row_scale, float rms_eps, const void* residual, int64_t ldr, void* out, int64_t ldo,
+                       void* workspace, size_t workspace_bytes, void* stream) {
+    if (n_tokens == 0) return TRMOE_OK;
+    TRMOE_REQUIRE(dense_decode_dims_ok(act_dtype, n_tokens, hidden, shared_width, num_experts, expert_width),
+                  "dense_decode: f32 or bf16, 1 to 128 tokens and positive dimensions");
+    TRMOE_REQUIRE(top_k >= 1 && top_k <= kMaxTopK && top_k <= num_experts && vocab_size > 0, "dense_decode: bad routing");
+    TRMOE_REQUIRE(ldx >= hidden && ldo >= hidden && (residual == nullptr || ldr >= hidden),
+                  "dense_decode: row stride < hidden");
+    TRMOE_REQUIRE(x && w_gate_up_frag && w_down_frag && token_ids && route_table && route_weights && out && workspace,
+                  "dense_decode: null pointer");
+    TRMOE_REQUIRE(rows_ok(x, ldx, elem_bytes(act_dtype)) && aligned16(w_gate_up_frag) && aligned16(w_down_frag) &&
+                      aligned16(workspace),
+                  "dense_decode: x, weights and workspace must be 16-byte aligned, x rows a multiple of 16 bytes");
+    TRMOE_REQUIRE(workspace_bytes >= trmoe_dense_decode_workspace_bytes(act_dtype, n_tokens, hidden, shared_width,
+                                                                        num_experts, expert_width),
+                  "dense_decode: workspace smaller than trmoe_dense_decode_workspace_bytes()");
+    const int64_t feats = trmoe_dense_routed_features(shared_width, num_experts, expert_width);
+    const DenseDecodeScratch s = dense_decode_scratch(act_dtype, n_tokens, hidden, feats);
+    char* ws = static_cast<char*>(workspace);
+    GateUpArgs g{};
+    g.x = x;
+    g.ldx = ldx;
+    g.M = n_tokens;
+    g.K = (int)hidden;
+    g.ldw = round_up(hidden, 8);
+    g.w_frag = w_gate_up_frag;
+    g.h = ws;
+    g.ldh = feats;
+    g.shared_mult = shared_scale;
+    g.shared_feats = round_up(shared_width, 128);
+    g.expert_feats = round_up(expert_width, 64);
+    g.ids = token_ids;
+    g.table = route_table;
+    g.vocab = vocab_size;
+    g.top_k = top_k;
+    for (int j = 0; j < 4; ++j) g.rw[j] = j < top_k ? routed_scale * route_weights[j] : 0.f;
+    g.row_scale = row_scale;
+    g.rms_eps = rms_eps;
+    DownArgs d{};
+    d.h = ws;
+    d.ldh = feats;
+    d.M = n_tokens;
+    d.K = (int)feats;
+    d.ldw = round_up(feats, 8);
+    d.N = (int)hidden;
+    d.shared_scale = 1.0f;
+    d.routed_scale = 1.0f;
+    d.residual = residual;
+    d.ldr = ldr;
+    d.out = out;
+    d.ldo = ldo;
+    d.w_frag = w_down_frag;
+    return launch_dense_decode(act_dtype, g, 2 * feats, d, ws + s.feats, reinterpret_cast<int*>(ws + s.feats + s.part),
+                               as_stream(stream));
+}
+
+// Scratch of trmoe_decoder_step: a hidden buffer, the attention output, then
+// the scratch of the output projection, the attention and the MLP half (used
+// at different times, kept apart).
 struct StepScratch {
-    size_t h, attn, feats, down, attn_ws, total;
+    size_t h, attn, down, attn_ws, mlp, total;
 };
 
 static bool step_dims(const trmoe_decoder_dims* d, int64_t batch, StepScratch* s) {
@@ -1072,13 +1163,11 @@ static bool step_dims(const trmoe_decoder_dims* d, int64_t batch, StepScratch* s
     auto up = [](size_t v) { return (v + 255) / 256 * 256; };
     s->h = up((size_t)batch * (size_t)d->hidden * 2);
     s->attn = up((size_t)batch * (size_t)qd * 2);
-    s->feats = up((size_t)batch * (size_t)feats * 2);
-    const size_t down_o = down_skinny_workspace_bytes(batch, d->hidden, qd, TRMOE_BF16);
-    const size_t down_m = down_skinny_workspace_bytes(batch, d->hidden, feats, TRMOE_BF16);
-    s->down = up(down_o > down_m ? down_o : down_m);
+    s->down = up(down_skinny_workspace_bytes(batch, d->hidden, qd, TRMOE_BF16));
+    s->mlp = dense_decode_scratch(TRMOE_BF16, batch, d->hidden, feats).total;
     s->attn_ws = up(trmoe_decode_attention_workspace_bytes(batch, d->hidden, d->num_heads, d->num_kv_heads,
                                                            d->cache_length));
-    s->total = s->h + s->attn + s->feats + s->down + s->attn_ws;
+    s->total = s->h + s->attn + s->down + s->attn_ws + s->mlp;
     return true;
 }
 
@@ -1100,15 +1189,13 @@ int trmoe_decoder_step(const trmoe_decoder_dims* d, const trmoe_decoder_layer* l
     char* p = static_cast<char*>(workspace);
     void* mid = p;
     void* attn = p + s.h;
-    void* feats = p + s.h + s.attn;
-    void* down = p + s.h + s.attn + s.feats;
-    void* attn_ws = p + s.h + s.attn + s.feats + s.down;
+    void* down = p + s.h + s.attn;
+    void* attn_ws = p + s.h + s.attn + s.down;
+    void* mlp = p + s.h + s.attn + s.down + s.attn_ws;
     const int64_t H = d->hidden, qd = (int64_t)d->num_heads * 64;
-    const int64_t F = trmoe_dense_routed_features(d->shared_width, d->num_experts, d->expert_width);
     for (int64_t i = 0; i < d->layers; ++i) {
         const trmoe_decoder_layer& l = layers[i];
-        TRMOE_REQUIRE(l.w_o && l.w_gate_up && l.w_gate_up_frag && l.w_down && l.w_down_frag,
-                      "decoder_step: null pointer in a layer");
+        TRMOE_REQUIRE(l.w_o != nullptr, "decoder_step: null pointer in a layer");
         int st = trmoe_decode_attention(hidden_rows, batch, H, H, l.input_norm, d->norm_eps, l.w_kqv, d->num_heads,
                                         d->num_kv_heads, l.q_norm, l.k_norm, d->qk_eps, cos, sin, positions, position,
                                         l.k_cache, l.v_cache, d->cache_length, d->attn_scale, attn, attn_ws, s.attn_ws,
@@ -1118,21 +1205,10 @@ int trmoe_decoder_step(const trmoe_decoder_dims* d, const trmoe_decoder_layer* l
         st = trmoe_shared_down_combine(TRMOE_BF16, TRMOE_BF16, attn, batch, qd, qd, l.w_o, nullptr, H, nullptr, H,
                                        nullptr, 1, one, 1.0f, 0.0f, hidden_rows, H, mid, H, down, s.down, stream);
         if (st) return st;
-        trmoe_call_extras ex{};
-        ex.rms_eps = d->norm_eps;
-        ex.w_frag = l.w_gate_up_frag;
-        ex.w_frag_cols = H;
-        st = trmoe_dense_routed_gate_up_ex(TRMOE_BF16, TRMOE_BF16, mid, batch, H, H, l.w_gate_up, nullptr,
-                                           d->shared_width, d->num_experts, d->expert_width, token_ids, l.route_table,
-                                           d->vocab_size, d->top_k, d->route_weights, d->shared_scale, d->routed_scale,
-                                           feats, F, &ex, stream);
-        if (st) return st;
-        ex = trmoe_call_extras{};
-        ex.w_frag = l.w_down_frag;
-        ex.w_frag_cols = F;
-        st = trmoe_shared_down_combine_ex(TRMOE_BF16, TRMOE_BF16, feats, batch, F, F, l.w_down, nullptr, H, nullptr, H,
-                                          nullptr, 1, one, 1.0f, 1.0f, mid, H, hidden_rows, H, down, s.down, &ex,
-                                          stream);
+        st = trmoe_dense_decode(TRMOE_BF16, mid, batch, H, H, l.w_gate_up_frag, l.w_down_frag, d->shared_width,
+                                d->num_experts, d->expert_width, token_ids, l.route_table, d->vocab_size, d->top_k,
+                                d->route_weights, d->shared_scale, d->routed_scale, nullptr, d->norm_eps, mid, H,
+                                hidden_rows, H, mlp, s.mlp, stream);
         if (st) return st;
     }
     return TRMOE_OK;

@@ -18,6 +18,7 @@
 
 #include "trmoe_common.h"
 #include "trmoe_internal.h"
+#include "trmoe_skinny.h"
 
 #include <algorithm>
 
@@ -170,15 +171,6 @@ __global__ __launch_bounds__(64 * kQkvWaves) void k_decode_qkv(DecodeAttnArgs a)
     }
 }
 
-// Device-scope accesses of the split partials: they bypass the XCD's own L2,
-// so a workgroup of another XCD sees them without a cache write-back.
-__device__ __forceinline__ void store_dev(float* p, float v) {
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ float load_dev(const float* p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
 // Attention of one new token: workgroup (split, kv head, sequence) takes the
 // cache positions [split * chunk, + chunk) below the current one; the split
 // that holds the current position normalises, rotates and stores its k and v
@@ -190,24 +182,26 @@ __device__ __forceinline__ float load_dev(const float* p) {
 // else to hide latency behind: the first K/V rows are requested before the
 // position is known, and reductions stay on the vector ALU.  Against all heads
 // in every wave and one 128-position split: 14.2 us at 213 positions before.
+// 16 waves: 256 positions per workgroup cost one batch of loads, and up to that
+// length nothing crosses workgroups (10.6 us with 4 waves and four splits).
+constexpr int kAttnWaves = 16;
 constexpr int kUnroll = 4;
 constexpr int kMaxSplits = 64;
 constexpr int kPart = kD + 2;   // 64 sums, the maximum, the weight
 template <int G>
 struct HeadSplit {
     static constexpr int HW = G >= 4 ? 4 : G;          // waves over heads
-    static constexpr int PW = 4 / HW;                  // waves over positions
+    static constexpr int PW = kAttnWaves / HW;         // waves over positions
     static constexpr int HPW = (G + HW - 1) / HW;      // heads per wave
 };
 
 template <int G>
-__global__ __launch_bounds__(256) void k_decode_attn(DecodeAttnArgs a, int chunk, int splits) {
+__global__ __launch_bounds__(64 * kAttnWaves) void k_decode_attn(DecodeAttnArgs a, int chunk, int splits) {
     using HS = HeadSplit<G>;
     constexpr int HPW = HS::HPW, PW = HS::PW;
     __shared__ float s_ml[PW][G][2];
     __shared__ float s_acc[PW][G][kD];
     __shared__ float s_f[G][kMaxSplits + 1];
-    __shared__ int s_last;
     const int split = (int)blockIdx.x, kvh = (int)blockIdx.y, b = (int)blockIdx.z;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     const int hw = wave / PW, pw = wave % PW;
@@ -328,7 +322,7 @@ __global__ __launch_bounds__(256) void k_decode_attn(DecodeAttnArgs a, int chunk
     __syncthreads();
     bf16_t* out = a.attn + (int64_t)b * (a.kvh * G * kD) + kvh * G * kD;
     float* part = a.part + ((int64_t)(b * a.kvh + kvh) * splits) * (G * kPart);
-    for (int i = threadIdx.x; i < G * kD; i += 256) {
+    for (int i = threadIdx.x; i < G * kD; i += 64 * kAttnWaves) {
         const int g = i / kD, d = i % kD;
         float mn = s_ml[0][g][0];
 #pragma unroll
@@ -352,16 +346,9 @@ __global__ __launch_bounds__(256) void k_decode_attn(DecodeAttnArgs a, int chunk
         }
     }
     if (splits == 1) return;
-    // this wave's partials have reached memory before the count that says so
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if (threadIdx.x == 0)
-        s_last = __hip_atomic_fetch_add(a.counters + b * a.kvh + kvh, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
-                 splits - 1;
-    __syncthreads();
-    if (!s_last) return;
+    if (!last_arrival(a.counters + b * a.kvh + kvh, splits)) return;
     // the splits' factors, one lane per split, then the weighted sums
-    for (int g = wave; g < G; g += 4) {
+    for (int g = wave; g < G; g += kAttnWaves) {
         const float* src = part + ((int64_t)lane * G + g) * kPart + kD;
         const float ms = lane < splits ? load_dev(src) : -1e30f, ls = lane < splits ? load_dev(src + 1) : 0.f;
         float mx = ms;
@@ -374,7 +361,7 @@ __global__ __launch_bounds__(256) void k_decode_attn(DecodeAttnArgs a, int chunk
         s_f[g][lane] = f / lt;
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < G * kD; i += 256) {
+    for (int i = threadIdx.x; i < G * kD; i += 64 * kAttnWaves) {
         const int g = i / kD, d = i % kD;
         const float* src = part + (int64_t)g * kPart + d;
         float v = 0.f;
@@ -397,12 +384,12 @@ int launch_qk_rope(const RopeArgs& a, hipStream_t stream) {
     return check_launch("qk_norm_rope");
 }
 
-// Positions per split: at least 64 (two batches of a lane group's loads), more
-// when the (sequence, kv head) pairs fill the CUs twice over or the splits
-// would pass one lane each in the merge.
+// Positions per split: at least 256 (a workgroup's first batch of loads or
+// two), more when the (sequence, kv head) pairs fill the CUs or the splits would
+// pass one lane each in the merge.
 static int decode_chunk(int64_t L, int pairs) {
-    int64_t splits = std::max(1, 512 / std::max(1, pairs));
-    splits = std::min<int64_t>({splits, (L + 63) / 64, kMaxSplits});
+    int64_t splits = std::max(1, 256 / std::max(1, pairs));
+    splits = std::min<int64_t>({splits, (L + 255) / 256, kMaxSplits});
     return (int)(((L + splits - 1) / splits + 31) / 32 * 32);
 }
 
@@ -425,7 +412,7 @@ int launch_decode_attn(const DecodeAttnArgs& a, int group, hipStream_t stream) {
                 : group == 8 ? k_decode_attn<8>
                              : nullptr;
     if (kern == nullptr) return set_error(TRMOE_ERR_UNSUPPORTED, "decode_attention: 1, 2, 4, 7 or 8 query heads per kv head");
-    hipLaunchKernelGGL(kern, grid, dim3(256), 0, stream, a, chunk, splits);
+    hipLaunchKernelGGL(kern, grid, dim3(64 * kAttnWaves), 0, stream, a, chunk, splits);
     return check_launch("decode_attention");
 }
 

@@ -500,9 +500,13 @@ __device__ __forceinline__ void tile_loop_dma(const AP& ap, const BP& bp, int K,
 // barrier, LDS read, MFMA): groups run KS such chains side by side.  Group g
 // takes stages g, g + KS, ...; requests past the last stage read zeros, and
 // the final barrier drains them before the caller reuses LDS.
-template <class Kind, class Shape, class AP, class BP>
+// `pre` runs while the first stages load (its own loads drain them).
+struct NoPre {
+    __device__ __forceinline__ void operator()() const {}
+};
+template <class Kind, class Shape, class AP, class BP, class Pre>
 __device__ __forceinline__ void tile_loop_ring(const AP& ap, const BP& bp, int K, char* lds, int wm0, int wn0,
-                                               f32x16 (&acc)[Shape::TM][Shape::TN]) {
+                                               f32x16 (&acc)[Shape::TM][Shape::TN], const Pre& pre) {
     constexpr int S = Shape::kStages, KS = Shape::KS;
     constexpr int kABytes = Shape::BM * kRowBytes;
     constexpr int kPer = AP::kInstr + BP::kInstr;
@@ -515,6 +519,7 @@ __device__ __forceinline__ void tile_loop_ring(const AP& ap, const BP& bp, int K
         ap.issue(s * KS + g, lds + s * Shape::kStageBytes);
         bp.issue(s * KS + g, lds + s * Shape::kStageBytes + kABytes);
     }
+    pre();
     int cur = 0, nxt = S - 1;
     for (int kt = 0; kt < nk; ++kt) {
         wait_vmcnt<kPer * (S - 2)>();   // this wave's loads of stage kt have landed
@@ -569,11 +574,12 @@ __device__ __forceinline__ bool reduce_groups(char* lds, f32x16 (&acc)[Shape::TM
     return g == 0;
 }
 
-template <class Kind, class Shape, class AProv, class BProv>
+template <class Kind, class Shape, class AProv, class BProv, class Pre = NoPre>
 __device__ __forceinline__ void tile_loop(const AProv& ap, const BProv& bp, int K, char* lds, int wm0, int wn0,
-                                          f32x16 (&acc)[Shape::TM][Shape::TN]) {
+                                          f32x16 (&acc)[Shape::TM][Shape::TN], const Pre& pre = Pre{}) {
+    if constexpr (!Shape::kRing) pre();
     if constexpr (Shape::kRing)
-        tile_loop_ring<Kind, Shape>(ap, bp, K, lds, wm0, wn0, acc);
+        tile_loop_ring<Kind, Shape>(ap, bp, K, lds, wm0, wn0, acc, pre);
     else if constexpr (Shape::PGR == 4 || Shape::PGR == 6)
         tile_loop_dma<Kind, Shape>(ap, bp, K, lds, wm0, wn0, acc);
     else

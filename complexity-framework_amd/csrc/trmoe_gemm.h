@@ -78,6 +78,9 @@ struct GateUpArgs {
     // exponent per token and 32 features (row stride ldhs bytes).
     void* hs;
     int64_t ldhs;
+    // Fused decode: the split counters of the down call that follows, cleared here.
+    int* zero;
+    int zero_n;
 };
 
 struct DownArgs {
@@ -102,6 +105,7 @@ struct DownArgs {
     int64_t ldo;
     int vec_ok;             // y / residual / out rows 16-byte aligned (vector epilogue)
     const void* w_frag;     // fragment-major copy of w for the decode kernels, or null
+    int* counters;          // decode split-K: one cleared count per column tile (the last split sums), or null
     // Expert-grouped mode (offsets != nullptr): blockIdx.x walks the
     // (expert, row tile) pairs of a K1 partition; A rows are
     // a[gather[r] % gather_mod] (contiguous partition rows r when gather is
@@ -261,6 +265,12 @@ struct WgradArgs {
 };
 
 int launch_pack(const PackArgs& p, hipStream_t stream);
+// Decode of a dense-routed layer: gate|up (a.w_frag) then down (d.w_frag) with
+// the splits summed by their last workgroup; `part` holds the down's partials
+// and dense_decode_counters(N) ints behind them are its counters.
+int dense_decode_counters(int64_t N);
+int launch_dense_decode(int act, const GateUpArgs& a, int64_t packed_rows, const DownArgs& d, void* part,
+                        int* counters, hipStream_t stream);
 int launch_gate_up_skinny(int act, int wdt, const GateUpArgs& a, int64_t packed_rows, hipStream_t stream);
 size_t down_skinny_workspace_bytes(int64_t M, int64_t N, int64_t K, int act);
 int launch_pack_fragments_e4m3(const void* src, int64_t rows, int64_t cols, int64_t ld, void* dst, int64_t dst_groups,

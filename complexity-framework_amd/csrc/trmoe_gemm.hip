@@ -224,25 +224,27 @@ __global__ __launch_bounds__(Shape::NT) void k_gate_up_swiglu(GateUpArgs a) {
     // fused RMSNorm: the row scales of the tile's rows (partition rows read
     // their token's), read back in the epilogue after the main loop's barriers
     __shared__ float s_rscale[Shape::BM];
-    if (a.row_scale != nullptr && threadIdx.x < Shape::BM) {
-        const int64_t row = m0 + threadIdx.x;
-        int64_t tok = row;
-        if constexpr (GROUPED) {
-            if (a.gather != nullptr && row < a.M) tok = (int64_t)((uint64_t)a.gather[row] % (uint64_t)a.gather_mod);
-        }
-        s_rscale[threadIdx.x] = row < a.M ? a.row_scale[tok] : 0.0f;
-    }
     typename BProvOf<Kind, FP8, Shape>::type bp;
     init_b<Kind, FP8, Shape>(bp, a.w, a.ldw, n0, a.K);
 
     // Routes of this tile's rows, gathered once while the first stages load;
     // read back in the epilogue after the main loop's barriers.
     __shared__ int s_route[ROUTED ? Shape::BM : 1][kMaxTopK];
-    gate_up_routes<Shape, ROUTED>(a, m0, n0, s_route);
+    auto row_data = [&]() {
+        if (a.row_scale != nullptr && threadIdx.x < Shape::BM) {
+            const int64_t row = m0 + threadIdx.x;
+            int64_t tok = row;
+            if constexpr (GROUPED) {
+                if (a.gather != nullptr && row < a.M) tok = (int64_t)((uint64_t)a.gather[row] % (uint64_t)a.gather_mod);
+            }
+            s_rscale[threadIdx.x] = row < a.M ? a.row_scale[tok] : 0.0f;
+        }
+        gate_up_routes<Shape, ROUTED>(a, m0, n0, s_route);
+    };
 
     f32x16 acc[Shape::TM][Shape::TN];
     zero_acc<Kind>(acc);
-    tile_loop<Kind, Shape>(ap, bp, a.K, lds, wm0, wn0, acc);
+    tile_loop<Kind, Shape>(ap, bp, a.K, lds, wm0, wn0, acc, row_data);
     const bool holder = reduce_groups<Shape>(lds, acc);
     if constexpr (SAVE) {
         if (holder) gate_up_save<Kind, Shape>(a, acc, m0, n0, a.n_base + (int64_t)gridDim.y * Shape::BN);

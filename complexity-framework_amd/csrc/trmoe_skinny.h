@@ -28,6 +28,28 @@ __device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t r, char* lds, int o
     __builtin_amdgcn_raw_ptr_buffer_load_lds(r, TRMOE_LDS_PTR(lds), 16, off, 0, 0, 0);
 }
 
+// Device-scope accesses of split partials: they pass the XCD's own L2, so a
+// workgroup of another XCD sees them without a cache write-back.
+__device__ __forceinline__ void store_dev(float* p, float v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float load_dev(const float* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// True for every thread of the last of `n` workgroups to arrive at *count,
+// after the partials each stored with store_dev (and before reading them).
+__device__ __forceinline__ bool last_arrival(int* count, int n) {
+    __shared__ int s_last;
+    // this wave's partials have reached memory before the count that says so
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0)
+        s_last = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == n - 1;
+    __syncthreads();
+    return s_last != 0;
+}
+
 // red[wave][e][lane] with e = (tm*NU+u)*4+i.
 template <int MT, int NU>
 __device__ __forceinline__ void skinny_stash(float* red, const f32x4 (&acc)[MT][NU]) {

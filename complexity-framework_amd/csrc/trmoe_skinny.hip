@@ -288,6 +288,8 @@ __global__ __launch_bounds__(64 * NW) void k_gate_up_skinny(GateUpArgs a) {
     const bool rms_in = a.row_scale == nullptr && a.rms_eps > 0.0f;
     const bool rms = rms_in || a.row_scale != nullptr;
     float ssq[ssq_rows<MT>()] = {};
+    if (blockIdx.x == 0)
+        for (int i = threadIdx.x; i < a.zero_n; i += NT) a.zero[i] = 0;
     staged_k_loop<Kind, FP8, MT, 2, SB, SW, 16, FRAG>(ar, (int)a.M, (int)(a.ldx * (int64_t)sizeof(T)), region, wr,
                                                       w_row0, (int)(a.ldw * kWB), w_off, s0, s1, kb_a, acc, rms_in,
                                                       ssq);
@@ -418,8 +420,29 @@ __global__ __launch_bounds__(64 * NW) void k_down_skinny(DownArgs a, float* part
         const float v = skinny_sum<MT, NU, NW>(red, tm, u, i, l);
         if (single)
             down_finish<T>(a, row, col, v);
+        else if (a.counters != nullptr)
+            store_dev(dst + row * (int64_t)a.N + col, v);
         else
             dst[row * (int64_t)a.N + col] = v;
+    }
+    if (single || a.counters == nullptr) return;
+    // the last split of the column tile sums them all, in split order: a
+    // round trip to memory instead of a launch (4.6 us at 64 tokens)
+    if (!last_arrival(a.counters + ct, splits)) return;
+    const int plane = (int)a.M * (int)a.N;
+    for (int qi = threadIdx.x; qi < (int)a.M * kCols; qi += NT) {
+        const int row = qi / kCols, col = (int)n0 + qi % kCols;
+        if (col >= a.N) continue;
+        const float* p = part + row * (int)a.N + col;
+        float s = 0.f;
+        for (int sp = 0; sp < splits; sp += 4) {
+            float t[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) t[j] = load_dev(p + (sp + j < splits ? sp + j : splits - 1) * plane);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) s += sp + j < splits ? t[j] : 0.f;
+        }
+        down_finish<T>(a, row, col, s);
     }
 }
 
@@ -521,7 +544,7 @@ int down_skinny_mt(const DownArgs& a, float* part, int sps, int splits, hipStrea
     const int ncol = (int)((a.N + COLS - 1) / COLS);
     hipLaunchKernelGGL(kern, dim3((unsigned)(ncol * splits)), dim3(64 * NW), kLds, stream, a, part, sps, ncol, splits);
     st = check_launch("shared_down_combine (skinny)");
-    if (st || splits == 1) return st;
+    if (st || splits == 1 || a.counters != nullptr) return st;
     const bool vec = a.N % 4 == 0 && (reinterpret_cast<uintptr_t>(part) & 15) == 0;
     auto red = vec ? k_down_reduce<typename Kind::T, 4> : k_down_reduce<typename Kind::T, 1>;
     const int64_t total = a.M * (int64_t)(vec ? a.N / 4 : a.N);
@@ -633,6 +656,29 @@ size_t down_skinny_workspace_bytes(int64_t M, int64_t N, int64_t K, int act) {
     const int spans = (int)((K * eb + 127) / 128);
     const int64_t splits = (spans + down_spans_per_split(M, spans) - 1) / down_spans_per_split(M, spans);
     return (size_t)(splits * M * N * (int64_t)sizeof(float));
+}
+
+int dense_decode_counters(int64_t N) { return (int)((N + 7) / 8); }
+
+int launch_dense_decode(int act, const GateUpArgs& g, int64_t packed_rows, const DownArgs& dn, void* part,
+                        int* counters, hipStream_t stream) {
+    if (dn.M * (int64_t)dn.N >= ((int64_t)1 << 31))
+        return set_error(TRMOE_ERR_UNSUPPORTED, "dense_decode: needs tokens * hidden < 2^31");
+    const int eb = act == TRMOE_F32 ? 4 : 2;
+    const int spans = (int)(((int64_t)dn.K * eb + 127) / 128);
+    const int sps = down_spans_per_split(dn.M, spans), splits = (spans + sps - 1) / sps;
+    GateUpArgs a = g;
+    DownArgs d = dn;
+    d.counters = splits > 1 ? counters : nullptr;
+    a.zero = counters;
+    a.zero_n = splits > 1 ? dense_decode_counters(dn.N) : 0;
+    int st;
+    if (act == TRMOE_BF16)
+        st = gate_up_skinny_frag<KindBF16, false, true>(a, packed_rows, stream);
+    else
+        st = gate_up_skinny_frag<KindF32, false, true>(a, packed_rows, stream);
+    if (st) return st;
+    return launch_down_skinny(act, act, d, part, stream);
 }
 
 int launch_down_skinny(int act, int wdt, const DownArgs& a, void* workspace, hipStream_t stream) {

@@ -504,6 +504,23 @@ int trmoe_shared_down_combine_ex(int act_dtype, int w_dtype, const void* h, int6
                                  const trmoe_call_extras* extras, void* stream);
 
 /*
+ * A dense-routed layer on at most 128 tokens in one call (bf16 / f32): the
+ * gate|up and down of the *_ex entry points above, on the fragment-major copies
+ * of the dense-routed packs (trmoe_pack_fragments with cols = hidden, and cols =
+ * trmoe_dense_routed_features() for the down), with the fused RMSNorm scales
+ * (row_scale, or rms_eps > 0) and the residual; the down's K splits are summed
+ * by the last of them.
+ */
+size_t trmoe_dense_decode_workspace_bytes(int act_dtype, int64_t n_tokens, int64_t hidden, int64_t shared_width,
+                                          int num_experts, int64_t expert_width);
+int trmoe_dense_decode(int act_dtype, const void* x, int64_t n_tokens, int64_t hidden, int64_t ldx,
+                       const void* w_gate_up_frag, const void* w_down_frag, int64_t shared_width, int num_experts,
+                       int64_t expert_width, const int64_t* token_ids, const int64_t* route_table, int64_t vocab_size,
+                       int top_k, const float* route_weights, float shared_scale, float routed_scale,
+                       const float* row_scale, float rms_eps, const void* residual, int64_t ldr, void* out, int64_t ldo,
+                       void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * One decode step of a whole decoder (bf16, dense-routed layers, batch <= 16):
  * for every layer trmoe_decode_attention, the output projection with its
  * residual, and the MLP half with its RMSNorm and residual, queued by one call
@@ -526,10 +543,8 @@ typedef struct trmoe_decoder_layer {
     const void* w_o;             /* [hidden, num_heads * 64] */
     void* k_cache;               /* [batch, num_kv_heads, cache_length, 64] */
     void* v_cache;
-    const void* w_gate_up;       /* the layer's dense-routed packs, its RMSNorm weight folded in, */
-    const void* w_gate_up_frag;  /* and their fragment-major copies */
-    const void* w_down;
-    const void* w_down_frag;
+    const void* w_gate_up_frag;  /* fragment-major copies of the layer's dense-routed packs, its */
+    const void* w_down_frag;     /* RMSNorm weight folded into the gate|up */
     const int64_t* route_table;  /* [top_k, vocab_size] */
 } trmoe_decoder_layer;
 
