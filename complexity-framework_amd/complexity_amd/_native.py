@@ -156,6 +156,8 @@ SIGNATURES = {
         [_c_vp, _c_i64, _c_i64, _c_int, _c_int, _c_i64, _c_vp, _c_vp, _c_float, _c_vp, _c_vp, _c_i64, _c_i64, _c_vp,
          _c_vp, _c_vp, _c_vp, _c_i64, _c_vp],
     ),
+    "trmoe_prefill_attention": (
+        _c_int, [_c_vp, _c_vp, _c_vp, _c_i64, _c_i64, _c_int, _c_int, _c_i64, _c_float, _c_vp, _c_vp]),
     "trmoe_decode_attention_workspace_bytes": (_c_size, [_c_i64, _c_i64, _c_int, _c_int, _c_i64]),
     "trmoe_decode_attention": (
         _c_int,

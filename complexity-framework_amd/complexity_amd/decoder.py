@@ -22,8 +22,9 @@ replays a HIP-graph capture of the decode step (the position is a device
 counter, so one capture serves every step).
 
 On a GPU in bf16 the attention half runs on the HIP kernels too
-(``ops.qk_norm_rope``, ``ops.decode_attention``): a prompt's q/k norm, rotation
-and cache writes are one pass over the projection, and a decode step of up to
+(``ops.qk_norm_rope``, ``ops.prefill_attention``, ``ops.decode_attention``): a
+prompt's q/k norm, rotation and cache writes are one pass over the projection,
+its attention reads the caches, and a decode step of up to
 16 sequences is three launches per block (norm + projection; q/k norm,
 rotation, cache write and attention; output projection + residual).
 
@@ -463,13 +464,13 @@ class TRGQADecoder(nn.Module):
             if hip:
                 q = ops.qk_norm_rope(F.linear(x, attn.kqv_weight()).view(B * T, -1), B, cfg.num_heads,
                                      attn.q_norm.weight, attn.k_norm.weight, attn.q_norm.eps, cos, sin,
-                                     self.k_cache[i], self.v_cache[i]).transpose(1, 2)
-                k, v = self.k_cache[i][:, :, :T], self.v_cache[i][:, :, :T]
+                                     self.k_cache[i], self.v_cache[i])
+                h = h + attn.o_proj(ops.prefill_attention(q, self.k_cache[i], self.v_cache[i], attn.scale))
             else:
                 q, k, v = attn.project(x, cos, sin)
                 self.k_cache[i][:, :, :T].copy_(k)
                 self.v_cache[i][:, :, :T].copy_(v)
-            h = h + attn.output(attn.prefill_attention(q, k, v))
+                h = h + attn.output(attn.prefill_attention(q, k, v))
             _end(ev)
             ev = _events(timings, "mlp")
             h = self._mlp(block, h, input_ids)

@@ -603,6 +603,23 @@ def qk_norm_rope(kqv: torch.Tensor, sequences: int, num_heads: int, q_weight: to
 
 
 @_on_tensor_device
+def prefill_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, scale: float) -> torch.Tensor:
+    """Causal attention [B, T, heads * 64] of a prompt's q [B, T, heads, 64] over
+    positions 0 .. T - 1 of the caches [B, kv heads, L, 64]."""
+    _require_cuda(q, k_cache, v_cache)
+    B, T, heads, D = q.shape
+    if (q.dtype != torch.bfloat16 or k_cache.dtype != q.dtype or v_cache.dtype != q.dtype or D != ATTN_HEAD_DIM
+            or k_cache.shape != v_cache.shape or k_cache.shape[0] != B or k_cache.shape[3] != D
+            or not (q.is_contiguous() and k_cache.is_contiguous() and v_cache.is_contiguous())):
+        raise ValueError("prefill_attention: contiguous bf16 q [B, T, heads, 64] and caches [B, kv heads, L, 64]")
+    out = torch.empty(B, T, heads * D, dtype=q.dtype, device=q.device)
+    st = _lib().trmoe_prefill_attention(_p(q), _p(k_cache), _p(v_cache), B, T, heads, k_cache.shape[1],
+                                        k_cache.shape[2], float(scale), _p(out), _stream(q))
+    N.check(st, "trmoe_prefill_attention")
+    return out
+
+
+@_on_tensor_device
 def decode_attention(x: torch.Tensor, norm_weight: torch.Tensor, norm_eps: float, w_kqv: torch.Tensor, num_heads: int,
                      q_weight: torch.Tensor, k_weight: torch.Tensor, qk_eps: float, cos: torch.Tensor,
                      sin: torch.Tensor, position: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,

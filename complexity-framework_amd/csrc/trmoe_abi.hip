@@ -983,6 +983,30 @@ int trmoe_qk_norm_rope(const void* kqv, int64_t sequences, int64_t tokens, int n
     return launch_qk_rope(a, as_stream(stream));
 }
 
+int trmoe_prefill_attention(const void* q, const void* k_cache, const void* v_cache, int64_t sequences, int64_t tokens,
+                            int num_heads, int num_kv_heads, int64_t cache_length, float scale, void* out,
+                            void* stream) {
+    TRMOE_REQUIRE(sequences >= 0 && tokens >= 0 && num_heads > 0 && num_kv_heads > 0 && num_heads % num_kv_heads == 0,
+                  "prefill_attention: bad dimensions");
+    TRMOE_REQUIRE(tokens <= cache_length && tokens < (int64_t)1 << 23, "prefill_attention: tokens past the cache or 2^23");
+    TRMOE_REQUIRE(sequences * num_heads < 65536, "prefill_attention: sequences * num_heads must be below 65536");
+    if (sequences == 0 || tokens == 0) return TRMOE_OK;
+    TRMOE_REQUIRE(q && k_cache && v_cache && out, "prefill_attention: null pointer");
+    TRMOE_REQUIRE(aligned16(q) && aligned16(k_cache) && aligned16(v_cache) && aligned16(out),
+                  "prefill_attention: operands must be 16-byte aligned");
+    PrefillAttnArgs a{};
+    a.q = static_cast<const bf16_t*>(q);
+    a.k = static_cast<const bf16_t*>(k_cache);
+    a.v = static_cast<const bf16_t*>(v_cache);
+    a.T = tokens;
+    a.L = cache_length;
+    a.heads = num_heads;
+    a.kvh = num_kv_heads;
+    a.scale = scale;
+    a.out = static_cast<bf16_t*>(out);
+    return launch_prefill_attn(a, sequences, as_stream(stream));
+}
+
 // Scratch of trmoe_decode_attention: the projection (fp32), the split
 // counters and the split partials, each 256-byte aligned.
 static void decode_attn_scratch(int64_t batch, int heads, int kvh, int64_t L, size_t* qkv, size_t* counters,

@@ -26,6 +26,16 @@ struct RopeArgs {
     const int64_t* pos;
 };
 
+struct PrefillAttnArgs {
+    const bf16_t* q;         // [sequences, T, heads, 64]
+    const bf16_t* k;         // [sequences, kvh, L, 64], positions 0 .. T - 1 filled
+    const bf16_t* v;
+    int64_t T, L;
+    int heads, kvh;
+    float scale;
+    bf16_t* out;             // [sequences, T, heads * 64]
+};
+
 struct DecodeAttnArgs {
     const bf16_t* x;         // [B, H] hidden rows
     int64_t ldx;
@@ -49,6 +59,7 @@ struct DecodeAttnArgs {
 };
 
 int launch_qk_rope(const RopeArgs& a, hipStream_t stream);
+int launch_prefill_attn(const PrefillAttnArgs& a, int64_t sequences, hipStream_t stream);
 int64_t decode_attn_splits(int64_t L, int pairs);
 int launch_decode_attn(const DecodeAttnArgs& a, int group, hipStream_t stream);
 

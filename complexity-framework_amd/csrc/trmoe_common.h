@@ -353,6 +353,15 @@ __device__ __forceinline__ void lds_barrier() {
     asm volatile("" ::: "memory");
 }
 
+typedef short trmoe_v4s __attribute__((ext_vector_type(4)));
+
+// 8 bytes of a transposing LDS read: lane i of each 16-lane group receives
+// element i of the 4 rows addressed by lanes 4j + i/4 (j = 0..3).
+__device__ __forceinline__ u32x2 ds_read_tr16(const char* p) {
+    const trmoe_v4s v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) trmoe_v4s*)(p));
+    return __builtin_bit_cast(u32x2, v);
+}
+
 template <int ROWS, int NT>
 struct DmaRows {
     static constexpr int kInstr = ROWS * 8 / NT;   // wave instructions per thread per stage

@@ -554,15 +554,6 @@ struct PPLayoutF8 {
     }
 };
 
-typedef short trmoe_v4s __attribute__((ext_vector_type(4)));
-
-// 8 bytes of a transposing LDS read: lane i of each 16-lane group receives
-// element i of the 4 rows addressed by lanes 4j + i/4 (j = 0..3).
-__device__ __forceinline__ u32x2 ds_read_tr16(const char* p) {
-    const trmoe_v4s v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) trmoe_v4s*)(p));
-    return __builtin_bit_cast(u32x2, v);
-}
-
 // One token-major operand (K across rows) loaded by one group of 4 waves: a
 // stage is 64 K rows of 256 columns (512 bytes), 16-byte chunk c of row k
 // stored at chunk c ^ ((k & 3) << 2), so that the transposing fragment reads

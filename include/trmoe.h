@@ -419,6 +419,10 @@ int trmoe_pack_fragments(int dtype, const void* packed, int64_t rows, int64_t co
  * first_position + t (+ *position, a device counter, when given; a position
  * past the cache is dropped).
  *
+ * trmoe_prefill_attention: softmax(scale q K^T) V of a prompt, token t over
+ * positions 0 .. t of the caches (trmoe_qk_norm_rope's outputs with
+ * first_position 0), into out [sequence, token, num_heads * 64].
+ *
  * trmoe_decode_attention: one token per sequence (batch <= 16) at the device
  * position *position: the projection of rmsnorm(hidden) * norm_weight through
  * w_kqv [(num_heads + 2 num_kv_heads) * 64, hidden], q and k normed and
@@ -430,6 +434,9 @@ int trmoe_qk_norm_rope(const void* kqv, int64_t sequences, int64_t tokens, int n
                        int64_t ldkqv, const void* q_weight, const void* k_weight, float eps, const float* cos,
                        const float* sin, int64_t positions, int64_t first_position, const int64_t* position, void* q,
                        void* k_cache, void* v_cache, int64_t cache_length, void* stream);
+int trmoe_prefill_attention(const void* q, const void* k_cache, const void* v_cache, int64_t sequences, int64_t tokens,
+                            int num_heads, int num_kv_heads, int64_t cache_length, float scale, void* out,
+                            void* stream);
 size_t trmoe_decode_attention_workspace_bytes(int64_t batch, int64_t hidden, int num_heads, int num_kv_heads,
                                               int64_t cache_length);
 int trmoe_decode_attention(const void* hidden_rows, int64_t batch, int64_t hidden, int64_t ldx, const void* norm_weight,

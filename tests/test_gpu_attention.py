@@ -1,6 +1,8 @@
 """The decoder's attention kernels against fp32 torch: q/k norm + rotation +
-cache writes, and one decode step's attention, at cache lengths around the
-128-position splits, positions at both ends, and every supported group size.
+cache writes, a prompt's causal attention at lengths around the 64-position
+tiles and the 128-query workgroups, and one decode step's attention at cache
+lengths around the 256-position splits, positions at both ends, and every
+supported group size.
 
 Bounds: the kernels round only their bf16 outputs (half a step, 2^-9, of the
 value), and the decode attention reads k and v rounded to bf16 as the caches
@@ -82,6 +84,25 @@ def test_decode_attention(gpu, B, hidden, heads, kvh, L, pos):
     p = torch.softmax((keys @ q.unsqueeze(-1)).squeeze(-1) * scale, -1)
     want = (p.unsqueeze(-1) * vals).sum(2)
     assert _rel(got.view(B, heads, D), want) <= 2.0 ** -6   # q's own error moves the weights of up to L positions
+
+
+@pytest.mark.parametrize("B,T,heads,kvh", [(1, 1, 14, 2), (2, 31, 4, 4), (1, 64, 14, 2), (3, 65, 8, 1), (1, 128, 2, 1),
+                                           (1, 197, 14, 2), (2, 300, 3, 1), (1, 2048, 14, 2)])
+def test_prefill_attention(gpu, B, T, heads, kvh):
+    g = torch.Generator().manual_seed(T)
+    L = (T + 63) // 64 * 64 + 64
+    q = torch.randn(B, T, heads, D, generator=g).to(gpu).bfloat16() * 2
+    kc, vc = (torch.randn(B, kvh, L, D, generator=g).to(gpu).bfloat16() for _ in range(2))
+    kc[:, :, T:] = float("nan")   # positions past the prompt are never read
+    vc[:, :, T:] = float("nan")
+    scale = 1.0 / math.sqrt(D)
+    got = ops.prefill_attention(q, kc, vc, scale)
+    k, v = (c[:, :, :T].float().repeat_interleave(heads // kvh, 1) for c in (kc, vc))
+    s = (q.float().transpose(1, 2) @ k.transpose(2, 3)) * scale
+    s.masked_fill_(torch.ones(T, T, dtype=torch.bool, device=gpu).triu(1), -math.inf)
+    want = (torch.softmax(s, -1) @ v).transpose(1, 2)
+    # the weights are rounded to bf16 (2^-9 each) before the second product
+    assert _rel(got.view(B, T, heads, D), want) <= 2.0 ** -7
 
 
 def test_decode_linear_adds_residual(gpu):
