@@ -170,6 +170,12 @@ SIGNATURES = {
         [_c_int, _c_vp, _c_i64, _c_i64, _c_i64, _c_vp, _c_vp, _c_i64, _c_int, _c_i64, _c_vp, _c_vp, _c_i64, _c_int,
          _c_vp, _c_float, _c_float, _c_vp, _c_float, _c_vp, _c_i64, _c_vp, _c_i64, _c_vp, _c_size, _c_vp],
     ),
+    "trmoe_dense_layer_workspace_bytes": (_c_size, [_c_int, _c_i64, _c_i64, _c_i64, _c_int, _c_i64]),
+    "trmoe_dense_layer": (
+        _c_int,
+        [_c_int, _c_vp, _c_i64, _c_i64, _c_i64, _c_vp, _c_vp, _c_i64, _c_int, _c_i64, _c_vp, _c_vp, _c_i64, _c_int,
+         _c_vp, _c_float, _c_float, _c_float, _c_vp, _c_i64, _c_vp, _c_i64, _c_vp, _c_size, _c_vp],
+    ),
     "trmoe_decoder_step_workspace_bytes": (_c_size, [_c_dims, _c_i64]),
     "trmoe_decoder_step": (
         _c_int,

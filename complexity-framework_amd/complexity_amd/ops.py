@@ -894,6 +894,34 @@ def dense_decode(x: torch.Tensor, token_ids: torch.Tensor, route_table: torch.Te
     return out
 
 
+def dense_layer(x: torch.Tensor, token_ids: torch.Tensor, route_table: torch.Tensor, packed: "PackedLayer",
+                route_weights: Sequence[float], shared_scale: float, routed_scale: float,
+                residual: Optional[torch.Tensor] = None, rms_eps: float = 0.0) -> torch.Tensor:
+    """A dense-routed layer on more than SKINNY_MAX_TOKENS tokens (trmoe_dense_layer)."""
+    lib = _lib()
+    _require_cuda(x, token_ids, route_table, residual)
+    n, hidden = x.shape
+    ids = token_ids.reshape(-1)
+    ids = (ids if ids.dtype == torch.int64 else ids.to(torch.int64)).contiguous()
+    table = route_table.contiguous()
+    top_k, vocab = table.shape
+    if x.dtype != packed.act_dtype or ids.numel() != n or table.dtype != torch.int64:
+        raise ValueError("dense_layer: the layer's activation dtype, one token id per row and an int64 route table")
+    code = dtype_code(x.dtype)
+    out = torch.empty(n, hidden, dtype=x.dtype, device=x.device)
+    ws_bytes = lib.trmoe_dense_layer_workspace_bytes(code, n, hidden, packed.shared_width, packed.num_experts,
+                                                     packed.expert_width)
+    ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=x.device)
+    rw = _weights_arg(route_weights)
+    st = lib.trmoe_dense_layer(code, _p(x), n, hidden, x.stride(0), _p(packed.dense_gate_up), _p(packed.dense_down),
+                               packed.shared_width, packed.num_experts, packed.expert_width, _p(ids), _p(table), vocab,
+                               top_k, ctypes.cast(rw, ctypes.c_void_p), float(shared_scale), float(routed_scale),
+                               float(rms_eps), _p(residual), residual.stride(0) if residual is not None else 0, _p(out),
+                               hidden, _p(ws), ws_bytes, _stream(x))
+    N.check(st, "trmoe_dense_layer")
+    return out
+
+
 def stream_read(src: torch.Tensor, sink: torch.Tensor) -> None:
     """One launch that reads src's bytes once (trmoe_stream_read): the
     single-launch streaming floor the decode kernels are compared with.
@@ -1016,9 +1044,9 @@ def layer_forward(x: torch.Tensor, token_ids: torch.Tensor, route_table: torch.T
     and one down over the shared and every expert's features.  dense: fused gate|up over shared and
     expert features with route-weighted expert outputs, then one down GEMM.
     norm_eps: the layer runs on rmsnorm(x) (the packs must hold the gate/up
-    weights times the norm weight); the per-token scales come from the decode
-    kernels themselves up to 128 tokens (dense strategy), else from
-    rms_row_scale.  save: returns (out, gu, h): the raw gate|up outputs and,
+    weights times the norm weight); the per-token scales come from the gate|up
+    kernels themselves up to 128 tokens and on ring tiles (dense strategy), else
+    from rms_row_scale.  save: returns (out, gu, h): the raw gate|up outputs and,
     for the dense strategy, the down GEMM's input h (else None), which the
     backward reuses.  act_fp8 (e4m3 packs, grouped strategy, above decode
     sizes, hidden a multiple of 128): True or "gate_up": the shared gate|up
@@ -1037,9 +1065,12 @@ def layer_forward(x: torch.Tensor, token_ids: torch.Tensor, route_table: torch.T
     x = rows16(x)
     gu = None
     rscale, eps_in = None, 0.0
+    if norm_eps is not None and save:
+        raise ValueError("layer_forward: the fused RMSNorm is inference-only")
+    if norm_eps is not None and norm_eps > 0 and packed.strategy == STRATEGY_DENSE and n > SKINNY_MAX_TOKENS:
+        return dense_layer(x, token_ids, route_table, packed, route_weights, shared_scale, routed_scale, residual,
+                           float(norm_eps))
     if norm_eps is not None:
-        if save:
-            raise ValueError("layer_forward: the fused RMSNorm is inference-only")
         if packed.strategy == STRATEGY_DENSE and n <= SKINNY_MAX_TOKENS:
             eps_in = float(norm_eps)
         else:

@@ -1170,6 +1170,51 @@ int trmoe_dense_decode(int act_dtype, const void* x, int64_t n_tokens, int64_t h
                                as_stream(stream));
 }
 
+size_t trmoe_dense_layer_workspace_bytes(int act_dtype, int64_t n_tokens, int64_t hidden, int64_t shared_width,
+                                         int num_experts, int64_t expert_width) {
+    if ((act_dtype != TRMOE_F32 && act_dtype != TRMOE_BF16) || n_tokens < 1 || hidden < 1 || shared_width < 0 ||
+        num_experts < 1 || expert_width < 1)
+        return 0;
+    const size_t h = (size_t)n_tokens * (size_t)trmoe_dense_routed_features(shared_width, num_experts, expert_width) *
+                     (size_t)elem_bytes(act_dtype);
+    return (h + 255) / 256 * 256 + (size_t)n_tokens * sizeof(float);
+}
+
+int trmoe_dense_layer(int act_dtype, const void* x, int64_t n_tokens, int64_t hidden, int64_t ldx,
+                      const void* w_gate_up, const void* w_down, int64_t shared_width, int num_experts,
+                      int64_t expert_width, const int64_t* token_ids, const int64_t* route_table, int64_t vocab_size,
+                      int top_k, const float* route_weights, float shared_scale, float routed_scale, float rms_eps,
+                      const void* residual, int64_t ldr, void* out, int64_t ldo, void* workspace,
+                      size_t workspace_bytes, void* stream) {
+    if (n_tokens == 0) return TRMOE_OK;
+    const size_t need = trmoe_dense_layer_workspace_bytes(act_dtype, n_tokens, hidden, shared_width, num_experts,
+                                                          expert_width);
+    TRMOE_REQUIRE(n_tokens > kSkinnyMaxTokens, "dense_layer: more than 128 tokens (else trmoe_dense_decode)");
+    TRMOE_REQUIRE(need > 0 && workspace != nullptr && workspace_bytes >= need && aligned16(workspace),
+                  "dense_layer: a 16-byte aligned workspace of trmoe_dense_layer_workspace_bytes()");
+    TRMOE_REQUIRE(rms_eps >= 0.0f, "dense_layer: rms_eps must be non-negative");
+    const int64_t feats = trmoe_dense_routed_features(shared_width, num_experts, expert_width);
+    float* scales = nullptr;
+    float eps = 0.0f;
+    if (rms_eps > 0.0f) {
+        if (gate_up_rms_inline(act_dtype, n_tokens, 2 * feats)) {
+            eps = rms_eps;
+        } else {
+            scales = reinterpret_cast<float*>(static_cast<char*>(workspace) + need - (size_t)n_tokens * sizeof(float));
+            const int st = trmoe_rms_row_scale(act_dtype, x, n_tokens, hidden, ldx, rms_eps, scales, stream);
+            if (st) return st;
+        }
+    }
+    const int st = dense_routed_gate_up_impl(act_dtype, act_dtype, x, n_tokens, hidden, ldx, w_gate_up, nullptr,
+                                             shared_width, num_experts, expert_width, token_ids, route_table,
+                                             vocab_size, top_k, route_weights, shared_scale, routed_scale, workspace,
+                                             feats, nullptr, 0, stream, scales, eps);
+    if (st) return st;
+    return trmoe_shared_down_combine(act_dtype, act_dtype, workspace, n_tokens, feats, feats, w_down, nullptr, hidden,
+                                     nullptr, hidden, nullptr, top_k, route_weights, 1.0f, 1.0f, residual, ldr, out,
+                                     ldo, nullptr, 0, stream);
+}
+
 // Scratch of trmoe_decoder_step: a hidden buffer, the attention output, then
 // the scratch of the output projection, the attention and the MLP half (used
 // at different times, kept apart).

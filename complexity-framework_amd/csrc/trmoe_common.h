@@ -60,6 +60,28 @@ template <class T> __device__ __forceinline__ T from_f32(float v);
 template <> __device__ __forceinline__ float from_f32<float>(float v) { return v; }
 template <> __device__ __forceinline__ bf16_t from_f32<bf16_t>(float v) { return (bf16_t)v; }
 
+// Sum of squares of the activation elements in one 16-byte chunk.
+__device__ __forceinline__ float chunk_sumsq(KindBF16, u32x4 v) {
+    float s = 0.f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const float lo = __builtin_bit_cast(float, v[j] << 16);
+        const float hi = __builtin_bit_cast(float, v[j] & 0xffff0000u);
+        s += lo * lo;
+        s += hi * hi;
+    }
+    return s;
+}
+__device__ __forceinline__ float chunk_sumsq(KindF32, u32x4 v) {
+    float s = 0.f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const float f = __builtin_bit_cast(float, (uint32_t)v[j]);
+        s += f * f;
+    }
+    return s;
+}
+
 // One 32-byte K group of an MFMA step: every lane supplies the 16-byte chunk
 // at K offset 16*(lane/32) bytes of the group for its row (A) / column (B).
 // Both operands use the same K mapping, so the dot product is exact for any
@@ -509,13 +531,17 @@ __device__ __forceinline__ void tile_loop_dma(const AP& ap, const BP& bp, int K,
 // barrier, LDS read, MFMA): groups run KS such chains side by side.  Group g
 // takes stages g, g + KS, ...; requests past the last stage read zeros, and
 // the final barrier drains them before the caller reuses LDS.
-// `pre` runs while the first stages load (its own loads drain them).
+// `pre` runs while the first stages load (its own loads drain them), `tap`
+// sees each stage's operand rows in LDS.
 struct NoPre {
     __device__ __forceinline__ void operator()() const {}
 };
-template <class Kind, class Shape, class AP, class BP, class Pre>
+struct NoTap {
+    __device__ __forceinline__ void operator()(const char*) const {}
+};
+template <class Kind, class Shape, class AP, class BP, class Pre, class Tap>
 __device__ __forceinline__ void tile_loop_ring(const AP& ap, const BP& bp, int K, char* lds, int wm0, int wn0,
-                                               f32x16 (&acc)[Shape::TM][Shape::TN], const Pre& pre) {
+                                               f32x16 (&acc)[Shape::TM][Shape::TN], const Pre& pre, const Tap& tap) {
     constexpr int S = Shape::kStages, KS = Shape::KS;
     constexpr int kABytes = Shape::BM * kRowBytes;
     constexpr int kPer = AP::kInstr + BP::kInstr;
@@ -542,6 +568,7 @@ __device__ __forceinline__ void tile_loop_ring(const AP& ap, const BP& bp, int K
             mma_stage_f8<Shape::TM, Shape::TN>(st, st + kABytes, wm0, wn0, acc);
         else
             mma_stage<Kind, Shape::TM, Shape::TN>(st, st + kABytes, wm0, wn0, acc);
+        tap(st);   // behind the MFMAs, which run on
         cur = cur + 1 == S ? 0 : cur + 1;
         nxt = nxt + 1 == S ? 0 : nxt + 1;
     }
@@ -583,12 +610,13 @@ __device__ __forceinline__ bool reduce_groups(char* lds, f32x16 (&acc)[Shape::TM
     return g == 0;
 }
 
-template <class Kind, class Shape, class AProv, class BProv, class Pre = NoPre>
+template <class Kind, class Shape, class AProv, class BProv, class Pre = NoPre, class Tap = NoTap>
 __device__ __forceinline__ void tile_loop(const AProv& ap, const BProv& bp, int K, char* lds, int wm0, int wn0,
-                                          f32x16 (&acc)[Shape::TM][Shape::TN], const Pre& pre = Pre{}) {
+                                          f32x16 (&acc)[Shape::TM][Shape::TN], const Pre& pre = Pre{},
+                                          const Tap& tap = Tap{}) {
     if constexpr (!Shape::kRing) pre();
     if constexpr (Shape::kRing)
-        tile_loop_ring<Kind, Shape>(ap, bp, K, lds, wm0, wn0, acc, pre);
+        tile_loop_ring<Kind, Shape>(ap, bp, K, lds, wm0, wn0, acc, pre, tap);
     else if constexpr (Shape::PGR == 4 || Shape::PGR == 6)
         tile_loop_dma<Kind, Shape>(ap, bp, K, lds, wm0, wn0, acc);
     else

@@ -281,6 +281,9 @@ int launch_down_e4m3_decode(const Down8Args& a, float* part, hipStream_t stream)
 int launch_stream_read(const void* src, int64_t bytes, uint32_t* sink, int blocks, hipStream_t stream);
 int launch_down_skinny(int act, int wdt, const DownArgs& a, void* workspace, hipStream_t stream);
 int launch_gate_up(int act, int wdt, const GateUpArgs& a, int64_t packed_rows, hipStream_t stream);
+// Whether launch_gate_up computes RMSNorm scales itself (a.rms_eps) above the
+// decode sizes.
+bool gate_up_rms_inline(int act, int64_t M, int64_t packed_rows);
 // Fragment-major copy of a packed [rows, ld] weight (rows % 16 == 0):
 // block (r / 16, K group g of 64 bytes) is 1 KiB at (r/16 * G + g) * 1024,
 // laid out [16-byte chunk q][row r % 16][16 bytes], zeros past kbytes.

@@ -244,13 +244,36 @@ __global__ __launch_bounds__(Shape::NT) void k_gate_up_swiglu(GateUpArgs a) {
 
     f32x16 acc[Shape::TM][Shape::TN];
     zero_acc<Kind>(acc);
-    tile_loop<Kind, Shape>(ap, bp, a.K, lds, wm0, wn0, acc, row_data);
+    // rms_eps without scales (ring tiles only): the tile streams all K of its
+    // rows through LDS, so it sums their squares on the way, kPer threads a row
+    bool rms_in = false;
+    if constexpr (Shape::kRing && Shape::KS == 1) {
+        constexpr int kPer = Shape::NT / Shape::BM, kC = 8 / kPer;
+        static_assert(kPer >= 1 && 8 % kPer == 0 && kPer <= 4, "threads of a row sit in one wave, whole chunks each");
+        rms_in = a.row_scale == nullptr && a.rms_eps > 0.0f;
+        const int row = (int)threadIdx.x / kPer, part = (int)threadIdx.x % kPer;
+        float ssq = 0.f;
+        tile_loop<Kind, Shape>(ap, bp, a.K, lds, wm0, wn0, acc, row_data, [&](const char* st) {
+            if (!rms_in) return;
+#pragma unroll
+            for (int c = 0; c < kC; ++c)
+                ssq += chunk_sumsq(Kind{}, *reinterpret_cast<const u32x4*>(st + lds_byte(row, part * kC + c)));
+        });
+        if (rms_in) {
+#pragma unroll
+            for (int o = 1; o < kPer; o <<= 1) ssq += __shfl_xor(ssq, o);
+            if (part == 0) s_rscale[row] = rsqrtf(ssq / (float)a.K + a.rms_eps);
+            __syncthreads();
+        }
+    } else {
+        tile_loop<Kind, Shape>(ap, bp, a.K, lds, wm0, wn0, acc, row_data);
+    }
     const bool holder = reduce_groups<Shape>(lds, acc);
     if constexpr (SAVE) {
         if (holder) gate_up_save<Kind, Shape>(a, acc, m0, n0, a.n_base + (int64_t)gridDim.y * Shape::BN);
     }
-    gate_up_epilogue<Kind, Shape, ROUTED>(a, acc, m0, n0, lds, s_route, a.row_scale != nullptr ? s_rscale : nullptr,
-                                          holder);
+    gate_up_epilogue<Kind, Shape, ROUTED>(a, acc, m0, n0, lds, s_route,
+                                          a.row_scale != nullptr || rms_in ? s_rscale : nullptr, holder);
 }
 
 // SwiGLU of one finished tile straight from the accumulators of the calling
@@ -278,22 +301,26 @@ __device__ __forceinline__ void gate_up_epi_direct(const GateUpArgs& a, const f3
     const int col = (int)((pbase >> 1) + r);
     if constexpr (PAIRS) {
         const int lb = pair_lane_offset(wm0, col, ld2);
+        // RS: lane l loads the scale of row wm0 + 32 tm + (l % 32) (clamped
+        // into the tile: rows at or past M are not stored), and element i
+        // takes its row's, acc_row(lane, i), from that lane; all of them
+        // requested before the first is used
+        float rsl[RS ? TMW : 1];
+        if constexpr (RS) {
+#pragma unroll
+            for (int tm = 0; tm < TMW; ++tm) {
+                const int rrow = wm0 + tm * 32 + r;
+                rsl[tm] = a.row_scale[m0 + (rrow < mlim ? rrow : mlim - 1)];
+            }
+        }
 #pragma unroll
         for (int tm = 0; tm < TMW; ++tm) {
-            // RS: lane l loads the scale of row wm0 + 32 tm + (l % 32) (clamped
-            // into the tile: rows at or past M are not stored), and element i
-            // takes its row's, acc_row(lane, i), from that lane
-            float rsl = 1.0f;
-            if constexpr (RS) {
-                const int rrow = wm0 + tm * 32 + r;
-                rsl = a.row_scale[m0 + (rrow < mlim ? rrow : mlim - 1)];
-            }
             float v[16];
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
                 float g = acc[tm][0][i] * sg, u = acc[tm][1][i] * su;
                 if constexpr (RS) {
-                    const float rs = __shfl(rsl, 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3));
+                    const float rs = __shfl(rsl[tm], 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3));
                     g *= rs;
                     u *= rs;
                 }
@@ -1327,6 +1354,15 @@ static int launch_gate_up_ring_shape(const GateUpArgs& a, int64_t rows, hipStrea
     return check_launch(ROUTED ? "dense_routed_gate_up" : "shared_gate_up");
 }
 
+// The shape rule of launch_gate_up_ring (bf16 / f32).
+bool gate_up_rms_inline(int act, int64_t M, int64_t packed_rows) {
+    const int64_t cus = device_cus();
+    if (M <= 0 || packed_rows % 128 != 0) return false;
+    if (act == TRMOE_F32) return tiles_of(M, 256, packed_rows, 256) < kBigTileMinBlocks;
+    return tiles_of(M, 64, packed_rows, 128) <= cus || tiles_of(M, 128, packed_rows, 128) <= cus ||
+           (packed_rows % 256 == 0 && tiles_of(M, 128, packed_rows, 256) <= cus);
+}
+
 // Launches of at most one round of workgroups (shared and expert columns
 // together): the smallest tile whose grid still fits the CUs once, because a
 // workgroup's time is its K stages and does not shrink with fewer of them.
@@ -1624,8 +1660,6 @@ int launch_gate_up(int act, int wdt, const GateUpArgs& a, int64_t packed_rows, h
     }
     if (a.M <= kSkinnyMaxTokens && packed_rows % 64 == 0)
         return launch_gate_up_skinny(act, wdt, a, packed_rows, stream);
-    if (a.row_scale == nullptr && a.rms_eps > 0.0f)
-        return set_error(TRMOE_ERR_INVALID, "gate_up: in-kernel RMSNorm scales need the decode kernels (n <= 128)");
     {
         int st = TRMOE_OK;
         const bool taken =
@@ -1636,6 +1670,8 @@ int launch_gate_up(int act, int wdt, const GateUpArgs& a, int64_t packed_rows, h
                 : false;
         if (taken) return st;
     }
+    if (a.row_scale == nullptr && a.rms_eps > 0.0f)
+        return set_error(TRMOE_ERR_INVALID, "gate_up: in-kernel RMSNorm scales need the decode kernels (n <= 128) or ring tiles");
     if (pp_eligible(act, wdt, a, packed_rows)) {
         if (wdt == TRMOE_FP8_E4M3)
             return a.ids != nullptr ? launch_gate_up_pp<true, false, true>(a, packed_rows, stream)

@@ -69,28 +69,6 @@ struct WFrag<Kind, true> {
 // FRAG (with SW off): the descriptor is a fragment-major copy whose block 0
 // is row 0, and weight fragments are 1 KiB contiguous loads.  Spans [s0, s1) in batches of SB;
 // `region` holds SB * (MT + (SW ? NU : 0)) * 16 rows of 128 bytes.
-// Sum of squares of the activation elements in one 16-byte chunk.
-__device__ __forceinline__ float chunk_sumsq(KindBF16, u32x4 v) {
-    float s = 0.f;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const float lo = __builtin_bit_cast(float, v[j] << 16);
-        const float hi = __builtin_bit_cast(float, v[j] & 0xffff0000u);
-        s += lo * lo;
-        s += hi * hi;
-    }
-    return s;
-}
-__device__ __forceinline__ float chunk_sumsq(KindF32, u32x4 v) {
-    float s = 0.f;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const float f = __builtin_bit_cast(float, (uint32_t)v[j]);
-        s += f * f;
-    }
-    return s;
-}
-
 template <int MT>
 constexpr int ssq_rows() { return (MT * 16 + 63) / 64; }
 

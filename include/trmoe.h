@@ -528,6 +528,22 @@ int trmoe_dense_decode(int act_dtype, const void* x, int64_t n_tokens, int64_t h
                        void* workspace, size_t workspace_bytes, void* stream);
 
 /*
+ * A dense-routed layer on more than 128 tokens in one call (bf16 / f32): the
+ * fused RMSNorm's scales (rms_eps > 0, packs with its weight folded in), the
+ * gate|up and the down of trmoe_dense_routed_gate_up and
+ * trmoe_shared_down_combine.  Up to about one round of workgroups the gate|up
+ * sums the squares of its own rows, without a launch for the scales.
+ */
+size_t trmoe_dense_layer_workspace_bytes(int act_dtype, int64_t n_tokens, int64_t hidden, int64_t shared_width,
+                                         int num_experts, int64_t expert_width);
+int trmoe_dense_layer(int act_dtype, const void* x, int64_t n_tokens, int64_t hidden, int64_t ldx,
+                      const void* w_gate_up, const void* w_down, int64_t shared_width, int num_experts,
+                      int64_t expert_width, const int64_t* token_ids, const int64_t* route_table, int64_t vocab_size,
+                      int top_k, const float* route_weights, float shared_scale, float routed_scale, float rms_eps,
+                      const void* residual, int64_t ldr, void* out, int64_t ldo, void* workspace,
+                      size_t workspace_bytes, void* stream);
+
+/*
  * One decode step of a whole decoder (bf16, dense-routed layers, batch <= 16):
  * for every layer trmoe_decode_attention, the output projection with its
  * residual, and the MLP half with its RMSNorm and residual, queued by one call
