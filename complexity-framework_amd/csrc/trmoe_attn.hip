@@ -386,19 +386,22 @@ __global__ __launch_bounds__(64 * kAttnWaves) void k_decode_attn(DecodeAttnArgs 
 // the scores' accumulator layout is the second product's operand as it stands
 // (K order: positions 16 t + 4 h + 0..3 and + 8, which the transposing V reads
 // follow).  The vector ALU bounds it (32 exponentials and about as much again
-// per 512 clocks of MFMA); two or three workgroups per CU overlap one's softmax
-// with another's products.  8 x 2048 tokens, 14 heads on 2: 174 us in the
-// library's flash kernel before.
-constexpr int kQTile = 128, kKTile = 64, kAttnStages = 3;
+// per 512 clocks of MFMA); three workgroups per CU overlap one's softmax
+// with another's products.  8 x 2048 tokens, 14 heads on 2: 92 us (174 us in
+// the library's flash kernel).  What it took from 132: the longest rows first
+// (25 us of a last wave that was nearly empty), masks on the diagonal tiles
+// alone and the rescaling only where the maximum moved (6), constant offsets in
+// the LDS reads (3) and two stages instead of three (6).
+constexpr int kQTile = 128, kKTile = 64, kAttnStages = 2;
 constexpr int kAttnStage = 2 * kKTile * kRowBytes;
 __global__ __launch_bounds__(256, 2) void k_prefill_attn(PrefillAttnArgs a) {
     __shared__ __align__(16) char lds[kAttnStages * kAttnStage];
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     const int r = lane & 31, h = lane >> 5;
-    // workgroups go to the XCDs in turn along x: every second head walks its
-    // query tiles the other way, so that each XCD gets long and short rows
-    const int qt = (blockIdx.y & 1) ? (int)blockIdx.x : (int)(gridDim.x - 1 - blockIdx.x);
-    const int b = (int)blockIdx.y / a.heads, head = (int)blockIdx.y % a.heads;
+    // the heads along x, the query tiles from the longest row to the shortest
+    // along y: the short ones fill the gaps that the long ones leave
+    const int qt = (int)(gridDim.y - 1 - blockIdx.y);
+    const int b = (int)blockIdx.x / a.heads, head = (int)blockIdx.x % a.heads;
     const int kvh = head / (a.heads / a.kvh);
     const int T = (int)a.T;
     const int q0 = qt * kQTile, qw = q0 + 32 * wave;
@@ -409,7 +412,7 @@ __global__ __launch_bounds__(256, 2) void k_prefill_attn(PrefillAttnArgs a) {
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
         const int row = (wave * 2 + j) * 8 + (lane >> 3);
-        off[j] = row * kRowBytes + 16 * ((lane & 7) ^ lds_swz(row));
+        off[j] = row * kRowBytes + 16 * ((lane & 7) ^ (row & 7));
     }
     auto issue = [&](int tile, char* st) {
 #pragma unroll
@@ -435,28 +438,41 @@ __global__ __launch_bounds__(256, 2) void k_prefill_attn(PrefillAttnArgs a) {
     float m = -__builtin_inff(), l = 0.f;
     const float c = a.scale * 1.4426950408889634f;   // exp2
     // transposing V reads: 16 lanes cover 4 positions x 16 columns
-    const int vrow = (lane & 15) >> 2, vchunk = 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1), vbyte = 8 * (lane & 1);
+    const int vrow = 4 * h + ((lane & 15) >> 2), vchunk = 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1);
+    // 16-byte chunks are swizzled by the row's low three bits alone, which rows
+    // 8 apart share: every read of a tile is one of six addresses plus a constant
+    int koff[4], voff[2];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) koff[g] = r * kRowBytes + (((2 * g + h) ^ (r & 7)) << 4);
+#pragma unroll
+    for (int d = 0; d < 2; ++d)
+        voff[d] = (kKTile + vrow) * kRowBytes + (((4 * d + vchunk) ^ vrow) << 4) + 8 * (lane & 1);
+    f32x16 zero;   // the first product's C operand, instead of clearing 32 accumulators a tile
+#pragma unroll
+    for (int i = 0; i < 16; ++i) zero[i] = 0.f;
     int cur = 0, nxt = kAttnStages - 1;
-    for (int kt = 0; kt < nt; ++kt) {
+    // one K/V tile; DIAG: positions ahead of the query are masked (only the
+    // tiles that reach the wave's first query hold any)
+    auto step = [&](int kt, auto diag) {
         wait_vmcnt<4 * (kAttnStages - 2)>();   // this wave's loads of tile kt have landed
         wait_lgkmcnt0();                       // and its reads of tile kt - 1 are complete
         lds_barrier();                         // ... and every other wave's
         const char* ks = lds + cur * kAttnStage;
-        const char* vs = ks + kKTile * kRowBytes;
         issue(kt + kAttnStages - 1, lds + nxt * kAttnStage);
         cur = cur + 1 == kAttnStages ? 0 : cur + 1;
         nxt = nxt + 1 == kAttnStages ? 0 : nxt + 1;
-        if (kt * kKTile > qw + 31) continue;   // wholly ahead of the wave's queries
+        if (kt * kKTile > qw + 31) return;   // wholly ahead of the wave's queries
         f32x16 s[2];
 #pragma unroll
-        for (int n = 0; n < 2; ++n) {
+        for (int n = 0; n < 2; ++n)
 #pragma unroll
-            for (int i = 0; i < 16; ++i) s[n][i] = 0.f;
-#pragma unroll
-            for (int g = 0; g < 4; ++g)
-                mfma_group(KindBF16{}, *reinterpret_cast<const u32x4*>(ks + lds_byte(32 * n + r, 2 * g + h)), qf[g], s[n]);
-        }
-        if (kt * kKTile + kKTile - 1 > qw) {   // the diagonal
+            for (int g = 0; g < 4; ++g) {
+                const u32x4 kf = *reinterpret_cast<const u32x4*>(ks + koff[g] + 32 * n * kRowBytes);
+                s[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, kf),
+                                                               __builtin_bit_cast(bf16x8, (u32x4)qf[g]),
+                                                               g == 0 ? zero : s[n], 0, 0, 0);
+            }
+        if constexpr (decltype(diag)::value) {
             const int ahead = qw + r - kt * kKTile;
 #pragma unroll
             for (int n = 0; n < 2; ++n)
@@ -470,9 +486,18 @@ __global__ __launch_bounds__(256, 2) void k_prefill_attn(PrefillAttnArgs a) {
 #pragma unroll
             for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[n][i]);
         mx = fmaxf(mx, __shfl_xor(mx, 32));
-        const float alpha = __builtin_amdgcn_exp2f((m - mx) * c), mc = mx * c;
-        m = mx;
-        float sum = 0.f;
+        // the reference point moves only when the maximum has grown by 2^8: the
+        // weights stay below that in fp32, and the sums need no rescaling
+        if (__builtin_amdgcn_ballot_w64((mx - m) * c > 8.0f) != 0) {
+            const float alpha = __builtin_amdgcn_exp2f((m - mx) * c);
+            m = mx;
+            l *= alpha;
+#pragma unroll
+            for (int d = 0; d < 2; ++d)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) o[d][i] *= alpha;
+        }
+        const float mc = m * c;
         u32x4 p[4];
 #pragma unroll
         for (int n = 0; n < 2; ++n)
@@ -482,30 +507,26 @@ __global__ __launch_bounds__(256, 2) void k_prefill_attn(PrefillAttnArgs a) {
 #pragma unroll
                 for (int i = 0; i < 8; ++i) {
                     e[i] = __builtin_amdgcn_exp2f(s[n][8 * t + i] * c - mc);
-                    sum += e[i];
+                    l += e[i];
                 }
                 p[2 * n + t] = pack8(e);
             }
-        l = l * alpha + sum;
-        if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
-#pragma unroll
-            for (int d = 0; d < 2; ++d)
-#pragma unroll
-                for (int i = 0; i < 16; ++i) o[d][i] *= alpha;
-        }
 #pragma unroll
         for (int t = 0; t < 4; ++t)
 #pragma unroll
             for (int d = 0; d < 2; ++d) {
                 u32x2 v[2];
 #pragma unroll
-                for (int e = 0; e < 2; ++e) {
-                    const int row = 16 * t + 8 * e + 4 * h + vrow;
-                    v[e] = ds_read_tr16(vs + row * kRowBytes + (((4 * d + vchunk) ^ lds_swz(row)) << 4) + vbyte);
-                }
+                for (int e = 0; e < 2; ++e) v[e] = ds_read_tr16(ks + voff[d] + (16 * t + 8 * e) * kRowBytes);
                 mfma_group(KindBF16{}, u32x4{v[0][0], v[0][1], v[1][0], v[1][1]}, p[t], o[d]);
             }
-    }
+    };
+    // tiles wholly at or before the workgroup's first query (uniform: the
+    // waves share the barriers), then the diagonal ones
+    const int full = std::min(nt, (q0 + 1) / kKTile);
+    int kt = 0;
+    for (; kt < full; ++kt) step(kt, std::false_type{});
+    for (; kt < nt; ++kt) step(kt, std::true_type{});
     wait_vmcnt<0>();   // nothing writes this LDS once the workgroup has left
     if (qw + r >= T) return;
     const float inv = 1.0f / (l + __shfl_xor(l, 32));
@@ -525,7 +546,7 @@ __global__ __launch_bounds__(256, 2) void k_prefill_attn(PrefillAttnArgs a) {
 }  // namespace
 
 int launch_prefill_attn(const PrefillAttnArgs& a, int64_t sequences, hipStream_t stream) {
-    const dim3 grid((unsigned)((a.T + kQTile - 1) / kQTile), (unsigned)(sequences * a.heads));
+    const dim3 grid((unsigned)(sequences * a.heads), (unsigned)((a.T + kQTile - 1) / kQTile));
     hipLaunchKernelGGL(k_prefill_attn, grid, dim3(256), 0, stream, a);
     return check_launch("prefill_attention");
 }

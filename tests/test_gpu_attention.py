@@ -105,6 +105,27 @@ def test_prefill_attention(gpu, B, T, heads, kvh):
     assert _rel(got.view(B, T, heads, D), want) <= 2.0 ** -7
 
 
+@pytest.mark.parametrize("rise", [0.01, 0.05, 0.5, -0.5])
+def test_prefill_attention_moving_maximum(gpu, rise):
+    # scores that climb (or fall) with the position by `rise` a step: the
+    # reference point of the exponentials stays for a while, moves at every
+    # tile, or never again
+    T, L = 700, 768
+    q = torch.zeros(1, T, 2, D, device=gpu).bfloat16()
+    q[..., 0], q[..., 1] = 8.0, 8.0
+    kc = torch.zeros(1, 1, L, D, device=gpu).bfloat16()
+    ramp = rise * torch.arange(L, device=gpu)
+    kc[..., 0] = ramp.bfloat16()
+    kc[..., 1] = (ramp - ramp.bfloat16().float()).bfloat16()   # the ramp to 16 bits
+    vc = torch.randn(1, 1, L, D, generator=torch.Generator().manual_seed(1)).to(gpu).bfloat16()
+    got = ops.prefill_attention(q, kc, vc, 0.125)
+    k, v = (c[:, :, :T].float().expand(1, 2, T, D) for c in (kc, vc))
+    s = (q.float().transpose(1, 2) @ k.transpose(2, 3)) * 0.125
+    s.masked_fill_(torch.ones(T, T, dtype=torch.bool, device=gpu).triu(1), -math.inf)
+    want = (torch.softmax(s, -1) @ v).transpose(1, 2)
+    assert _rel(got.view(1, T, 2, D), want) <= 2.0 ** -7
+
+
 def test_decode_linear_adds_residual(gpu):
     g = torch.Generator().manual_seed(0)
     for n in (1, 8, 9, 16):
