@@ -248,6 +248,12 @@ __device__ __forceinline__ void mma_stage_tr(const char* As, const char* Bs, int
 // ---------------------------------------------------------------------------
 using ShapeBwdGU = TileShape<256, 256, 2, 4, 4>;   // packed gate|up columns of 128 features
 using ShapeBwdDH = TileShape<256, 128, 2, 4, 4>;   // the same 128 features of dh
+// The grouped bf16 rows: a segment per expert leaves few large tiles (16
+// experts of 375 rows: 40 row tiles of 256), so 128 rows x 64 features on rings of
+// four LDS stages (that case, hidden 2048, 256 features: 80 -> 252 workgroups,
+// 127 -> 52 us).
+using ShapeBwdGroupGU = RingGateUp128<false>;
+using ShapeBwdGroupDH = TileShape<128, 64, 4, 2, 4, 4>;
 
 // Epilogue of the saved-g|u bf16 SwiGLU backward without LDS: lanes pair up
 // (DPP swap of one dh value, as in store_bf16_pairs) so that each lane owns
@@ -344,11 +350,10 @@ __device__ __forceinline__ void swiglu_bwd_pairs(const SwigluBwdArgs& a, const f
 
 // SAVED: g|u come from a.gu (written by the forward) instead of a
 // recomputing tile loop.
-template <class Kind, bool GROUPED, bool ROUTED, bool SAVED = false>
-__global__ __launch_bounds__(512) void k_swiglu_bwd(SwigluBwdArgs a) {
+template <class Kind, bool GROUPED, bool ROUTED, bool SAVED, class SG, class SD>
+__global__ __launch_bounds__(SG::NT) void k_swiglu_bwd(SwigluBwdArgs a) {
     using T = typename Kind::T;
-    using SG = ShapeBwdGU;
-    using SD = ShapeBwdDH;
+    static_assert(!SAVED || SG::BN == 256, "the saved g|u is staged for 128 features");
     static_assert(SG::BM == SD::BM && SG::WAVES_M == SD::WAVES_M && SG::WAVES_N == SD::WAVES_N &&
                       SG::WN == 2 * SD::WN && SD::TN == 1 && SG::TN == 2,
                   "a wave holds gate, up and dh of the same 32 features");
@@ -365,6 +370,7 @@ __global__ __launch_bounds__(512) void k_swiglu_bwd(SwigluBwdArgs a) {
     const char* wdt = static_cast<const char*>(a.wdt);
 
     typename AProvOf<SG>::type ax, ad;
+    __shared__ float s_mult[GROUPED ? SG::BM : 1];
     if constexpr (GROUPED) {
         __shared__ int s_tile[3];
         grouped_tile<SG::BM>(a.offsets, a.E, (int)blockIdx.x, s_tile);
@@ -372,6 +378,11 @@ __global__ __launch_bounds__(512) void k_swiglu_bwd(SwigluBwdArgs a) {
         const int64_t e = s_tile[0];
         m0 = s_tile[1];
         m_end = s_tile[2];
+        if (threadIdx.x < SG::BM) {   // the rows' route weights; read after the tile loops' barriers
+            const int64_t row = m0 + threadIdx.x;
+            const int64_t slot = row < m_end ? (int64_t)((uint64_t)a.gather[row] / (uint64_t)a.gather_mod) : 0;
+            s_mult[threadIdx.x] = a.rw[slot < kMaxTopK ? slot : kMaxTopK - 1];
+        }
         wgu += e * a.wgu_expert_stride * kElem;
         wdt += e * a.wdt_expert_stride * kElem;
         init_gather_rows(ax, a.x, a.gather, a.gather_mod, m0, m_end - m0, a.ldx * kElem, a.K * (int)kElem);
@@ -476,12 +487,7 @@ __global__ __launch_bounds__(512) void k_swiglu_bwd(SwigluBwdArgs a) {
                     mult = tw;
                 }
             }
-            if constexpr (GROUPED) {
-                if (valid) {
-                    const int64_t slot = (int64_t)((uint64_t)a.gather[row] / (uint64_t)a.gather_mod);
-                    mult = a.rw[slot < kMaxTopK ? slot : kMaxTopK - 1];
-                }
-            }
+            if constexpr (GROUPED) mult = s_mult[rl];
             const float e = __builtin_amdgcn_exp2f(-g * 1.4426950408889634f);
             const float s = __builtin_amdgcn_rcpf(1.0f + e);   // sigmoid(g)
             const float sl = silu_f(g);
@@ -505,11 +511,11 @@ __global__ __launch_bounds__(512) void k_swiglu_bwd(SwigluBwdArgs a) {
         }
     }
     if constexpr (kLdsOut) {
-        // copy the dg|du tile out: 256 rows x 4 stages x 8 chunks of 16 bytes
+        // copy the dg|du tile out, 64-column stages of 8 chunks of 16 bytes
         wait_lgkmcnt0();
         __syncthreads();
-        const int64_t cols = 2 * (a.F - f0) < 256 ? 2 * (a.F - f0) : 256;
-        for (int q = threadIdx.x; q < SG::BM * 32; q += SG::NT) {
+        const int64_t cols = 2 * (a.F - f0) < SG::BN ? 2 * (a.F - f0) : SG::BN;
+        for (int q = threadIdx.x; q < SG::BM * (SG::BN / 8); q += SG::NT) {
             const int kt = q / (SG::BM * 8), r = (q / 8) % SG::BM, c = q % 8;
             const int col = kt * 64 + c * 8;
             if (m0 + r < m_end && col < cols)
@@ -892,17 +898,16 @@ static int bwd_lds(F* fn, int bytes) {
     return set_kernel_lds(reinterpret_cast<const void*>(fn), bytes);
 }
 
-template <class Kind, bool GROUPED, bool ROUTED, bool SAVED = false>
+template <class Kind, bool GROUPED, bool ROUTED, bool SAVED = false, class SG = ShapeBwdGU, class SD = ShapeBwdDH>
 static int swiglu_bwd_kind(const SwigluBwdArgs& a, int64_t assignments, hipStream_t stream) {
-    auto kern = k_swiglu_bwd<Kind, GROUPED, ROUTED, SAVED>;
-    constexpr int kLds = ShapeBwdGU::kLdsBytes;
+    auto kern = k_swiglu_bwd<Kind, GROUPED, ROUTED, SAVED, SG, SD>;
+    constexpr int kLds = SG::kLdsBytes > SD::kLdsBytes ? SG::kLdsBytes : SD::kLdsBytes;
     int st = bwd_lds(kern, kLds);
     if (st) return st;
-    const int64_t tiles_m =
-        GROUPED ? (assignments + ShapeBwdGU::BM - 1) / ShapeBwdGU::BM + a.E : (a.M + ShapeBwdGU::BM - 1) / ShapeBwdGU::BM;
-    const int64_t tiles_f = (a.F - a.f_base + ShapeBwdDH::BN - 1) / ShapeBwdDH::BN;
+    const int64_t tiles_m = GROUPED ? (assignments + SG::BM - 1) / SG::BM + a.E : (a.M + SG::BM - 1) / SG::BM;
+    const int64_t tiles_f = (a.F - a.f_base + SD::BN - 1) / SD::BN;
     if (tiles_m <= 0 || tiles_f <= 0) return TRMOE_OK;
-    hipLaunchKernelGGL(kern, dim3((unsigned)tiles_m, (unsigned)tiles_f), dim3(512), kLds, stream, a);
+    hipLaunchKernelGGL(kern, dim3((unsigned)tiles_m, (unsigned)tiles_f), dim3(SG::NT), kLds, stream, a);
     return check_launch("swiglu_backward");
 }
 
@@ -948,7 +953,8 @@ int launch_swiglu_bwd(int act, const SwigluBwdArgs& a, int64_t assignments, hipS
                       : swiglu_bwd_kind<KindF32, false, false, true>(a, assignments, stream);
     }
     if (act == TRMOE_BF16) {
-        if (grouped) return swiglu_bwd_kind<KindBF16, true, false>(a, assignments, stream);
+        if (grouped)
+            return swiglu_bwd_kind<KindBF16, true, false, false, ShapeBwdGroupGU, ShapeBwdGroupDH>(a, assignments, stream);
         if (routed) return swiglu_bwd_kind<KindBF16, false, true>(a, assignments, stream);
         return swiglu_bwd_kind<KindBF16, false, false>(a, assignments, stream);
     }

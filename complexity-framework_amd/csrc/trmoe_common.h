@@ -572,6 +572,7 @@ __device__ __forceinline__ void tile_loop_ring(const AP& ap, const BP& bp, int K
         cur = cur + 1 == S ? 0 : cur + 1;
         nxt = nxt + 1 == S ? 0 : nxt + 1;
     }
+    wait_vmcnt<0>();   // the loads past the last stage, which the caller's use of the LDS must not meet
     __syncthreads();
 }
 
