@@ -26,6 +26,11 @@ ORDER_ASSIGNMENT = N.ORDER_ASSIGNMENT
 # Padding the packed layouts use (must match the kernel tiles).
 SHARED_GATE_UP_ALIGN = 256   # rows = 2 * round_up(S, 128)
 SKINNY_MAX_TOKENS = 128      # token counts the decode-shape kernels take
+# bf16 layers above this many tokens run on tiles, as prompts do: the decode-shape
+# kernels keep a wave's activations in registers, and at 65..128 tokens there is
+# room for half the waves only (16 layers of the 200M model in one graph: 65
+# tokens 414 -> 358 us, 102 448 -> 372, 128 466 -> 400)
+DECODE_BF16_TOKENS = 64
 EXPERT_GATE_UP_ALIGN = 128   # rows = 2 * round_up(W, 64)
 DOWN_ALIGN = 256             # rows = round_up(H, 256)
 
@@ -897,7 +902,7 @@ def dense_decode(x: torch.Tensor, token_ids: torch.Tensor, route_table: torch.Te
 def dense_layer(x: torch.Tensor, token_ids: torch.Tensor, route_table: torch.Tensor, packed: "PackedLayer",
                 route_weights: Sequence[float], shared_scale: float, routed_scale: float,
                 residual: Optional[torch.Tensor] = None, rms_eps: float = 0.0) -> torch.Tensor:
-    """A dense-routed layer on more than SKINNY_MAX_TOKENS tokens (trmoe_dense_layer)."""
+    """A dense-routed layer on more than 64 tokens (trmoe_dense_layer)."""
     lib = _lib()
     _require_cuda(x, token_ids, route_table, residual)
     n, hidden = x.shape
@@ -1067,9 +1072,12 @@ def layer_forward(x: torch.Tensor, token_ids: torch.Tensor, route_table: torch.T
     rscale, eps_in = None, 0.0
     if norm_eps is not None and save:
         raise ValueError("layer_forward: the fused RMSNorm is inference-only")
-    if norm_eps is not None and norm_eps > 0 and packed.strategy == STRATEGY_DENSE and n > SKINNY_MAX_TOKENS:
+    if packed.strategy == STRATEGY_DENSE and not save and (
+            norm_eps is not None and norm_eps > 0 and n > SKINNY_MAX_TOKENS
+            or x.dtype == torch.bfloat16 and DECODE_BF16_TOKENS < n <= SKINNY_MAX_TOKENS
+            and (norm_eps is None or norm_eps > 0)):
         return dense_layer(x, token_ids, route_table, packed, route_weights, shared_scale, routed_scale, residual,
-                           float(norm_eps))
+                           float(norm_eps or 0.0))
     if norm_eps is not None:
         if packed.strategy == STRATEGY_DENSE and n <= SKINNY_MAX_TOKENS:
             eps_in = float(norm_eps)

@@ -476,7 +476,7 @@ static int dense_routed_gate_up_impl(int act_dtype, int w_dtype, const void* x, 
                                      const float* route_weights, float shared_scale, float routed_scale, void* h,
                                      int64_t ldh, void* gu, int64_t ldgu, void* stream,
                                      const float* row_scale = nullptr, float rms_eps = 0.0f,
-                                     const void* w_frag = nullptr) {
+                                     const void* w_frag = nullptr, bool on_tiles = false) {
     TRMOE_REQUIRE(valid_pair(act_dtype, w_dtype), "dense_routed_gate_up: unsupported dtype pair");
     TRMOE_REQUIRE(n_tokens >= 0 && hidden > 0 && shared_width >= 0 && expert_width > 0,
                   "dense_routed_gate_up: bad dimensions");
@@ -517,6 +517,7 @@ static int dense_routed_gate_up_impl(int act_dtype, int w_dtype, const void* x, 
     a.gu = gu;
     a.ldgu = ldgu;
     a.row_scale = row_scale;
+    a.on_tiles = on_tiles;
     a.rms_eps = rms_eps;
     a.w_frag = w_frag;
     return launch_gate_up(act_dtype, w_dtype, a, 2 * feats, as_stream(stream));
@@ -1189,7 +1190,7 @@ int trmoe_dense_layer(int act_dtype, const void* x, int64_t n_tokens, int64_t hi
     if (n_tokens == 0) return TRMOE_OK;
     const size_t need = trmoe_dense_layer_workspace_bytes(act_dtype, n_tokens, hidden, shared_width, num_experts,
                                                           expert_width);
-    TRMOE_REQUIRE(n_tokens > kSkinnyMaxTokens, "dense_layer: more than 128 tokens (else trmoe_dense_decode)");
+    TRMOE_REQUIRE(n_tokens > 64, "dense_layer: more than 64 tokens (else trmoe_dense_decode)");
     TRMOE_REQUIRE(need > 0 && workspace != nullptr && workspace_bytes >= need && aligned16(workspace),
                   "dense_layer: a 16-byte aligned workspace of trmoe_dense_layer_workspace_bytes()");
     TRMOE_REQUIRE(rms_eps >= 0.0f, "dense_layer: rms_eps must be non-negative");
@@ -1208,7 +1209,7 @@ int trmoe_dense_layer(int act_dtype, const void* x, int64_t n_tokens, int64_t hi
     const int st = dense_routed_gate_up_impl(act_dtype, act_dtype, x, n_tokens, hidden, ldx, w_gate_up, nullptr,
                                              shared_width, num_experts, expert_width, token_ids, route_table,
                                              vocab_size, top_k, route_weights, shared_scale, routed_scale, workspace,
-                                             feats, nullptr, 0, stream, scales, eps);
+                                             feats, nullptr, 0, stream, scales, eps, nullptr, true);
     if (st) return st;
     return trmoe_shared_down_combine(act_dtype, act_dtype, workspace, n_tokens, feats, feats, w_down, nullptr, hidden,
                                      nullptr, hidden, nullptr, top_k, route_weights, 1.0f, 1.0f, residual, ldr, out,

@@ -58,6 +58,7 @@ struct GateUpArgs {
     // kernels compute 1 / sqrt(mean(x_t^2) + rms_eps) themselves.
     const float* row_scale;
     float rms_eps;
+    bool on_tiles;   // keep decode-sized launches (at most kSkinnyMaxTokens) off the decode kernels
     // Fragment-major copy of w (trmoe_pack_fragments) for the decode kernels,
     // or null: bf16/f32 weights, K groups of 64 bytes per 16-row block.
     const void* w_frag;

@@ -193,6 +193,26 @@ __device__ __forceinline__ void gate_up_save(const GateUpArgs& a, const f32x16 (
 // per-token expert weights compiled in); the shared-feature launches leave
 // that code out.  SAVE: also write the raw gate|up outputs to a.gu (training
 // forwards), passed the launch's packed row count as gridDim-independent bound.
+// Tile of a ring launch of at most about one round, grid (row tiles, column
+// tiles).  Workgroups go to the 8 XCDs round-robin; XCD x takes a run of
+// consecutive tiles, down the columns of the longer side's split, so that its
+// L2 fetches one eighth of the larger operand and the whole of the smaller
+// instead of nearly all of both.  Down of 1906 tokens (15 x 14
+// tiles, K = 3328) 26.4 -> 22.4 us in the layer; 1800 tokens' layer 65.0 -> 60.7.
+template <class Shape>
+__device__ __forceinline__ void ring_tile(uint32_t& mt, uint32_t& nt) {
+    const uint32_t gm = gridDim.x, gn = gridDim.y, total = gm * gn;
+    const uint32_t id = blockIdx.x + blockIdx.y * gm, x = id & 7, rem = total & 7;
+    const uint32_t t = x * (total >> 3) + (x < rem ? x : rem) + (id >> 3);
+    if (gm * Shape::BM >= gn * Shape::BN) {
+        mt = t / gn;
+        nt = t - mt * gn;
+    } else {
+        nt = t / gm;
+        mt = t - nt * gm;
+    }
+}
+
 template <class Kind, bool FP8, class Shape, bool GROUPED = false, bool ROUTED = false, bool SAVE = false>
 __global__ __launch_bounds__(Shape::NT) void k_gate_up_swiglu(GateUpArgs a) {
     using T = typename Kind::T;
@@ -200,8 +220,10 @@ __global__ __launch_bounds__(Shape::NT) void k_gate_up_swiglu(GateUpArgs a) {
     const int wave = (threadIdx.x >> 6) % (Shape::NTG / 64);
     const int wm0 = (wave / Shape::WAVES_N) * Shape::WM;
     const int wn0 = (wave % Shape::WAVES_N) * Shape::WN;
-    int64_t m0 = (int64_t)blockIdx.x * Shape::BM;
-    const int64_t n0 = a.n_base + (int64_t)blockIdx.y * Shape::BN;
+    uint32_t mt = blockIdx.x, nt = blockIdx.y;
+    if constexpr (Shape::kRing && !GROUPED) ring_tile<Shape>(mt, nt);
+    int64_t m0 = (int64_t)mt * Shape::BM;
+    const int64_t n0 = a.n_base + (int64_t)nt * Shape::BN;
 
     typename AProvOf<Shape>::type ap;
     if constexpr (GROUPED) {
@@ -636,8 +658,10 @@ __global__ __launch_bounds__(Shape::NT) void k_down_combine(DownArgs a) {
     const int wave = (threadIdx.x >> 6) % (Shape::NTG / 64), lane = threadIdx.x & 63;
     const int wm0 = (wave / Shape::WAVES_N) * Shape::WM;
     const int wn0 = (wave % Shape::WAVES_N) * Shape::WN;
-    int64_t m0 = (int64_t)blockIdx.x * Shape::BM;
-    const int64_t n0 = (int64_t)blockIdx.y * Shape::BN;
+    uint32_t mt = blockIdx.x, nt = blockIdx.y;
+    if constexpr (Shape::kRing && !GROUPED) ring_tile<Shape>(mt, nt);
+    int64_t m0 = (int64_t)mt * Shape::BM;
+    const int64_t n0 = (int64_t)nt * Shape::BN;
 
     if constexpr (GROUPED) {
         __shared__ int s_tile[3];
@@ -684,8 +708,13 @@ __global__ __launch_bounds__(Shape::NT) void k_down_combine(DownArgs a) {
     if constexpr (sizeof(T) == 2) {
         // bf16: the scaled shared term goes to LDS as a [BM][BN] tile (rows
         // padded by 16 bytes); the routed gather, residual and store then run
-        // over 16-byte chunks of 8 columns.
-        constexpr int kORowBytes = Shape::BN * 2 + 16;
+        // over 16-byte chunks of 8 columns.  The narrow ring tiles, which also run
+        // decode-sized launches, keep the term in fp32 until it is whole, as the
+        // decode kernels do.
+        constexpr bool kWide = Shape::kRing && Shape::BN <= 64;
+        using ST = std::conditional_t<kWide, float, T>;
+        constexpr int kORowBytes = Shape::BN * (int)sizeof(ST) + 16;
+        static_assert(!kWide || Shape::BM * kORowBytes <= Shape::kLdsBytes, "the fp32 tile fits the stages' LDS");
         if (holder) {
 #pragma unroll
             for (int tm = 0; tm < Shape::TM; ++tm)
@@ -694,8 +723,8 @@ __global__ __launch_bounds__(Shape::NT) void k_down_combine(DownArgs a) {
                     const int rl = wm0 + tm * 32 + acc_row(lane, i);
 #pragma unroll
                     for (int tn = 0; tn < Shape::TN; ++tn)
-                        *reinterpret_cast<T*>(lds + rl * kORowBytes + (wn0 + tn * 32 + r) * 2) =
-                            from_f32<T>(acc[tm][tn][i] * cscale[tn]);
+                        *reinterpret_cast<ST*>(lds + rl * kORowBytes + (wn0 + tn * 32 + r) * (int)sizeof(ST)) =
+                            from_f32<ST>(acc[tm][tn][i] * cscale[tn]);
                 }
         }
         __syncthreads();
@@ -705,11 +734,17 @@ __global__ __launch_bounds__(Shape::NT) void k_down_combine(DownArgs a) {
             const int64_t row = m0 + rl;
             const int64_t col = n0 + c * 8;
             if (row >= a.M || col >= a.N) continue;
-            const u32x4 sv = *reinterpret_cast<const u32x4*>(lds + rl * kORowBytes + c * 16);
-            const bf16x8 sb = __builtin_bit_cast(bf16x8, sv);
             float v[8];
+            const char* sp = lds + rl * kORowBytes + c * 8 * (int)sizeof(ST);
+            if constexpr (kWide) {
+                const f32x4 s0 = *reinterpret_cast<const f32x4*>(sp), s1 = *reinterpret_cast<const f32x4*>(sp + 16);
 #pragma unroll
-            for (int e = 0; e < 8; ++e) v[e] = (float)sb[e];
+                for (int e = 0; e < 8; ++e) v[e] = e < 4 ? s0[e & 3] : s1[e & 3];
+            } else {
+                const bf16x8 sb = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(sp));
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[e] = (float)sb[e];
+            }
             if (a.vec_ok && col + 8 <= a.N) {
                 if (y != nullptr) {
                     float acc_r[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -1371,7 +1406,8 @@ bool gate_up_rms_inline(int act, int64_t M, int64_t packed_rows) {
 // were a second launch, 11.8 more), 1024 21.4 -> 19.9; with e4m3 weights at
 // hidden 2048, 11264 rows: 130 tokens 25.6 -> 20.6, 512 39.2 -> 31.4.  At the
 // next size up the 256-row ping-pong tiles are as fast (777 tokens of that
-// layer: 46.9 against 60.4 on 128x256).  f32 takes 64x128 throughout: its
+// layer: 46.9 against 60.4 on 128x256).  128 tokens of the 200M layer on 64x64
+// tiles of two K groups: 9.3 -> 6.9.  f32 takes 64x128 throughout: its
 // MFMAs bound the stage (2048 tokens 252 -> 216 with the merged launch).
 // Returns whether it took the launch.
 template <class Kind, bool FP8, bool SAVE>
@@ -1390,6 +1426,13 @@ static bool launch_gate_up_ring(const GateUpArgs& a, int64_t packed_rows, hipStr
         st = run(RingGateUp64<false>{});
         return true;
     } else {
+        if constexpr (!FP8) {
+            // its groups of waves each see half of K, so none has a row's squares
+            if (tiles_of(a.M, 64, rows, 64) <= cus && !(a.row_scale == nullptr && a.rms_eps > 0.0f)) {
+                st = run(RingGateUp64x64{});
+                return true;
+            }
+        }
         if (tiles_of(a.M, 64, rows, 128) <= cus)
             st = run(RingGateUp64<FP8>{});
         else if (tiles_of(a.M, 128, rows, 128) <= cus)
@@ -1658,7 +1701,7 @@ int launch_gate_up(int act, int wdt, const GateUpArgs& a, int64_t packed_rows, h
                                     : launch_gate_up_pp<false, true>(a, packed_rows, stream);
         return launch_gate_up_save(act, wdt, a, packed_rows, stream);
     }
-    if (a.M <= kSkinnyMaxTokens && packed_rows % 64 == 0)
+    if (a.M <= kSkinnyMaxTokens && packed_rows % 64 == 0 && !a.on_tiles)
         return launch_gate_up_skinny(act, wdt, a, packed_rows, stream);
     {
         int st = TRMOE_OK;
@@ -1739,7 +1782,8 @@ int launch_down_combine_a8(const DownArgs& a, hipStream_t stream) {
 //
 // bf16 and e4m3 weights: the smallest tile whose grid fits the CUs once, as
 // for the gate|up, then the 256x256 ping-pong tiles.  us before -> now, bf16
-// K = 3328, N = 896: 512 tokens 19.0 -> 13.6, 777 19.7 -> 17.8, 2048 21.9 ->
+// K = 3328, N = 896: 128 tokens 13.1 -> 7.8 (32x32), 256 13.0 -> 10.4 (64x32; 11.2
+// on 32x32 tiles, more than half a round of them), 512 tokens 19.0 -> 12.6, 777 19.7 -> 17.8, 2048 21.9 ->
 // 20.7, 3001 43.8 -> 28.6, 4096 42.5 -> 31.4, 8192 59.7 -> 52.7 (256x128: N is
 // half a 256-column tile over), 10000 118 -> 62.6; bf16 K = 5632, N = 2048:
 // 3001 tokens 95 -> 83, 4096 104 -> 92, 5000 146 -> 103; e4m3 there: 130 tokens
@@ -1750,6 +1794,10 @@ static int launch_down_kind(const DownArgs& a, hipStream_t stream) {
     const int64_t mt = (a.M + 255) / 256, cus = device_cus();
     if constexpr (std::is_same_v<Kind, KindBF16>) {
         if (a.K > 0 && a.K % 64 == 0 && (!FP8 || a.ldw % 16 == 0)) {
+            if constexpr (!FP8) {
+                if (tiles_of(a.M, 32, a.N, 32) * 2 <= cus) return launch_down_shape<Kind, FP8, RingDown32>(a, stream);
+                if (tiles_of(a.M, 64, a.N, 32) <= cus) return launch_down_shape<Kind, FP8, RingDown64x32>(a, stream);
+            }
             if (tiles_of(a.M, 64, a.N, 64) <= cus) return launch_down_shape<Kind, FP8, RingDown64<FP8>>(a, stream);
             if (tiles_of(a.M, 128, a.N, 64) <= cus) return launch_down_shape<Kind, FP8, RingDown128x64<FP8>>(a, stream);
             if (tiles_of(a.M, 128, a.N, 128) <= cus) return launch_down_shape<Kind, FP8, RingDown128<FP8>>(a, stream);
@@ -1822,6 +1870,11 @@ static int launch_gate_up_grouped_pps(const GateUpArgs& a, hipStream_t stream) {
 template <class Kind, bool FP8>
 static int gate_up_grouped_kind(const GateUpArgs& a, int64_t assignments, int64_t packed_rows, hipStream_t stream) {
     if constexpr (std::is_same_v<Kind, KindBF16>) {
+        // up to one round of 128x128 tiles: the 256-row tiles of small segments leave
+        // most CUs idle (16 experts x 512 rows, 6002 assignments, hidden 2048: 61 -> 32 us)
+        if (a.K > 0 && a.K % 64 == 0 && packed_rows % 128 == 0 && (!FP8 || a.ldw % 16 == 0) &&
+            ((assignments + 127) / 128 + a.E) * (packed_rows / 128) <= device_cus())
+            return launch_gate_up_grouped_shape<Kind, FP8, RingGateUp128<FP8>>(a, assignments, packed_rows, stream);
         if (a.K > 0 && a.K % 64 == 0 && packed_rows % 256 == 0 && a.gather != nullptr && a.row_scale == nullptr &&
             a.rms_eps == 0.0f && a.gu == nullptr && a.w_expert_stride == packed_rows * a.ldw)
             return launch_gate_up_grouped_pps<FP8>(a, stream);

@@ -95,6 +95,11 @@ template <bool FP8> using RingDown128x64 = TileShape<128, 64, 2, 2, kRingPgr<FP8
 template <bool FP8> using RingDown128 = TileShape<128, 128, 2, 4, kRingPgr<FP8>, 4>;
 template <bool FP8> using Ring128x256 = TileShape<128, 256, 2, 4, kRingPgr<FP8>, 3>;
 using RingDown256x128 = TileShape<256, 128, 4, 2, 4, 3>;
+// ... and of launches that leave most CUs idle even so (bf16, about 128 tokens of
+// the 200M layer): narrower tiles, K over two and four groups.
+using RingGateUp64x64 = TileShape<64, 64, 2, 1, 4, 3, 2>;
+using RingDown32 = TileShape<32, 32, 1, 1, 4, 4, 4>;
+using RingDown64x32 = TileShape<64, 32, 2, 1, 4, 3, 4>;
 using RingDown64F32 = TileShape<64, 64, 2, 2, 4, 2, 4>;
 
 // ---------------------------------------------------------------------------

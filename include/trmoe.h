@@ -528,7 +528,7 @@ int trmoe_dense_decode(int act_dtype, const void* x, int64_t n_tokens, int64_t h
                        void* workspace, size_t workspace_bytes, void* stream);
 
 /*
- * A dense-routed layer on more than 128 tokens in one call (bf16 / f32): the
+ * A dense-routed layer on more than 64 tokens in one call (bf16 / f32): the
  * fused RMSNorm's scales (rms_eps > 0, packs with its weight folded in), the
  * gate|up and the down of trmoe_dense_routed_gate_up and
  * trmoe_shared_down_combine.  Up to about one round of workgroups the gate|up
