@@ -1,4 +1,4 @@
-// K2/K3/K4: MFMA tile kernels of the TR-MoE layer, plus weight packing.
+// K2/K3/K4: MFMA tile kernels of the TR-MoE layer.
 //
 //   k_gate_up_swiglu   shared SwiGLU gate|up GEMM with the SwiGLU epilogue
 //                      (engine.py:333-349, first half)
@@ -476,9 +476,8 @@ __device__ __forceinline__ void gate_up_epi_direct_routed(const GateUpArgs& a, c
 // gate|up + SwiGLU over bf16 activations and weights, K a multiple of 64.
 // ROUTED: the launch covers dense-routed expert columns (route gather and
 // per-token expert weights for the tiles that hold them).  TMW = 4: 256-row
-// tiles; 2: 128-row tiles (the trailing columns of a launch whose last round
-// of 256-row tiles would leave most CUs idle).  SAVE: also write the raw
-// gate|up outputs to a.gu (training forward).
+// tiles, the only ones launched.  SAVE: also write the raw gate|up outputs to
+// a.gu (training forward).
 template <bool ROUTED, int TMW, bool SAVE = false, bool FP8 = false>
 __global__ __launch_bounds__(512, 1) void k_gate_up_pp(GateUpArgs a) {
     using Shape = ShapePP<TMW>;
@@ -1328,7 +1327,9 @@ static int ensure_lds(F* fn, int bytes) {
 // at least two workgroups per CU; the down GEMM uses 256x224 when the hidden
 // size is a multiple of 224 (896 = 4 x 224: one full wave of 256 tiles with
 // no padded columns).  bf16/f32 operands take the direct buffer->LDS loads
-// (PGR 4); e4m3 weights the register-staged loop that expands them.
+// (PGR 4); e4m3 weights the register-staged loop that expands them.  bf16 and
+// e4m3 launches of K % 64 == 0 come here no more: they take ring tiles up to one
+// round and the ping-pong tiles above.
 constexpr int64_t kBigTileMinBlocks = 512;
 // The ping-pong gate|up keeps its 256x256 tiles down to half a wave of
 // workgroups: its two 4-wave groups hide the loads that an underfilled grid of
