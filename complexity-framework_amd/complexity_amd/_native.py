@@ -16,7 +16,7 @@ LIB_PATH = Path(
     os.environ.get("TRMOE_LIBRARY", str(Path(__file__).resolve().parent / "lib" / "libtrmoe.so"))
 )
 
-ABI_VERSION = 1
+ABI_VERSION = 2
 
 OK, ERR_INVALID, ERR_UNSUPPORTED, ERR_HIP = 0, 1, 2, 3
 F32, BF16, FP8_E4M3 = 0, 1, 2
@@ -53,6 +53,7 @@ class DecoderDims(ctypes.Structure):
         *((n, ctypes.c_int32) for n in ("num_heads", "num_kv_heads", "num_experts", "top_k")),
         *((n, ctypes.c_float) for n in ("norm_eps", "qk_eps", "attn_scale", "shared_scale", "routed_scale")),
         ("route_weights", ctypes.c_float * 4),
+        ("cache_batch", ctypes.c_int64),
     ]
 
 

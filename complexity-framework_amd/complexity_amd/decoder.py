@@ -313,6 +313,7 @@ class _StepPlan:
         d.num_heads, d.num_kv_heads = cfg.num_heads, cfg.num_kv_heads
         d.norm_eps, d.qk_eps, d.attn_scale, d.shared_scale, d.routed_scale = e_in, e_q, scale, ss, rs
         d.route_weights[:] = (list(rw) + [0.0] * 4)[:4]
+        d.cache_batch = dec.k_cache[0].shape[0]
         plan.layers = (ops.N.DecoderLayer * len(rows))(*rows)
         return plan
 
@@ -484,6 +485,8 @@ class TRGQADecoder(nn.Module):
         returns logits [B, V].  Graph-capturable: no host reads."""
         cfg = self.cfg
         B = ids.shape[0]
+        if B != self.k_cache[0].shape[0]:   # the caches' rows are the batch's sequences
+            raise RuntimeError(f"decode of {B} sequences over a KV cache of {self.k_cache[0].shape[0]}")
         L = self.k_cache[0].shape[2]
         dt = self.embed_tokens.weight.dtype
         pos = self._pos

@@ -665,11 +665,12 @@ def decode_linear(x: torch.Tensor, weight: torch.Tensor, residual: Optional[torc
 def decoder_step(h: torch.Tensor, dims: N.DecoderDims, layers, token_ids: torch.Tensor, position: torch.Tensor,
                  cos: torch.Tensor, sin: torch.Tensor) -> None:
     """trmoe_decoder_step: h [B, hidden] (contiguous, bf16) goes through every
-    layer of `layers` (an array of N.DecoderLayer) in place."""
+    layer of `layers` (an array of N.DecoderLayer) in place; B is the number of
+    sequences in the caches."""
     lib = _lib()
     _require_cuda(h, token_ids, position, cos, sin)
     if h.dtype != torch.bfloat16 or not h.is_contiguous() or h.shape[1] != dims.hidden or len(layers) != dims.layers \
-            or token_ids.dtype != torch.int64 or token_ids.numel() != h.shape[0] or not token_ids.is_contiguous() \
+            or h.shape[0] != dims.cache_batch or token_ids.dtype != torch.int64 or token_ids.numel() != h.shape[0] or not token_ids.is_contiguous() \
             or position.dtype != torch.int64:
         raise ValueError("decoder_step: shapes or dtypes do not match")
     n = h.shape[0]

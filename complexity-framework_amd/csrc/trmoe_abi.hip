@@ -1251,6 +1251,7 @@ int trmoe_decoder_step(const trmoe_decoder_dims* d, const trmoe_decoder_layer* l
                        int64_t positions, void* workspace, size_t workspace_bytes, void* stream) {
     StepScratch s;
     TRMOE_REQUIRE(step_dims(d, batch, &s), "decoder_step: dimensions outside trmoe_decode_attention's or the layer's");
+    TRMOE_REQUIRE(batch == d->cache_batch, "decoder_step: batch differs from the caches' sequences");
     TRMOE_REQUIRE(layers && hidden_rows && token_ids && position && cos && sin && workspace,
                   "decoder_step: null pointer");
     TRMOE_REQUIRE(d->hidden % 32 == 0 && aligned16(hidden_rows) && aligned16(workspace),

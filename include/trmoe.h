@@ -46,7 +46,7 @@
 extern "C" {
 #endif
 
-#define TRMOE_ABI_VERSION 1
+#define TRMOE_ABI_VERSION 2
 
 enum trmoe_status {
     TRMOE_OK = 0,
@@ -549,13 +549,15 @@ int trmoe_dense_layer(int act_dtype, const void* x, int64_t n_tokens, int64_t hi
  * residual, and the MLP half with its RMSNorm and residual, queued by one call
  * (the host's share of a step is then the launches alone).  hidden_rows
  * [batch, hidden] holds the embedded tokens on entry and the last layer's
- * output when the work completes.
+ * output when the work completes.  A batch other than cache_batch is refused:
+ * each sequence's keys and values go into the caches at its row.
  */
 typedef struct trmoe_decoder_dims {
     int64_t layers, hidden, cache_length, vocab_size, shared_width, expert_width;
     int32_t num_heads, num_kv_heads, num_experts, top_k;
     float norm_eps, qk_eps, attn_scale, shared_scale, routed_scale;
     float route_weights[4];
+    int64_t cache_batch;         /* sequences the caches hold: the batch of every step */
 } trmoe_decoder_dims;
 
 typedef struct trmoe_decoder_layer {
@@ -564,7 +566,7 @@ typedef struct trmoe_decoder_layer {
     const void* q_norm;          /* [64] */
     const void* k_norm;
     const void* w_o;             /* [hidden, num_heads * 64] */
-    void* k_cache;               /* [batch, num_kv_heads, cache_length, 64] */
+    void* k_cache;               /* [cache_batch, num_kv_heads, cache_length, 64] */
     void* v_cache;
     const void* w_gate_up_frag;  /* fragment-major copies of the layer's dense-routed packs, its */
     const void* w_down_frag;     /* RMSNorm weight folded into the gate|up */

@@ -1,0 +1,83 @@
+"""The host side of the decode step's native call on the CPU: the kernels'
+entry points are replaced by recorders, so that what a step hands to them, and
+what it refuses, can be looked at without a device."""
+
+import ctypes
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+from complexity_amd import _native, ops
+from complexity_amd import decoder as dec
+from complexity_amd.decoder import TRGQAConfig, TRGQADecoder
+from complexity_amd.tr_hash import TRHashBackend, TRHashEngine
+
+CFG = TRGQAConfig(vocab_size=64, hidden_size=64, num_layers=2, num_heads=2, num_kv_heads=1, shared_width=64,
+                  num_experts=4, expert_width=8, max_position_embeddings=64)
+IDS = torch.arange(2 * 6).view(2, 6)
+
+
+def _fake_pack(self, norm_weight=None, current=None):
+    if self._packed_norm is None:
+        frag = torch.zeros(64, dtype=torch.uint8)
+        self._packed_norm = ("key", SimpleNamespace(
+            strategy=ops.STRATEGY_DENSE, act_dtype=torch.bfloat16, shared_width=64, num_experts=4, expert_width=8,
+            dense_features=128, fragments=lambda name, cols: (frag, cols)))
+    return self._packed_norm[1]
+
+
+@pytest.fixture()
+def model(monkeypatch):
+    """A decoder after a prompt of two sequences whose steps go to recorders
+    (`model.calls`: one (name, arguments) per kernel call)."""
+    torch.manual_seed(0)
+    m = TRGQADecoder(CFG, backend="pytorch").to(torch.bfloat16).init_weights(1).eval()
+    m.prefill(IDS, max_new_tokens=8)
+    m.calls = []
+    monkeypatch.setattr(TRGQADecoder, "_hip_attention", lambda self, device: True)
+    monkeypatch.setattr(TRHashEngine, "_decide", lambda self, h: SimpleNamespace(selected=TRHashBackend.HIP))
+    monkeypatch.setattr(TRHashEngine, "_hip_packed", _fake_pack)
+    monkeypatch.setattr(TRGQADecoder, "_mlp", lambda self, block, h, ids: h)
+    monkeypatch.setattr(ops, "decoder_step", lambda *a: m.calls.append(("step", a)))
+
+    def attention(x, *a):
+        m.calls.append(("attention", (x, *a)))
+        return torch.zeros(x.shape[0], CFG.num_heads * 64, dtype=x.dtype)
+
+    monkeypatch.setattr(ops, "decode_attention", attention)
+    monkeypatch.setattr(ops, "decode_linear", lambda a, w, h: h)
+    return m
+
+
+def _names(m):
+    return [n for n, _ in m.calls]
+
+
+def test_step_goes_to_one_call(model):
+    model.decode_step(IDS[:, 0])
+    assert _names(model) == ["step"]
+    h, dims, layers = model.calls[0][1][:3]
+    assert h.shape == (2, 64) and dims.cache_batch == 2 and len(layers) == 2
+    assert [l.k_cache for l in layers] == [c.data_ptr() for c in model.k_cache]
+
+
+@pytest.mark.parametrize("batch", [1, 3, 5, 16])
+def test_other_batch_than_the_caches_is_refused(model, batch):
+    with pytest.raises(RuntimeError):
+        model.decode_step(torch.zeros(batch, dtype=torch.int64))
+    assert model.calls == [] and model.cache_len == 6
+
+
+def test_native_step_refuses_another_batch():
+    lib = _native.load()
+    d = _native.DecoderDims()
+    d.layers, d.hidden, d.cache_length, d.vocab_size, d.shared_width, d.expert_width = 1, 64, 64, 64, 64, 8
+    d.num_heads, d.num_kv_heads, d.num_experts, d.top_k, d.cache_batch = 2, 1, 4, 2, 2
+    buf = ctypes.create_string_buffer(4096)
+    p = ctypes.c_void_p((ctypes.addressof(buf) + 255) // 256 * 256)
+    layer = (_native.DecoderLayer * 1)()
+    nbytes = lib.trmoe_decoder_step_workspace_bytes(ctypes.byref(d), 5)
+    assert nbytes > 0
+    st = lib.trmoe_decoder_step(ctypes.byref(d), ctypes.cast(layer, ctypes.c_void_p), p, 5, p, p, p, p, 64, p, nbytes, None)
+    assert st == _native.ERR_INVALID and b"batch" in lib.trmoe_last_error()
