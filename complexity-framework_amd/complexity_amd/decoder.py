@@ -227,9 +227,10 @@ class _StepPlan:
     """The layers of a decode step as one native call takes them
     (``trmoe_decoder_step``): the pointers of every block's weights, packs and
     caches, with what they were read from.  ``current`` looks at all of it
-    again before each step: module and parameter objects, in-place versions,
-    storage, packs, routing.  Without it a step spends about 100 us per layer
-    in Python, against 30 us of kernels."""
+    again before each step: module, parameter and cache objects, in-place
+    versions, storage, norm and attention constants, packs, routing.  Without
+    the plan a step spends about 100 us per layer in Python, against 30 us of
+    kernels."""
 
     def __init__(self):
         self.dims = ops.N.DecoderDims()
@@ -237,6 +238,8 @@ class _StepPlan:
         self.engines = []   # (engine, config, strategy, E, W, pack entry, route table)
         self.members = []   # (owner's dict, name, object)
         self.tensors = []   # (owner's dict, name, tensor, version, pointer)
+        self.values = []    # (object's dict, name, value)
+        self.caches = []    # (k or v, layer, tensor, pointer, shape)
         self.keep = []      # what the pointers point into
 
     def _watch(self, owner: nn.Module, name: str) -> nn.Module:
@@ -249,14 +252,26 @@ class _StepPlan:
         self.tensors.append((owner._parameters, name, t, t._version, t.data_ptr()))
         return t
 
+    def _value(self, owner: nn.Module, name: str) -> float:
+        v = getattr(owner, name)
+        self.values.append((owner.__dict__, name, v))
+        return v
+
+    def _cache(self, dec: "TRGQADecoder", name: str, layer: int) -> torch.Tensor:
+        t = getattr(dec, name)[layer]
+        self.caches.append((name == "k_cache", layer, t, t.data_ptr(), t.shape))
+        return t
+
     @classmethod
     def build(cls, dec: "TRGQADecoder", device: torch.device) -> Optional["_StepPlan"]:
         """None when a block needs the general path: a replaced MLP half,
         adapted or e4m3 weights, grouped experts, layers that differ in shape."""
-        if dec.mlp_fn is not None:
+        if dec.mlp_fn is not None or len(dec.k_cache) != len(dec.layers) or len(dec.v_cache) != len(dec.layers):
             return None
         plan = cls()
         cfg, rows, shapes = dec.cfg, [], set()
+        plan.values.append((dec.__dict__, "cfg", cfg))
+        plan._watch(dec, "layers")
         for i, (name, block) in enumerate(dec.layers._modules.items()):
             plan.members.append((dec.layers._modules, name, block))
             attn, mlp = plan._watch(block, "self_attn"), plan._watch(block, "mlp")
@@ -284,8 +299,15 @@ class _StepPlan:
             if table.dtype is not torch.int64 or not table.is_contiguous():
                 return None
             shapes.add((packed.shared_width, packed.num_experts, packed.expert_width, tuple(table.shape),
-                        tuple(c.route_weights), c.shared_output_scale, c.routed_output_scale, norm_in.eps,
-                        norm_post.eps, attn.q_norm.eps, attn.k_norm.eps, attn.scale))
+                        tuple(c.route_weights), c.shared_output_scale, c.routed_output_scale,
+                        plan._value(norm_in, "eps"), plan._value(norm_post, "eps"), plan._value(attn.q_norm, "eps"),
+                        plan._value(attn.k_norm, "eps"), plan._value(attn, "scale")))
+            caches = plan._cache(dec, "k_cache", i), plan._cache(dec, "v_cache", i)
+            for t in caches:
+                if (t.dtype is not torch.bfloat16 or t.device != dec.k_cache[0].device or not t.is_contiguous()
+                        or t.ndim != 4 or t.shape != dec.k_cache[0].shape
+                        or t.shape[1:] != (cfg.num_kv_heads, t.shape[2], cfg.head_dim)):
+                    return None
             for n in ("k_proj", "q_proj", "v_proj"):
                 plan._weight(plan._watch(attn, n), "weight")
             kqv = attn.kqv_weight()
@@ -293,8 +315,7 @@ class _StepPlan:
             dn = packed.fragments("dense_down", packed.dense_features)[0]
             ptrs = (plan._weight(norm_in, "weight"), kqv, plan._weight(plan._watch(attn, "q_norm"), "weight"),
                     plan._weight(plan._watch(attn, "k_norm"), "weight"),
-                    plan._weight(plan._watch(attn, "o_proj"), "weight"), dec.k_cache[i], dec.v_cache[i],
-                    gu, dn, table)
+                    plan._weight(plan._watch(attn, "o_proj"), "weight"), *caches, gu, dn, table)
             if any(t.data_ptr() % 16 for t in ptrs) or kqv.dtype is not torch.bfloat16:
                 return None
             plan.keep.append(ptrs)
@@ -325,7 +346,13 @@ class _StepPlan:
                     or eng._active_num_experts != E or eng._active_expert_width != W
                     or eng._active_route_table is not table or eng._fp8):
                 return False
-        return (all(d.get(n) is m for d, n, m in self.members)
+        k, v, n = dec.k_cache, dec.v_cache, len(self.engines)
+        if len(k) != n or len(v) != n:
+            return False
+        for is_k, i, t, p, shape in self.caches:
+            if (k if is_k else v)[i] is not t or t.data_ptr() != p or t.shape != shape:
+                return False
+        return (all(d.get(n) is m for d, n, m in self.members) and all(d.get(n) == x for d, n, x in self.values)
                 and all(d.get(n) is t and t._version == v and t.data_ptr() == p for d, n, t, v, p in self.tensors))
 
 

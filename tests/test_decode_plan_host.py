@@ -69,6 +69,63 @@ def test_other_batch_than_the_caches_is_refused(model, batch):
     assert model.calls == [] and model.cache_len == 6
 
 
+def _caches(m):
+    m.k_cache = [c.clone() for c in m.k_cache]
+
+
+def _longer_caches(m):
+    m.k_cache = [torch.cat((c, c), 2) for c in m.k_cache]
+    m.v_cache = [torch.cat((c, c), 2) for c in m.v_cache]
+
+
+def _one_cache(m):
+    m.v_cache[1] = m.v_cache[1].clone()
+
+
+def _cache_storage(m):
+    m.v_cache[0].set_(m.v_cache[0].clone())
+
+
+def _scale(m):
+    for b in m.layers:
+        b.self_attn.scale = 0.25
+
+
+def _eps(m):
+    for b in m.layers:
+        b.input_layernorm.eps = b.post_attention_layernorm.eps = 1e-3
+
+
+def _qk_eps(m):
+    for b in m.layers:
+        b.self_attn.q_norm.eps = b.self_attn.k_norm.eps = 1e-4
+
+
+@pytest.mark.parametrize("change", [_caches, _longer_caches, _one_cache, _cache_storage, _scale, _eps, _qk_eps])
+def test_changes_between_steps_are_seen(model, change):
+    model.decode_step(IDS[:, 0])
+    plan = model._step_plan
+    model.decode_step(IDS[:, 0])
+    assert model._step_plan is plan   # nothing changed: the same plan again
+    change(model)
+    model.decode_step(IDS[:, 1])
+    assert _names(model) == ["step"] * 3
+    dims, layers = model.calls[2][1][1:3]
+    assert [l.k_cache for l in layers] == [c.data_ptr() for c in model.k_cache]
+    assert [l.v_cache for l in layers] == [c.data_ptr() for c in model.v_cache]
+    b = model.layers[0]
+    got = (dims.cache_length, dims.norm_eps, dims.qk_eps, dims.attn_scale)
+    assert got == pytest.approx((model.k_cache[0].shape[2], b.input_layernorm.eps, b.self_attn.q_norm.eps,
+                                 b.self_attn.scale))
+
+
+def test_unequal_caches_take_the_blocks(model):
+    model.decode_step(IDS[:, 0])
+    model.k_cache[1] = torch.cat((model.k_cache[1], model.k_cache[1]), 2)
+    model.decode_step(IDS[:, 1])
+    assert _names(model) == ["step"] + ["attention"] * 2
+
+
 def test_native_step_refuses_another_batch():
     lib = _native.load()
     d = _native.DecoderDims()

@@ -96,6 +96,33 @@ def test_changes_between_steps(model, change):
     assert torch.equal(got[0], plain[0]) and not torch.equal(got[1], plain[1])
 
 
+def _reorder(m, s):
+    """A beam's caches follow another sequence."""
+    if s == 1:
+        order = torch.tensor([1, 0], device=m.norm.weight.device)
+        m.k_cache = [c.index_select(0, order) for c in m.k_cache]
+        m.v_cache = [c.index_select(0, order) for c in m.v_cache]
+
+
+def _eps(m, s):
+    for b in m.layers:
+        b.self_attn.q_norm.eps = b.self_attn.k_norm.eps = 1e-2 if s == 1 else 1e-6
+
+
+def _scale(m, s):
+    for b in m.layers:
+        b.self_attn.scale = 0.5 if s == 1 else 0.125
+
+
+@pytest.mark.parametrize("change", [_reorder, _eps, _scale])
+def test_caches_and_constants_between_steps(model, change):
+    got, used = _steps(model, 2, 4, True, change)
+    want, _ = _steps(model, 2, 4, False, change)
+    plain, _ = _steps(model, 2, 4, True)
+    assert all(used) and torch.equal(got, want)
+    assert torch.equal(got[0], plain[0]) and not torch.equal(got[1], plain[1])
+
+
 def test_hooked_norm_is_called(model):
     seen = []
     handle = model.layers[1].input_layernorm.register_forward_hook(lambda mod, args, out: seen.append(1))
