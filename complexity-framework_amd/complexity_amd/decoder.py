@@ -309,7 +309,9 @@ class _StepPlan:
                         or t.shape[1:] != (cfg.num_kv_heads, t.shape[2], cfg.head_dim)):
                     return None
             for n in ("k_proj", "q_proj", "v_proj"):
-                plan._weight(plan._watch(attn, n), "weight")
+                if "weight" not in plan._watch(attn, n)._parameters:
+                    return None   # parametrized: kqv_weight() materialises it per call
+                plan._weight(attn._modules[n], "weight")
             kqv = attn.kqv_weight()
             gu = packed.fragments("dense_gate_up", cfg.hidden_size)[0]
             dn = packed.fragments("dense_down", packed.dense_features)[0]

@@ -126,6 +126,31 @@ def test_unequal_caches_take_the_blocks(model):
     assert _names(model) == ["step"] + ["attention"] * 2
 
 
+class _Twice(torch.nn.Module):
+    def forward(self, w):
+        return w * 2
+
+
+@pytest.mark.parametrize("name", ["q_proj", "k_proj", "v_proj"])
+def test_parametrized_projection_takes_the_blocks(model, name):
+    attn = model.layers[1].self_attn
+    torch.nn.utils.parametrize.register_parametrization(getattr(attn, name), "weight", _Twice())
+    model.decode_step(IDS[:, 0])
+    assert _names(model) == ["attention"] * 2
+    kqv = model.calls[1][1][3]
+    assert torch.equal(kqv, torch.cat([getattr(attn, n).weight for n in ("k_proj", "q_proj", "v_proj")]))
+
+
+def test_parametrization_between_steps_is_seen(model):
+    model.decode_step(IDS[:, 0])
+    attn = model.layers[0].self_attn
+    torch.nn.utils.parametrize.register_parametrization(attn.q_proj, "weight", _Twice())
+    model.decode_step(IDS[:, 1])
+    torch.nn.utils.parametrize.remove_parametrizations(attn.q_proj, "weight", leave_parametrized=True)
+    model.decode_step(IDS[:, 2])
+    assert _names(model) == ["step"] + ["attention"] * 2 + ["step"]
+
+
 def test_native_step_refuses_another_batch():
     lib = _native.load()
     d = _native.DecoderDims()
