@@ -383,6 +383,11 @@ class TRGQADecoder(nn.Module):
         self._step_plan: Optional[_StepPlan] = None
         self._graph = None
 
+    def __getstate__(self):
+        # a copy builds a plan of its own: this one points at this module's
+        # weights and caches
+        return {**self.__dict__, "_step_plan": None}
+
     # ------------------------------------------------------------------ weights
     @torch.no_grad()
     def init_weights(self, seed: int = 0) -> "TRGQADecoder":

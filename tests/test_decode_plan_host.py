@@ -2,7 +2,10 @@
 entry points are replaced by recorders, so that what a step hands to them, and
 what it refuses, can be looked at without a device."""
 
+import copy
 import ctypes
+import io
+import pickle
 from types import SimpleNamespace
 
 import pytest
@@ -18,12 +21,16 @@ CFG = TRGQAConfig(vocab_size=64, hidden_size=64, num_layers=2, num_heads=2, num_
 IDS = torch.arange(2 * 6).view(2, 6)
 
 
+class _Pack(SimpleNamespace):
+    def fragments(self, name, cols):
+        return self.frag, cols
+
+
 def _fake_pack(self, norm_weight=None, current=None):
     if self._packed_norm is None:
-        frag = torch.zeros(64, dtype=torch.uint8)
-        self._packed_norm = ("key", SimpleNamespace(
+        self._packed_norm = ("key", _Pack(
             strategy=ops.STRATEGY_DENSE, act_dtype=torch.bfloat16, shared_width=64, num_experts=4, expert_width=8,
-            dense_features=128, fragments=lambda name, cols: (frag, cols)))
+            dense_features=128, frag=torch.zeros(64, dtype=torch.uint8)))
     return self._packed_norm[1]
 
 
@@ -149,6 +156,32 @@ def test_parametrization_between_steps_is_seen(model):
     torch.nn.utils.parametrize.remove_parametrizations(attn.q_proj, "weight", leave_parametrized=True)
     model.decode_step(IDS[:, 2])
     assert _names(model) == ["step"] + ["attention"] * 2 + ["step"]
+
+
+@pytest.mark.parametrize("how", ["deepcopy", "pickle", "save"])
+def test_copies_do_not_take_the_plan_along(model, how):
+    model.decode_step(IDS[:, 0])
+    assert model._step_plan is not None
+    calls, model.calls = model.calls, []
+    if how == "deepcopy":
+        other = copy.deepcopy(model)
+    else:
+        f = io.BytesIO()
+        if how == "pickle":
+            pickle.dump(model, f)
+            f.seek(0)
+            other = pickle.load(f)   # written just above
+        else:
+            torch.save(model, f)
+            f.seek(0)
+            other = torch.load(f, weights_only=False)
+    assert model._step_plan is not None and other._step_plan is None
+    model.calls = calls
+    for m in (other, model):
+        m.decode_step(IDS[:, 1])
+        layers = calls[-1][1][2]
+        assert [l.k_cache for l in layers] == [c.data_ptr() for c in m.k_cache]
+    assert _names(model) == ["step"] * 3
 
 
 def test_native_step_refuses_another_batch():
