@@ -447,6 +447,8 @@ class TRGQADecoder(nn.Module):
             if not (_plain(m["input_layernorm"], RMSNorm) and _plain(a["q_norm"], RMSNorm)
                     and _plain(a["k_norm"], RMSNorm) and _plain(a["o_proj"], nn.Linear)):
                 return False
+            if a["q_norm"].eps != a["k_norm"].eps:   # the kernels norm both with one
+                return False
         return True
 
     def _norm(self, norm: RMSNorm, h: torch.Tensor, hip: bool) -> torch.Tensor:

@@ -196,3 +196,26 @@ def test_native_step_refuses_another_batch():
     assert nbytes > 0
     st = lib.trmoe_decoder_step(ctypes.byref(d), ctypes.cast(layer, ctypes.c_void_p), p, 5, p, p, p, p, 64, p, nbytes, None)
     assert st == _native.ERR_INVALID and b"batch" in lib.trmoe_last_error()
+
+
+# ---------------------------------------------------------------------------
+# which decoders the HIP attention half takes (looks at modules only)
+# ---------------------------------------------------------------------------
+CUDA = torch.device("cuda:0")
+
+
+def _decoder(cfg=CFG, **kw):
+    return TRGQADecoder(cfg, **kw).to(torch.bfloat16).eval()
+
+
+def test_attention_takes_the_decoder_as_built():
+    assert _decoder()._hip_attention(CUDA)
+
+
+def test_unequal_q_and_k_eps_take_the_general_path():
+    """The kernels norm q and k with one eps."""
+    m = _decoder()
+    m.layers[1].self_attn.k_norm.eps = 1e-2
+    assert not m._hip_attention(CUDA)
+    m.layers[1].self_attn.q_norm.eps = 1e-2
+    assert m._hip_attention(CUDA)

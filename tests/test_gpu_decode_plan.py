@@ -130,3 +130,17 @@ def test_hooked_norm_is_called(model):
     assert len(seen) == 3 and not any(used)   # the prompt and two steps
     handle.remove()
     assert all(_steps(model, 2, 2, True)[1])
+
+
+def test_k_norm_eps_of_its_own(model):
+    """k is normed with k_norm's own eps: the prompt and the steps of the
+    general path, whose rounding to bf16 after each operation is the bound."""
+    for b in model.layers:
+        b.self_attn.k_norm.eps = 0.5
+    got, _ = _steps(model, 2, 3, True)
+    ref = TRGQADecoder(CFG, backend="pytorch").to(got.device).eval()
+    ref.load_state_dict({k: v.float() if v.is_floating_point() else v for k, v in model.state_dict().items()})
+    for b in ref.layers:
+        b.self_attn.k_norm.eps = 0.5
+    want, _ = _steps(ref, 2, 3, True)
+    assert float((got.float() - want).abs().max() / want.abs().max()) <= 2e-2
