@@ -223,6 +223,12 @@ def _plain(mod: nn.Module, cls: type) -> bool:
     return w is not None and w.dtype is torch.bfloat16 and w.is_contiguous() and mod._parameters.get("bias") is None
 
 
+def _pinned(block: nn.Module) -> bool:
+    """A block whose engine is pinned to PYTORCH (a replaced MLP half is not)."""
+    config = getattr(block._modules.get("mlp"), "config", None)
+    return getattr(config, "backend", None) is TRHashBackend.PYTORCH
+
+
 class _StepPlan:
     """The layers of a decode step as one native call takes them
     (``trmoe_decoder_step``): the pointers of every block's weights, packs and
@@ -441,7 +447,7 @@ class TRGQADecoder(nn.Module):
         for block in self.layers:
             m = block._modules
             attn = m["self_attn"]
-            if type(attn) is not GQAttention or m["mlp"].config.backend is TRHashBackend.PYTORCH:
+            if type(attn) is not GQAttention or _pinned(block):
                 return False
             a = attn._modules
             if not (_plain(m["input_layernorm"], RMSNorm) and _plain(a["q_norm"], RMSNorm)
@@ -456,10 +462,14 @@ class TRGQADecoder(nn.Module):
             return norm(h)
         return ops.rmsnorm_forward(h.reshape(-1, h.shape[-1]), norm.weight, norm.eps)[0].view(h.shape)
 
+    def _hip_norm(self, norm: RMSNorm, h: torch.Tensor) -> bool:
+        """Whether a GPU's h goes through `norm` on the RMSNorm kernel."""
+        return (not torch.is_grad_enabled() and h.dtype is torch.bfloat16 and _plain(norm, RMSNorm)
+                and ops.rmsnorm_unsupported(h, norm.weight) is None
+                and not any(_pinned(b) for b in list(self.layers._modules.values())[:1]))
+
     def logits(self, h: torch.Tensor) -> torch.Tensor:
-        hip = (not torch.is_grad_enabled() and h.device.type == "cuda" and h.dtype is torch.bfloat16
-               and _plain(self.norm, RMSNorm) and ops.rmsnorm_unsupported(h, self.norm.weight) is None
-               and self.layers[0].mlp.config.backend is not TRHashBackend.PYTORCH)
+        hip = h.device.type == "cuda" and self._hip_norm(self.norm, h)
         return F.linear(self._norm(self.norm, h, hip), self.embed_tokens.weight)
 
     # ------------------------------------------------------------------ prompt

@@ -219,3 +219,23 @@ def test_unequal_q_and_k_eps_take_the_general_path():
     assert not m._hip_attention(CUDA)
     m.layers[1].self_attn.q_norm.eps = 1e-2
     assert m._hip_attention(CUDA)
+
+
+def test_replaced_mlps_need_no_engine():
+    """A replaced MLP half is only called: it has no engine's configuration."""
+    m = _decoder()
+    for b in m.layers:
+        b.mlp = torch.nn.Identity()
+    assert m._hip_attention(CUDA)
+    assert not _decoder(backend="pytorch")._hip_attention(CUDA)
+
+
+@pytest.mark.parametrize("what", ["identity", "no_layers"])
+def test_logits_without_engines(what):
+    m = _decoder(TRGQAConfig(vocab_size=64, hidden_size=64, num_layers=0) if what == "no_layers" else CFG)
+    for b in m.layers:
+        b.mlp = torch.nn.Identity()
+    with torch.no_grad():
+        assert m._hip_norm(m.norm, torch.zeros(2, 64, dtype=torch.bfloat16))
+        pinned = _decoder(backend="pytorch")
+        assert not pinned._hip_norm(pinned.norm, torch.zeros(2, 64, dtype=torch.bfloat16))

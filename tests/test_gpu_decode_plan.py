@@ -144,3 +144,21 @@ def test_k_norm_eps_of_its_own(model):
         b.self_attn.k_norm.eps = 0.5
     want, _ = _steps(ref, 2, 3, True)
     assert float((got.float() - want).abs().max() / want.abs().max()) <= 2e-2
+
+
+class _Wrapped(torch.nn.Module):
+    """A replaced MLP half that offers what the decoder calls, and no more."""
+
+    def __init__(self, engine):
+        super().__init__()
+        self.engine = [engine]
+
+    def forward_norm_residual(self, *a):
+        return self.engine[0].forward_norm_residual(*a)
+
+
+def test_replaced_mlp_module(model):
+    want, _ = _steps(model, 2, 3, False)
+    model.layers[1].mlp = _Wrapped(model.layers[1].mlp)
+    got, used = _steps(model, 2, 3, True)
+    assert not any(used) and torch.equal(got, want)
