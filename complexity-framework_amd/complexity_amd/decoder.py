@@ -560,11 +560,12 @@ class TRGQADecoder(nn.Module):
         B = ids.shape[0]
         cos, sin = self._rope_tables32(L, ids.device)
         tok = ids.view(B, 1)
-        h = self.embed_tokens(ids)
+        h = self.embed_tokens(tok).view(B, -1)
         if self._step_plan is None or not self._step_plan.current(self):
             self._step_plan = _StepPlan.build(self, ids.device)
         if self._step_plan is not None and h.is_contiguous():
-            ops.decoder_step(h, self._step_plan.dims, self._step_plan.layers, ids.contiguous(), pos, cos, sin)
+            ids = tok.view(B).to(torch.int64).contiguous()
+            ops.decoder_step(h, self._step_plan.dims, self._step_plan.layers, ids, pos, cos, sin)
             return self.logits(h)
         for i, block in enumerate(self.layers):
             attn, norm = block.self_attn, block.input_layernorm

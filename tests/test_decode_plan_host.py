@@ -10,6 +10,7 @@ from types import SimpleNamespace
 
 import pytest
 import torch
+import torch.nn.functional as F
 
 from complexity_amd import _native, ops
 from complexity_amd import decoder as dec
@@ -67,6 +68,21 @@ def test_step_goes_to_one_call(model):
     h, dims, layers = model.calls[0][1][:3]
     assert h.shape == (2, 64) and dims.cache_batch == 2 and len(layers) == 2
     assert [l.k_cache for l in layers] == [c.data_ptr() for c in model.k_cache]
+
+
+@pytest.mark.parametrize("blocks", [False, True])
+@pytest.mark.parametrize("ids", [IDS[:, :1], IDS[:, 0].int(), IDS[:, :1].int(), IDS.t()[0]],
+                         ids=["column", "int32", "int32_column", "strided"])
+def test_forms_of_the_token_ids(model, ids, blocks):
+    if blocks:
+        model.mlp_fn = lambda i, h, tok, block: h
+    out = model.decode_step(ids)
+    assert out.shape == (2, CFG.vocab_size)
+    want = F.embedding(IDS[:, 0], model.embed_tokens.weight)
+    for name, a in model.calls:
+        assert torch.equal(a[0], want)
+        if name == "step":
+            assert a[3].dtype == torch.int64 and a[3].is_contiguous() and torch.equal(a[3], IDS[:, 0])
 
 
 @pytest.mark.parametrize("batch", [1, 3, 5, 16])
