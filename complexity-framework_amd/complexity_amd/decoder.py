@@ -214,13 +214,15 @@ class TRGQABlock(nn.Module):
         self.layer_index = layer_index
 
 
-def _plain(mod: nn.Module, cls: type) -> bool:
+def _plain(mod: nn.Module, cls: type, *shape: int) -> bool:
     """A module of exactly `cls` (so not parametrized or replaced) without
-    hooks or bias, its weight in bf16: what a kernel may stand in for."""
+    hooks or bias, its weight in bf16, of `shape` and laid out as the kernels
+    read it (contiguous, 16-byte aligned): what a kernel may stand in for."""
     if type(mod) is not cls or mod._forward_hooks or mod._forward_pre_hooks:
         return False
     w = mod._parameters.get("weight")
-    return w is not None and w.dtype is torch.bfloat16 and w.is_contiguous() and mod._parameters.get("bias") is None
+    return (w is not None and w.dtype is torch.bfloat16 and w.shape == shape and w.is_contiguous()
+            and w.data_ptr() % 16 == 0 and mod._parameters.get("bias") is None)
 
 
 def _pinned(block: nn.Module) -> bool:
@@ -282,7 +284,7 @@ class _StepPlan:
             plan.members.append((dec.layers._modules, name, block))
             attn, mlp = plan._watch(block, "self_attn"), plan._watch(block, "mlp")
             norm_in, norm_post = plan._watch(block, "input_layernorm"), plan._watch(block, "post_attention_layernorm")
-            if not _plain(norm_post, RMSNorm) or type(mlp) is not TRHashEngine or mlp._fp8:
+            if not _plain(norm_post, RMSNorm, cfg.hidden_size) or type(mlp) is not TRHashEngine or mlp._fp8:
                 return None
             for n in ("shared_gate", "shared_up", "shared_down"):
                 mod = mlp._modules.get(n)
@@ -450,8 +452,9 @@ class TRGQADecoder(nn.Module):
             if type(attn) is not GQAttention or _pinned(block):
                 return False
             a = attn._modules
-            if not (_plain(m["input_layernorm"], RMSNorm) and _plain(a["q_norm"], RMSNorm)
-                    and _plain(a["k_norm"], RMSNorm) and _plain(a["o_proj"], nn.Linear)):
+            H, D = cfg.hidden_size, cfg.head_dim
+            if not (_plain(m["input_layernorm"], RMSNorm, H) and _plain(a["q_norm"], RMSNorm, D)
+                    and _plain(a["k_norm"], RMSNorm, D) and _plain(a["o_proj"], nn.Linear, H, cfg.num_heads * D)):
                 return False
             if a["q_norm"].eps != a["k_norm"].eps:   # the kernels norm both with one
                 return False
@@ -464,7 +467,7 @@ class TRGQADecoder(nn.Module):
 
     def _hip_norm(self, norm: RMSNorm, h: torch.Tensor) -> bool:
         """Whether a GPU's h goes through `norm` on the RMSNorm kernel."""
-        return (not torch.is_grad_enabled() and h.dtype is torch.bfloat16 and _plain(norm, RMSNorm)
+        return (not torch.is_grad_enabled() and h.dtype is torch.bfloat16 and _plain(norm, RMSNorm, h.shape[-1])
                 and ops.rmsnorm_unsupported(h, norm.weight) is None
                 and not any(_pinned(b) for b in list(self.layers._modules.values())[:1]))
 

@@ -255,3 +255,37 @@ def test_logits_without_engines(what):
         assert m._hip_norm(m.norm, torch.zeros(2, 64, dtype=torch.bfloat16))
         pinned = _decoder(backend="pytorch")
         assert not pinned._hip_norm(pinned.norm, torch.zeros(2, 64, dtype=torch.bfloat16))
+
+
+def _misaligned(p):
+    flat = torch.zeros(p.numel() + 8, dtype=p.dtype)
+    return torch.nn.Parameter(flat[1:1 + p.numel()].view_as(p))
+
+
+def _misaligned_o(m):
+    m.layers[1].self_attn.o_proj.weight = _misaligned(m.layers[1].self_attn.o_proj.weight)
+
+
+def _one_q(m):
+    m.layers[0].self_attn.q_norm.weight = torch.nn.Parameter(torch.ones(1, dtype=torch.bfloat16))
+
+
+def _one_in(m):
+    m.layers[0].input_layernorm.weight = torch.nn.Parameter(torch.ones(1, dtype=torch.bfloat16))
+
+
+@pytest.mark.parametrize("change", [_misaligned_o, _one_q, _one_in])
+def test_weights_the_kernels_cannot_read_take_the_general_path(change):
+    """Kernels read 16 bytes at a time, and whole rows of norm weights."""
+    m = _decoder()
+    change(m)
+    assert not m._hip_attention(CUDA)
+
+
+def test_logits_norm_weight_of_one_value():
+    m = _decoder()
+    h = torch.zeros(2, 64, dtype=torch.bfloat16)
+    with torch.no_grad():
+        assert m._hip_norm(m.norm, h)
+        m.norm.weight = torch.nn.Parameter(torch.ones(1, dtype=torch.bfloat16))
+        assert not m._hip_norm(m.norm, h)
