@@ -446,6 +446,8 @@ class TRGQADecoder(nn.Module):
         if (device.type != "cuda" or self.embed_tokens.weight.dtype is not torch.bfloat16
                 or ops.attention_unsupported(cfg.hidden_size, cfg.num_heads, cfg.num_kv_heads, cfg.head_dim)):
             return False
+        if torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") is not torch.bfloat16:
+            return False   # the projections come out in another dtype
         for block in self.layers:
             m = block._modules
             attn = m["self_attn"]

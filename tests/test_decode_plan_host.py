@@ -289,3 +289,12 @@ def test_logits_norm_weight_of_one_value():
         assert m._hip_norm(m.norm, h)
         m.norm.weight = torch.nn.Parameter(torch.ones(1, dtype=torch.bfloat16))
         assert not m._hip_norm(m.norm, h)
+
+
+@pytest.mark.parametrize("dtype,takes", [(torch.float16, False), (torch.bfloat16, True)])
+def test_autocast_to_another_type_takes_the_general_path(monkeypatch, dtype, takes):
+    """Under autocast to fp16 the projections come out in fp16."""
+    m = _decoder()
+    monkeypatch.setattr(torch, "is_autocast_enabled", lambda device_type="cuda": True)
+    monkeypatch.setattr(torch, "get_autocast_dtype", lambda device_type: dtype)
+    assert m._hip_attention(CUDA) is takes

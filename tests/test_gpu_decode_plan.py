@@ -162,3 +162,12 @@ def test_replaced_mlp_module(model):
     model.layers[1].mlp = _Wrapped(model.layers[1].mlp)
     got, used = _steps(model, 2, 3, True)
     assert not any(used) and torch.equal(got, want)
+
+
+def test_prompt_under_fp16_autocast(model):
+    ids = torch.arange(20, device=model.norm.weight.device).view(2, 10)
+    want = model.prefill(ids)
+    with torch.autocast("cuda", dtype=torch.float16):
+        got = model.prefill(ids)
+    # fp16 projections of a bf16 residual stream: the decoder's bf16 bar
+    assert float((got.float() - want.float()).abs().max() / want.float().abs().max()) <= 2e-2
