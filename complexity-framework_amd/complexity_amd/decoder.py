@@ -225,6 +225,15 @@ def _plain(mod: nn.Module, cls: type, *shape: int) -> bool:
             and w.data_ptr() % 16 == 0 and mod._parameters.get("bias") is None)
 
 
+def _values(t: torch.Tensor) -> bool:
+    """A tensor whose memory a kernel may read in place of the torch
+    operations: no function transform, forward-mode derivative or trace has to
+    see them."""
+    return (type(t) in (torch.Tensor, nn.Parameter) and torch.autograd.forward_ad._current_level < 0
+            and torch._C._functorch.peek_interpreter_stack() is None and torch._C._len_torch_dispatch_stack() == 0
+            and not torch.jit.is_tracing() and not torch.compiler.is_compiling())
+
+
 def _pinned(block: nn.Module) -> bool:
     """A block whose engine is pinned to PYTORCH (a replaced MLP half is not)."""
     config = getattr(block._modules.get("mlp"), "config", None)
@@ -469,7 +478,7 @@ class TRGQADecoder(nn.Module):
 
     def _hip_norm(self, norm: RMSNorm, h: torch.Tensor) -> bool:
         """Whether a GPU's h goes through `norm` on the RMSNorm kernel."""
-        return (not torch.is_grad_enabled() and h.dtype is torch.bfloat16 and _plain(norm, RMSNorm, h.shape[-1])
+        return (_values(h) and not torch.is_grad_enabled() and h.dtype is torch.bfloat16 and _plain(norm, RMSNorm, h.shape[-1])
                 and ops.rmsnorm_unsupported(h, norm.weight) is None
                 and not any(_pinned(b) for b in list(self.layers._modules.values())[:1]))
 

@@ -10,7 +10,9 @@ from types import SimpleNamespace
 
 import pytest
 import torch
+import torch.autograd.forward_ad as fwAD
 import torch.nn.functional as F
+from torch.fx.experimental.proxy_tensor import make_fx
 
 from complexity_amd import _native, ops
 from complexity_amd import decoder as dec
@@ -298,3 +300,24 @@ def test_autocast_to_another_type_takes_the_general_path(monkeypatch, dtype, tak
     monkeypatch.setattr(torch, "is_autocast_enabled", lambda device_type="cuda": True)
     monkeypatch.setattr(torch, "get_autocast_dtype", lambda device_type: dtype)
     assert m._hip_attention(CUDA) is takes
+
+
+def test_logits_under_function_transforms():
+    """vmap, forward-mode derivatives and traces see the torch operations."""
+    m = _decoder()
+    h = torch.randn(3, 2, 64, generator=torch.Generator().manual_seed(0)).bfloat16()
+    seen = []
+
+    def look(x):
+        seen.append(m._hip_norm(m.norm, x))
+        return x
+
+    with torch.no_grad():
+        look(h)
+        torch.func.vmap(look)(h)
+        with fwAD.dual_level():
+            look(fwAD.make_dual(h, h))
+        with torch._subclasses.FakeTensorMode() as mode:
+            look(mode.from_tensor(h))
+        make_fx(look)(h)
+    assert seen == [True, False, False, False, False]

@@ -5,6 +5,7 @@ active capacity, routing, the MLP override, a new prompt."""
 
 import pytest
 import torch
+import torch.nn.functional as F
 
 from complexity_amd import decoder as dec
 from complexity_amd.decoder import TRGQAConfig, TRGQADecoder
@@ -171,3 +172,12 @@ def test_prompt_under_fp16_autocast(model):
         got = model.prefill(ids)
     # fp16 projections of a bf16 residual stream: the decoder's bf16 bar
     assert float((got.float() - want.float()).abs().max() / want.float().abs().max()) <= 2e-2
+
+
+def test_logits_under_vmap_and_forward_mode(model):
+    h = torch.randn(3, 2, 256, generator=torch.Generator().manual_seed(0)).to(model.norm.weight.device).bfloat16()
+    with torch.no_grad(), torch.autograd.forward_ad.dual_level():
+        want = F.linear(model.norm(h), model.embed_tokens.weight)   # the torch operations
+        assert torch.equal(torch.func.vmap(model.logits)(h), want)
+        out, tangent = torch.autograd.forward_ad.unpack_dual(model.logits(torch.autograd.forward_ad.make_dual(h, h * 0.5)))
+    assert torch.equal(out, want) and tangent is not None and bool(tangent.float().abs().sum() > 0)
