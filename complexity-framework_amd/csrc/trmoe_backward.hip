@@ -248,10 +248,8 @@ __device__ __forceinline__ void mma_stage_tr(const char* As, const char* Bs, int
 // ---------------------------------------------------------------------------
 using ShapeBwdGU = TileShape<256, 256, 2, 4, 4>;   // packed gate|up columns of 128 features
 using ShapeBwdDH = TileShape<256, 128, 2, 4, 4>;   // the same 128 features of dh
-// The grouped bf16 rows: a segment per expert leaves few large tiles (16
-// experts of 375 rows: 40 row tiles of 256), so 128 rows x 64 features on rings of
-// four LDS stages (that case, hidden 2048, 256 features: 80 -> 252 workgroups,
-// 127 -> 52 us).
+// Grouped bf16 rows in few segments: 128 rows x 64 features on rings of four LDS
+// stages (swiglu_bwd_small_tiles says when).
 using ShapeBwdGroupGU = RingGateUp128<false>;
 using ShapeBwdGroupDH = TileShape<128, 64, 4, 2, 4, 4>;
 
@@ -913,6 +911,26 @@ static int swiglu_bwd_kind(const SwigluBwdArgs& a, int64_t assignments, hipStrea
 
 static int bwd_device_cus() { return current_device_cus(); }
 
+// Grouped bf16 rows: whether the 128 x 64 tiles take less time than the 256 x
+// 128 ones.  A workgroup of either holds a CU, so a launch takes whole rounds:
+// a round of large tiles 36 + 0.042 K us, one of small tiles (a quarter of the
+// work) 7.5 + 0.017 K.  Small tiles win while the large ones leave CUs idle
+// and lose where both fill them.  us large -> small, 16 experts x 256 features at
+// hidden 2048: 375 rows an expert 113 -> 53, 750 119 -> 98, 1024 119 / 121, 1536 122 /
+// 190, 2048 229 -> 227, 3000 257 / 258; at hidden 768: 375 66 -> 26, 1536 71 / 85, 4096
+// 201 -> 178; 8 experts x 128 features at hidden 512: 55 -> 17 at 750 rows, 114 -> 103
+// at 12288.  Of 67 measured launches this choice is never slower than the large
+// tiles and at most 7% behind the better one.
+static bool swiglu_bwd_small_tiles(const SwigluBwdArgs& a, int64_t assignments) {
+    const int64_t cus = bwd_device_cus();
+    auto rounds = [&](int64_t bm, int64_t bf) {
+        const int64_t tiles = ((assignments + bm - 1) / bm + a.E) * ((a.F - a.f_base + bf - 1) / bf);
+        return (tiles + cus - 1) / cus;
+    };
+    return rounds(ShapeBwdGU::BM, ShapeBwdDH::BN) * 5 * (860 + a.K) >=
+           rounds(ShapeBwdGroupGU::BM, ShapeBwdGroupDH::BN) * 2 * (450 + a.K);
+}
+
 // The persistent launch: 256-feature tiles over features [0, feats).
 static int launch_swiglu_bwd_pps(const SwigluBwdArgs& a, int64_t feats, hipStream_t stream) {
     const int64_t tiles_m = (a.M + 255) / 256;
@@ -954,7 +972,10 @@ int launch_swiglu_bwd(int act, const SwigluBwdArgs& a, int64_t assignments, hipS
     }
     if (act == TRMOE_BF16) {
         if (grouped)
-            return swiglu_bwd_kind<KindBF16, true, false, false, ShapeBwdGroupGU, ShapeBwdGroupDH>(a, assignments, stream);
+            return swiglu_bwd_small_tiles(a, assignments)
+                       ? swiglu_bwd_kind<KindBF16, true, false, false, ShapeBwdGroupGU, ShapeBwdGroupDH>(a, assignments,
+                                                                                                         stream)
+                       : swiglu_bwd_kind<KindBF16, true, false>(a, assignments, stream);
         if (routed) return swiglu_bwd_kind<KindBF16, false, true>(a, assignments, stream);
         return swiglu_bwd_kind<KindBF16, false, false>(a, assignments, stream);
     }

@@ -264,6 +264,41 @@ def test_routed_swiglu_backward_and_grouped_linear(gpu, dtype, E, k, W, n):
         assert _err(dxa[s0:s1], ref_dx) <= BOUND[dtype], e
 
 
+@pytest.mark.parametrize("H,E,W,n", [(2048, 16, 256, 5999), (2048, 16, 256, 12365), (2048, 16, 300, 8000),
+                                     (768, 16, 256, 12288), (512, 8, 128, 12288)])
+def test_routed_swiglu_backward_tile_choice(gpu, H, E, W, n):
+    """bf16 rows of enough tokens that either tile size may run them (the
+    second to fourth case take the large one): every row, empty and uneven
+    segments, features past the last whole tile."""
+    from complexity_amd import ops
+
+    print(f"routed_swiglu_backward tiles H={H} E={E} W={W} n={n}", flush=True)
+    g = torch.Generator(device=gpu).manual_seed(n)
+    rnd = lambda *s, k=1.0: (torch.randn(*s, generator=g, device=gpu) * k).bfloat16()  # noqa: E731
+    x, dout = rnd(n, H), rnd(n, H)
+    gate, up, down = rnd(E, H, W, k=H ** -0.5), rnd(E, H, W, k=H ** -0.5), rnd(E, W, H, k=W ** -0.5)
+    table = torch.stack([(torch.arange(50, device=gpu) ** 2 + j) % (E - 1) for j in range(2)])   # the last expert: none
+    ids = torch.randint(0, 50, (n,), generator=g, device=gpu)
+    srt, _, off, _ = ops.route_sort(ids, table, E)
+    egu, _ = ops.pack_expert_gate_up(gate, up)
+    dgu, hm = ops.routed_swiglu_backward(x, dout, srt, off, E, 2, egu, ops.pack_expert_down_t(down), W, (0.6, 0.4), 2.0)
+    dg, du = _split_dgu(dgu, -(-W // 64) * 64)
+    off = off.tolist()
+    assert off[E - 1] == off[E] == 2 * n
+    for e in range(E - 1):
+        rows = slice(off[e], off[e + 1])
+        if off[e] == off[e + 1]:
+            continue
+        t = srt[rows] % n
+        mult = torch.tensor((1.2, 0.8), dtype=torch.float64, device=gpu)[srt[rows] // n].unsqueeze(1)
+        want = O.swiglu_backward(x[t].double(), dout[t].double(), gate[e].T.double(), up[e].T.double(),
+                                 down[e].T.double(), mult)
+        for got, ref in zip((dg, du, hm), want):
+            # each row rounded to bf16 from fp32 sums of bf16 products: 2^-8 of its norm
+            err = (got[rows, :W].double() - ref).norm(dim=1) / ref.norm(dim=1).clamp_min(1e-9)
+            assert float(err.max()) <= 2.0 ** -8, (e, float(err.max()))
+
+
 # --------------------------------------------------------------------------- layer
 
 
