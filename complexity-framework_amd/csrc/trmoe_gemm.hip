@@ -1399,6 +1399,20 @@ bool gate_up_rms_inline(int act, int64_t M, int64_t packed_rows) {
            (packed_rows % 256 == 0 && tiles_of(M, 128, packed_rows, 256) <= cus);
 }
 
+// Whether an f32 launch without expert columns is shorter on 64x128 ring tiles
+// (two workgroups per CU) than on the 128x128 register-staged ones: fewer
+// half-rounds of the one than of the other; while 128x128 tiles leave CUs idle,
+// the two-stage 64x128 tiles take its place, as fast at K = 768 and above and
+// 3-8% faster below.  us 128x128 -> ring, K = 896, 6144 rows: 1300 tokens 178 -> 124,
+// 2048 180 / 185, 3001 292 -> 275, 4096 352 / 366; K = 256, 2048 rows: 512 tokens 12.5 /
+// 13.6, 2600 39 -> 32, 8192 76 / 79; K = 4096, 28672 rows: 129 tokens 521 -> 415, 1024 1809 /
+// 1882.
+static bool f32_ring(int64_t M, int64_t K, int64_t rows) {
+    const int64_t cus = device_cus(), t64 = tiles_of(M, 64, rows, 128), t128 = tiles_of(M, 128, rows, 128);
+    if (t128 < cus) return K >= 768;
+    return (t64 + cus - 1) / cus < 2 * ((t128 + cus - 1) / cus);
+}
+
 // Launches of at most one round of workgroups (shared and expert columns
 // together): the smallest tile whose grid still fits the CUs once, because a
 // workgroup's time is its K stages and does not shrink with fewer of them.
@@ -1408,8 +1422,9 @@ bool gate_up_rms_inline(int act, int64_t M, int64_t packed_rows) {
 // hidden 2048, 11264 rows: 130 tokens 25.6 -> 20.6, 512 39.2 -> 31.4.  At the
 // next size up the 256-row ping-pong tiles are as fast (777 tokens of that
 // layer: 46.9 against 60.4 on 128x256).  128 tokens of the 200M layer on 64x64
-// tiles of two K groups: 9.3 -> 6.9.  f32 takes 64x128 throughout: its
-// MFMAs bound the stage (2048 tokens 252 -> 216 with the merged launch).
+// tiles of two K groups: 9.3 -> 6.9.  f32 takes 64x128, whose stages its MFMAs
+// bound: always with expert columns (2048 tokens 252 -> 216 with the merged
+// launch), else where f32_ring says.
 // Returns whether it took the launch.
 template <class Kind, bool FP8, bool SAVE>
 static bool launch_gate_up_ring(const GateUpArgs& a, int64_t packed_rows, hipStream_t stream, int& st) {
@@ -1424,6 +1439,7 @@ static bool launch_gate_up_ring(const GateUpArgs& a, int64_t packed_rows, hipStr
     };
     if constexpr (std::is_same_v<Kind, KindF32>) {
         if (tiles_of(a.M, 256, rows, 256) >= kBigTileMinBlocks) return false;
+        if (a.ids == nullptr && !f32_ring(a.M, a.K, rows)) return false;
         st = run(RingGateUp64<false>{});
         return true;
     } else {
