@@ -1390,11 +1390,14 @@ static int launch_gate_up_ring_shape(const GateUpArgs& a, int64_t rows, hipStrea
     return check_launch(ROUTED ? "dense_routed_gate_up" : "shared_gate_up");
 }
 
-// The shape rule of launch_gate_up_ring (bf16 / f32).
+// The shape rule of launch_gate_up_ring (bf16 / f32).  f32 only up to one round
+// (two workgroups per CU): the squares delay every stage, a launch for the
+// scales costs the same at any size (4-6 us; in the kernel 3 us at 512 tokens of
+// the 200M layer, 8 at 1300, 18 at 4096).
 bool gate_up_rms_inline(int act, int64_t M, int64_t packed_rows) {
     const int64_t cus = device_cus();
     if (M <= 0 || packed_rows % 128 != 0) return false;
-    if (act == TRMOE_F32) return tiles_of(M, 256, packed_rows, 256) < kBigTileMinBlocks;
+    if (act == TRMOE_F32) return tiles_of(M, 64, packed_rows, 128) <= 2 * cus;
     return tiles_of(M, 64, packed_rows, 128) <= cus || tiles_of(M, 128, packed_rows, 128) <= cus ||
            (packed_rows % 256 == 0 && tiles_of(M, 128, packed_rows, 256) <= cus);
 }
