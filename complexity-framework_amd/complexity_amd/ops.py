@@ -652,6 +652,7 @@ def decode_attention(x: torch.Tensor, norm_weight: torch.Tensor, norm_eps: float
     return attn
 
 
+@_on_tensor_device
 def decode_linear(x: torch.Tensor, weight: torch.Tensor, residual: Optional[torch.Tensor] = None) -> torch.Tensor:
     """x [n, K] . weight^T (+ residual) for n <= SKINNY_MAX_TOKENS rows and an
     nn.Linear weight [N, K] with N % 32 == 0, K % 8 == 0, on the decode down kernel."""

@@ -321,3 +321,11 @@ def test_logits_under_function_transforms():
             look(mode.from_tensor(h))
         make_fx(look)(h)
     assert seen == [True, False, False, False, False]
+
+
+@pytest.mark.parametrize("name", ["qk_norm_rope", "prefill_attention", "decode_attention", "decode_linear",
+                                  "decoder_step", "rmsnorm_forward", "layer_forward"])
+def test_calls_of_the_decoder_run_on_their_tensors_device(name):
+    """The library launches on the current device: what the decoder calls by
+    itself makes the tensors' GPU current."""
+    assert hasattr(getattr(ops, name), "__wrapped__")
