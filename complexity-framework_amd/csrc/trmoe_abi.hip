@@ -962,7 +962,10 @@ int trmoe_qk_norm_rope(const void* kqv, int64_t sequences, int64_t tokens, int n
     TRMOE_REQUIRE(aligned16(kqv) && ldkqv % 8 == 0 && aligned16(q_weight) && aligned16(k_weight) && aligned16(q) &&
                       aligned16(k_cache) && aligned16(v_cache),
                   "qk_norm_rope: operands must be 16-byte aligned, ldkqv a multiple of 8");
-    TRMOE_REQUIRE(sequences * tokens * (num_heads + 2 * num_kv_heads) < (int64_t)1 << 36, "qk_norm_rope: too many rows");
+    // 8 threads per head row, 2^32 along the grid's x
+    TRMOE_REQUIRE(sequences < (int64_t)1 << 29 && tokens < (int64_t)1 << 29 &&
+                      sequences * tokens < ((int64_t)1 << 29) / (num_heads + 2 * num_kv_heads),
+                  "qk_norm_rope: too many rows");
     RopeArgs a{};
     a.kqv = static_cast<const bf16_t*>(kqv);
     a.ldkqv = ldkqv;
@@ -990,7 +993,9 @@ int trmoe_prefill_attention(const void* q, const void* k_cache, const void* v_ca
     TRMOE_REQUIRE(sequences >= 0 && tokens >= 0 && num_heads > 0 && num_kv_heads > 0 && num_heads % num_kv_heads == 0,
                   "prefill_attention: bad dimensions");
     TRMOE_REQUIRE(tokens <= cache_length && tokens < (int64_t)1 << 23, "prefill_attention: tokens past the cache or 2^23");
-    TRMOE_REQUIRE(sequences * num_heads < 65536, "prefill_attention: sequences * num_heads must be below 65536");
+    // 256 threads per workgroup, 2^32 along the grid's x
+    TRMOE_REQUIRE(sequences < (int64_t)1 << 24 && sequences * num_heads < (int64_t)1 << 24,
+                  "prefill_attention: sequences * num_heads must be below 2^24");
     if (sequences == 0 || tokens == 0) return TRMOE_OK;
     TRMOE_REQUIRE(q && k_cache && v_cache && out, "prefill_attention: null pointer");
     TRMOE_REQUIRE(aligned16(q) && aligned16(k_cache) && aligned16(v_cache) && aligned16(out),

@@ -93,3 +93,13 @@ def test_rmsnorm_workspace_and_validation_without_a_device(lib):
     st = lib.trmoe_rmsnorm_backward(bf, None, 16, 896, 896, None, None, None, 896, None, 0, None, 896, None,
                                     None, 0, None)
     assert st == _native.ERR_INVALID
+
+
+def test_prefill_attention_takes_many_prompts(lib):
+    """The heads lie along the launch grid's x, whose limit is 2^32 threads:
+    5000 prompts of 14 heads are refused for their null pointers alone."""
+    def call(sequences, heads, scale=0.125):
+        return lib.trmoe_prefill_attention(None, None, None, sequences, 2, heads, heads, 64, scale, None, None)
+
+    assert call(5000, 14) == _native.ERR_INVALID and b"null" in lib.trmoe_last_error()
+    assert call((1 << 24) // 16, 16) == _native.ERR_INVALID and b"null" not in lib.trmoe_last_error()

@@ -133,3 +133,14 @@ def test_decode_linear_adds_residual(gpu):
         w = (torch.randn(896, 896, generator=g) * 0.03).to(gpu).bfloat16()
         r = torch.randn(n, 896, generator=g).to(gpu).bfloat16()
         assert _rel(ops.decode_linear(x, w, r), F.linear(x.float(), w.float()) + r.float()) <= 2.0 ** -8
+
+
+def test_prefill_attention_of_many_prompts(gpu):
+    # more (prompt, head) pairs than 65535: the first, middle and last prompts
+    B, T, heads, kvh, L = 4700, 3, 14, 2, 64
+    g = torch.Generator(device=gpu).manual_seed(0)
+    q = torch.randn(B, T, heads, D, generator=g, device=gpu).bfloat16()
+    kc, vc = (torch.randn(B, kvh, L, D, generator=g, device=gpu).bfloat16() for _ in range(2))
+    got = ops.prefill_attention(q, kc, vc, 0.125).view(B, T, heads, D)
+    for b in (0, 2340, 4680, 4681, 4699):
+        assert torch.equal(got[b], ops.prefill_attention(q[b:b + 1], kc[b:b + 1], vc[b:b + 1], 0.125).view(T, heads, D))
