@@ -467,7 +467,8 @@ class TRGQADecoder(nn.Module):
             if not (_plain(m["input_layernorm"], RMSNorm, H) and _plain(a["q_norm"], RMSNorm, D)
                     and _plain(a["k_norm"], RMSNorm, D) and _plain(a["o_proj"], nn.Linear, H, cfg.num_heads * D)):
                 return False
-            if a["q_norm"].eps != a["k_norm"].eps:   # the kernels norm both with one
+            # the kernels norm q and k with one eps, and take a positive scale
+            if a["q_norm"].eps != a["k_norm"].eps or not attn.scale > 0:
                 return False
         return True
 

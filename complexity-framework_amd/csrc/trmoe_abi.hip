@@ -7,6 +7,7 @@
 #include <atomic>
 #include <mutex>
 #include <set>
+#include <cmath>
 #include <string>
 #include <utility>
 
@@ -996,6 +997,8 @@ int trmoe_prefill_attention(const void* q, const void* k_cache, const void* v_ca
     // 256 threads per workgroup, 2^32 along the grid's x
     TRMOE_REQUIRE(sequences < (int64_t)1 << 24 && sequences * num_heads < (int64_t)1 << 24,
                   "prefill_attention: sequences * num_heads must be below 2^24");
+    // the kernel's running maximum is that of the unscaled scores
+    TRMOE_REQUIRE(scale > 0.0f && std::isfinite(scale), "prefill_attention: scale must be positive and finite");
     if (sequences == 0 || tokens == 0) return TRMOE_OK;
     TRMOE_REQUIRE(q && k_cache && v_cache && out, "prefill_attention: null pointer");
     TRMOE_REQUIRE(aligned16(q) && aligned16(k_cache) && aligned16(v_cache) && aligned16(out),

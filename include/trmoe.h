@@ -419,7 +419,7 @@ int trmoe_pack_fragments(int dtype, const void* packed, int64_t rows, int64_t co
  * first_position + t (+ *position, a device counter, when given; a position
  * past the cache is dropped).
  *
- * trmoe_prefill_attention: softmax(scale q K^T) V of a prompt, token t over
+ * trmoe_prefill_attention: softmax(scale q K^T) V (scale > 0) of a prompt, token t over
  * positions 0 .. t of the caches (trmoe_qk_norm_rope's outputs with
  * first_position 0), into out [sequence, token, num_heads * 64].
  *

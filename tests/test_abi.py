@@ -103,3 +103,10 @@ def test_prefill_attention_takes_many_prompts(lib):
 
     assert call(5000, 14) == _native.ERR_INVALID and b"null" in lib.trmoe_last_error()
     assert call((1 << 24) // 16, 16) == _native.ERR_INVALID and b"null" not in lib.trmoe_last_error()
+
+
+@pytest.mark.parametrize("scale", [0.0, -0.125, float("nan"), float("inf")])
+def test_prefill_attention_refuses_a_scale_that_is_not_positive(lib, scale):
+    """The running maximum is kept on the unscaled scores."""
+    assert lib.trmoe_prefill_attention(None, None, None, 1, 2, 2, 2, 64, scale, None, None) == _native.ERR_INVALID
+    assert b"scale" in lib.trmoe_last_error()

@@ -329,3 +329,10 @@ def test_calls_of_the_decoder_run_on_their_tensors_device(name):
     """The library launches on the current device: what the decoder calls by
     itself makes the tensors' GPU current."""
     assert hasattr(getattr(ops, name), "__wrapped__")
+
+
+@pytest.mark.parametrize("scale,takes", [(0.0, False), (-0.125, False), (0.25, True)])
+def test_attention_scale_that_is_not_positive_takes_the_general_path(scale, takes):
+    m = _decoder()
+    m.layers[1].self_attn.scale = scale
+    assert m._hip_attention(CUDA) is takes
