@@ -16,4 +16,11 @@ __host__ __device__ inline int64_t mapped_dest(int64_t off, int64_t idx, int64_t
     return (d >= 0 && d < out_elems) ? d : -1;
 }
 
+// Index of one element of a K split's fp32 partial: the splits' [rows, cols]
+// planes follow each other, so it passes 32 bits at sizes whose rows * cols does
+// not.
+__host__ __device__ inline int64_t split_index(int64_t split, int64_t rows, int64_t cols, int64_t row, int64_t col) {
+    return (split * rows + row) * cols + col;
+}
+
 }  // namespace trmoe

@@ -20,6 +20,7 @@
 #include "trmoe_common.h"
 #include "trmoe_internal.h"
 #include "trmoe_gemm.h"
+#include "trmoe_map.h"
 #include "trmoe_skinny.h"
 
 #include <stdlib.h>
@@ -389,7 +390,7 @@ __global__ __launch_bounds__(64 * NW) void k_down_skinny(DownArgs a, float* part
     __syncthreads();
 
     const bool single = splits == 1;
-    float* dst = part + (int64_t)split * a.M * a.N;
+    float* dst = part + split_index(split, a.M, a.N, 0, 0);
     for (int qi = threadIdx.x; qi < MT * NU * 4 * 64; qi += NT) {
         const int l = qi & 63, i = (qi >> 6) & 3, u = (qi >> 8) % NU, tm = (qi >> 8) / NU;
         const int row = tm * 16 + 4 * (l >> 4) + i;
@@ -407,16 +408,15 @@ __global__ __launch_bounds__(64 * NW) void k_down_skinny(DownArgs a, float* part
     // the last split of the column tile sums them all, in split order: a
     // round trip to memory instead of a launch (4.6 us at 64 tokens)
     if (!last_arrival(a.counters + ct, splits)) return;
-    const int plane = (int)a.M * (int)a.N;
     for (int qi = threadIdx.x; qi < (int)a.M * kCols; qi += NT) {
         const int row = qi / kCols, col = (int)n0 + qi % kCols;
         if (col >= a.N) continue;
-        const float* p = part + row * (int)a.N + col;
         float s = 0.f;
         for (int sp = 0; sp < splits; sp += 4) {
             float t[4];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) t[j] = load_dev(p + (sp + j < splits ? sp + j : splits - 1) * plane);
+            for (int j = 0; j < 4; ++j)
+                t[j] = load_dev(part + split_index(sp + j < splits ? sp + j : splits - 1, a.M, a.N, row, col));
 #pragma unroll
             for (int j = 0; j < 4; ++j) s += sp + j < splits ? t[j] : 0.f;
         }
@@ -432,23 +432,22 @@ __global__ __launch_bounds__(64 * NW) void k_down_skinny(DownArgs a, float* part
 template <class T, int V>
 __global__ __launch_bounds__(256) void k_down_reduce(DownArgs a, const float* part, int splits) {
     // V consecutive columns per thread (16-byte partial loads when V = 4);
-    // the launcher keeps M * N below 2^31, so every index fits an int
+    // the launcher keeps M * N below 2^31, so a row and column fit an int
     const int nv = (int)a.N / V;
     const int idx = (int)blockIdx.x * 256 + (int)threadIdx.x;
     if (idx >= (int)a.M * nv) return;
     const int row = idx / nv, c0 = (idx - row * nv) * V;
-    const int plane = (int)a.M * (int)a.N;
-    const float* p = part + row * (int)a.N + c0;
+    auto at = [&](int sp) { return part + split_index(sp, a.M, a.N, row, c0); };
     using VT = typename std::conditional<V == 4, f32x4, float>::type;
     VT acc{};
     int sp = 0;
     for (; sp + 2 <= splits; sp += 2) {   // two partials in flight; the sum keeps split order
-        const VT v0 = *reinterpret_cast<const VT*>(p + sp * plane);
-        const VT v1 = *reinterpret_cast<const VT*>(p + (sp + 1) * plane);
+        const VT v0 = *reinterpret_cast<const VT*>(at(sp));
+        const VT v1 = *reinterpret_cast<const VT*>(at(sp + 1));
         acc += v0;
         acc += v1;
     }
-    for (; sp < splits; ++sp) acc += *reinterpret_cast<const VT*>(p + sp * plane);
+    for (; sp < splits; ++sp) acc += *reinterpret_cast<const VT*>(at(sp));
     if constexpr (V == 4) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) down_finish<T>(a, row, c0 + j, acc[j]);
