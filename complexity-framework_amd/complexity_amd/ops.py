@@ -1017,6 +1017,12 @@ class PackedLayer:
                 return True
         return False
 
+    @property
+    def wholly_e4m3(self) -> bool:
+        """True when every weight of a grouped layer holds e4m3 codes."""
+        ws = (self.expert_gate_up, self.expert_down) + ((self.shared_gate_up, self.shared_down) if self.shared_width else ())
+        return all(w is not None and w.dtype == torch.float8_e4m3fn for w in ws)
+
     def fragments(self, name: str, cols: int):
         """pack_fragments of the bf16/f32 weight `name` (None for fp8)."""
         if self.act_dtype not in (torch.bfloat16, torch.float32):
@@ -1101,7 +1107,7 @@ def layer_forward(x: torch.Tensor, token_ids: torch.Tensor, route_table: torch.T
         out = shared_down_combine(h, packed.dense_features, packed.dense_down, None, hidden, None, None,
                                   top_k, route_weights, 1.0, 1.0, residual)
         return (out, gu, h) if save else out
-    if decode and rscale is None and x.dtype == torch.bfloat16 and packed.expert_gate_up.dtype == torch.float8_e4m3fn:
+    if decode and rscale is None and x.dtype == torch.bfloat16 and packed.wholly_e4m3:
         return e4m3_decode_layer(x, token_ids, route_table, packed, route_weights, shared_scale, routed_scale, residual)
     sorted_idx, inverse, offsets, _ = route_sort(token_ids, route_table, packed.num_experts, order)
     y = routed_experts(x, sorted_idx, offsets, packed.num_experts, top_k, packed.expert_gate_up,
