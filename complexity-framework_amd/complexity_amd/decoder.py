@@ -330,8 +330,11 @@ class _StepPlan:
                     return None   # parametrized: kqv_weight() materialises it per call
                 plan._weight(attn._modules[n], "weight")
             kqv = attn.kqv_weight()
-            gu = packed.fragments("dense_gate_up", cfg.hidden_size)[0]
-            dn = packed.fragments("dense_down", packed.dense_features)[0]
+            frags = packed.fragments("dense_gate_up", cfg.hidden_size), packed.fragments("dense_down",
+                                                                                         packed.dense_features)
+            if None in frags:
+                return None   # a graph records, and nothing has built them before
+            gu, dn = frags[0][0], frags[1][0]
             ptrs = (plan._weight(norm_in, "weight"), kqv, plan._weight(plan._watch(attn, "q_norm"), "weight"),
                     plan._weight(plan._watch(attn, "k_norm"), "weight"),
                     plan._weight(plan._watch(attn, "o_proj"), "weight"), *caches, gu, dn, table)

@@ -13,6 +13,7 @@ from __future__ import annotations
 
 import ctypes
 import functools
+import threading
 from dataclasses import dataclass, field
 from typing import Optional, Sequence, Tuple
 
@@ -977,6 +978,28 @@ def choose_strategy(shared_width: int, num_experts: int, expert_width: int, top_
     return STRATEGY_DENSE if extra <= 0.08 * useful else STRATEGY_GROUPED
 
 
+_COPY_LOCK = threading.Lock()
+
+
+def _decode_copy(weight: torch.Tensor, have, build, keep):
+    """`have()`, or what `build()` makes and `keep` stores: a pack's copy for the
+    decode kernels, built by the first call that wants it and complete before
+    any other call, thread, stream or graph finds it.  None while a graph
+    records and there is no copy yet: one built there would lie in the graph's
+    memory and hold nothing before its first replay, so that call is recorded
+    on the packs themselves."""
+    got = have()
+    if got is not None or torch.cuda.is_current_stream_capturing():
+        return got
+    with _COPY_LOCK:
+        got = have()
+        if got is None:
+            got = build()
+            torch.cuda.current_stream(weight.device).synchronize()
+            keep(got)
+    return got
+
+
 @dataclass
 class PackedLayer:
     """Weights of one layer in kernel layout (built by TRHashEngine)."""
@@ -1003,10 +1026,10 @@ class PackedLayer:
 
     e4m3_frag: Optional[E4M3Decode] = None           # decode copy of an e4m3 layer, built on first use
 
-    def e4m3_decode(self, hidden: int) -> E4M3Decode:
-        if self.e4m3_frag is None:
-            self.e4m3_frag = pack_e4m3_decode(self, hidden)
-        return self.e4m3_frag
+    def e4m3_decode(self, hidden: int) -> Optional[E4M3Decode]:
+        """pack_e4m3_decode of a layer wholly in e4m3 (None: _decode_copy)."""
+        return _decode_copy(self.expert_gate_up, lambda: self.e4m3_frag, lambda: pack_e4m3_decode(self, hidden),
+                            lambda c: setattr(self, "e4m3_frag", c))
 
     @property
     def fp8(self) -> bool:
@@ -1024,17 +1047,14 @@ class PackedLayer:
         return all(w is not None and w.dtype == torch.float8_e4m3fn for w in ws)
 
     def fragments(self, name: str, cols: int):
-        """pack_fragments of the bf16/f32 weight `name` (None for fp8)."""
+        """pack_fragments of the bf16/f32 weight `name` (None for fp8, and see _decode_copy)."""
         if self.act_dtype not in (torch.bfloat16, torch.float32):
             return None
         w = getattr(self, name)
         if w is None or w.dtype != self.act_dtype:
             return None
-        got = self.frag.get(name)
-        if got is None:
-            got = pack_fragments(w, cols)
-            self.frag[name] = got
-        return got
+        return _decode_copy(w, lambda: self.frag.get(name), lambda: pack_fragments(w, cols),
+                            lambda c: self.frag.__setitem__(name, c))
 
 
 def fp8_activation_mode(mode):
@@ -1107,7 +1127,8 @@ def layer_forward(x: torch.Tensor, token_ids: torch.Tensor, route_table: torch.T
         out = shared_down_combine(h, packed.dense_features, packed.dense_down, None, hidden, None, None,
                                   top_k, route_weights, 1.0, 1.0, residual)
         return (out, gu, h) if save else out
-    if decode and rscale is None and x.dtype == torch.bfloat16 and packed.wholly_e4m3:
+    if (decode and rscale is None and x.dtype == torch.bfloat16 and packed.wholly_e4m3
+            and packed.e4m3_decode(hidden) is not None):
         return e4m3_decode_layer(x, token_ids, route_table, packed, route_weights, shared_scale, routed_scale, residual)
     sorted_idx, inverse, offsets, _ = route_sort(token_ids, route_table, packed.num_experts, order)
     y = routed_experts(x, sorted_idx, offsets, packed.num_experts, top_k, packed.expert_gate_up,

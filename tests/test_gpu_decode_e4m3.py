@@ -11,6 +11,7 @@ import pytest
 import torch
 import torch.nn.functional as F
 
+from complexity_amd import ops
 from complexity_amd.tr_hash import TRHashEngine, TRHashEngineConfig
 
 pytestmark = pytest.mark.gpu
@@ -87,3 +88,36 @@ def test_unrouted_overflow_stays_out(gpu):
         out = e(x, ids).float().view(40, -1)
     assert not torch.isfinite(out[:25]).all()
     assert torch.isfinite(out[25:]).all()
+
+
+def test_graph_recorded_before_any_decode(gpu):
+    """A decode call recorded after prompts alone, without a warm-up: eager calls
+    before the first replay, between replays and after the graph is gone give
+    what they gave without it, and so does every replay."""
+    shape, n = "scaled", 32
+    g = torch.Generator().manual_seed(0)
+    H = SHAPES[shape][0]
+    x = torch.randn(n, 1, H, generator=g).to(gpu).bfloat16()
+    ids = torch.randint(0, 500, (n, 1), generator=g).to(gpu)
+    e, other = _engine(shape, gpu), _engine(shape, gpu)
+    other.load_state_dict(e.state_dict())
+    with torch.no_grad():
+        prompt = torch.randn(1, 300, H, generator=g).to(gpu).bfloat16()
+        e(prompt, torch.zeros(1, 300, dtype=torch.int64, device=gpu))
+        scope = ops.workspace_scope()
+        graph = torch.cuda.CUDAGraph()
+        with scope, torch.cuda.graph(graph):
+            recorded = e(x, ids)
+        want = other(x, ids)          # fused, its copy built eagerly
+        ref = _reference(e, x.view(-1, H), ids, None)
+        assert torch.equal(e(x, ids), want)
+        for _ in range(3):
+            graph.replay()
+            assert torch.equal(e(x, ids), want)
+            # the grouped kernels round the experts' outputs to bf16 once more than the fused ones: 2^-8 each
+            err = (recorded.view(-1, H).float() - ref).norm(dim=1) / ref.norm(dim=1)
+            assert float(err.max()) <= 2.0 ** -7
+        del graph, recorded
+        torch.cuda.synchronize()
+        torch.cuda.empty_cache()
+        assert torch.equal(e(x, ids), want)
