@@ -452,6 +452,76 @@ def test_c2_bf16_layer_backward_full_size(gpu):
     _check(got, ref, "bf16")
 
 
+def test_c2_training_step_every_row_and_repeatable_with_cold_caches(gpu):
+    """The training forward and backward at the C2 shape (16384 tokens): all 6656
+    columns of the saved g|u, every row of h and of dx, and each of the six
+    weight gradients against float64, and equal bit for bit over calls
+    separated by a cache-evicting write (a row that is lost now and then moves a
+    token-summed gradient by 1/128 of its norm at most)."""
+    from complexity_amd import ops
+    from complexity_amd import workloads as W
+
+    w = W.C2
+    eng = W.build_engine(w, gpu, backend="hip")
+    p = eng._hip_packed()
+    x = W.make_hidden(w).to(gpu).to(torch.bfloat16).reshape(-1, w.hidden).contiguous()
+    ids = W.make_token_ids(w).to(gpu).reshape(-1).contiguous()
+    n, H, S, E, Wd, F_ = x.shape[0], w.hidden, p.shared_width, p.num_experts, p.expert_width, p.dense_features
+    table, rw, ss, rs = eng._active_route_table, eng.config.route_weights, 0.5, 2.0
+    dout = (torch.randn(n, H, generator=torch.Generator(device=gpu).manual_seed(3), device=gpu) * 0.1).bfloat16()
+    wt = {k: getattr(eng, k).detach() for k in ("expert_gate", "expert_up", "expert_down")}
+    wt |= {k: getattr(eng, k).weight.detach() for k in ("shared_gate", "shared_up", "shared_down")}
+    bwd = ops.backward_packs(p, H, wt["shared_down"], wt["expert_down"])
+    evict = torch.empty(1 << 28, dtype=torch.float32, device=gpu)   # 1 GiB: more than L2 and MALL together
+    first = None
+    for call in range(6):
+        evict.add_(1.0)
+        _, gu, h = ops.layer_forward(x, ids, table, p, rw, ss, rs, save=True)
+        evict.add_(1.0)
+        dx, grads = ops.layer_backward(dout, x, ids, table, p, bwd, rw, ss, rs, saved_gu=gu, saved_h=h)
+        got = {"gu": gu, "h": h, "dx": dx, **grads}
+        if first is None:
+            first = {k: v.clone() for k, v in got.items()}
+        for k, v in got.items():
+            assert torch.equal(v.contiguous().view(torch.int16), first[k].contiguous().view(torch.int16)), (call, k)
+    del got, gu, h, dx, grads, evict
+
+    # float64, one block of features at a time: the shared branch, then each expert
+    xd, dd = x.double(), dout.double()
+    routes = table[:, ids]
+    dx_ref = torch.zeros(n, H, dtype=torch.float64, device=gpu)
+    packed = first["gu"].view(n, F_ // 32, 2, 32)
+
+    def rows(name, got, ref, bound):
+        err = (got.double() - ref).norm(dim=1) / ref.norm(dim=1).clamp_min(1e-9)
+        assert float(err.max()) <= bound, (name, int(err.argmax()), float(err.max()))
+
+    blocks = [(None, 0, S)] + [(e, S + e * Wd, Wd) for e in range(E)]
+    for e, f0, width in blocks:
+        if e is None:
+            wg, wu, wd = (wt[k].double() for k in ("shared_gate", "shared_up", "shared_down"))
+            mult = torch.full((n, 1), ss, dtype=torch.float64, device=gpu)
+        else:
+            wg, wu, wd = (wt[k][e].double().T for k in ("expert_gate", "expert_up", "expert_down"))
+            mult = sum(rs * rw[j] * (routes[j] == e).double() for j in range(routes.shape[0])).unsqueeze(1)
+        cols = slice(f0, f0 + width)
+        g, u = xd @ wg.T, xd @ wu.T
+        rows("g", packed[:, :, 0].reshape(n, -1)[:, cols], g, 2.0 ** -8)   # one rounding to bf16
+        rows("u", packed[:, :, 1].reshape(n, -1)[:, cols], u, 2.0 ** -8)
+        sg = torch.sigmoid(g)
+        hd = mult * g * sg * u
+        rows("h", first["h"][:, cols], hd, 2.0 ** -8)
+        dh = mult * (dd @ wd)
+        dg, du = dh * u * (sg + g * sg * (1 - sg)), dh * g * sg
+        dx_ref += dg @ wg + du @ wu
+        # bf16 g|u, dg|du and h (2^-9 each, averaging out over the tokens) and the output's rounding
+        name = (lambda k: first["shared_" + k]) if e is None else (lambda k: first["expert_" + k][e].T)
+        rows("dgate", name("gate"), dg.T @ xd, 2.0 ** -6)
+        rows("dup", name("up"), du.T @ xd, 2.0 ** -6)
+        rows("ddown", name("down"), dd.T @ hd, 2.0 ** -6)
+    rows("dx", first["dx"], dx_ref, 2.0 ** -6)
+
+
 @pytest.mark.parametrize("strategy", ["dense", "grouped"])
 @pytest.mark.parametrize("tokens", [2048, 8192])
 def test_c2_shape_layer_backward_mid_sizes(gpu, strategy, tokens):

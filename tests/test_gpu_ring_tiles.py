@@ -56,6 +56,10 @@ def test_gate_up_routed(gpu, n, H, S, E, W, dtype):
     packed = saved.view(n, -1, 2, 32)
     assert _rel(packed[:, :, 0].reshape(n, -1)[:, :S], _matmul(x, sg)) <= _bound(dtype)
     assert _rel(packed[:, :, 1].reshape(n, -1)[:, :S], _matmul(x, su)) <= _bound(dtype)
+    for e in range(E):   # the expert columns are saved raw, whatever the token's routes
+        cols = slice(S + e * W, S + (e + 1) * W)
+        assert _rel(packed[:, :, 0].reshape(n, -1)[:, cols], _matmul(x, eg[e].t())) <= _bound(dtype)
+        assert _rel(packed[:, :, 1].reshape(n, -1)[:, cols], _matmul(x, eu[e].t())) <= _bound(dtype)
 
 
 @pytest.mark.parametrize("kind", ["bf16", "f32", "e4m3"])
