@@ -475,11 +475,11 @@ __device__ __forceinline__ void gate_up_epi_direct_routed(const GateUpArgs& a, c
 
 // gate|up + SwiGLU over bf16 activations and weights, K a multiple of 64.
 // ROUTED: the launch covers dense-routed expert columns (route gather and
-// per-token expert weights for the tiles that hold them).  TMW = 4: 256-row
-// tiles, the only ones launched.  SAVE: also write the raw gate|up outputs to
-// a.gu (training forward).
-template <bool ROUTED, int TMW, bool SAVE = false, bool FP8 = false>
+// per-token expert weights for the tiles that hold them), 256-row tiles.  SAVE:
+// also write the raw gate|up outputs to a.gu (training forward).
+template <bool ROUTED, bool SAVE = false, bool FP8 = false>
 __global__ __launch_bounds__(512, 1) void k_gate_up_pp(GateUpArgs a) {
+    constexpr int TMW = 4;
     using Shape = ShapePP<TMW>;
     using Kind = KindBF16;
     constexpr int BM = Shape::BM;
@@ -526,9 +526,9 @@ __global__ __launch_bounds__(512, 1) void k_gate_up_pp(GateUpArgs a) {
     using Lay = std::conditional_t<FP8, PPLayoutF8<TMW>, PPLayoutK<TMW>>;
     // bf16 weights without row scales: each group stores its h rows straight
     // from the accumulators (group 0 while group 1 multiplies the last
-    // stage); otherwise, and for the saving 256-row tiles (whose registers
-    // would spill), through the LDS tile
-    const bool direct = !FP8 && (TMW == 2 || !SAVE) && a.row_scale == nullptr;
+    // stage); otherwise, and when saving (the registers would spill), through
+    // the LDS tile
+    const bool direct = !FP8 && !SAVE && a.row_scale == nullptr;
     pp_main<TMW, Lay>(ap, bp, a.K / 64, lds, group, wm0, wn0, acc, [&](const f32x16 (&c)[TMW][2]) {
         if (direct) {
             if constexpr (ROUTED)
@@ -1618,14 +1618,14 @@ static bool pp_eligible(int act, int wdt, const GateUpArgs& a, int64_t packed_ro
            ((a.M + 255) / 256) * (cols / 256) >= kPPGateUpMinBlocks;
 }
 
-template <bool ROUTED, int TMW, bool SAVE, bool FP8>
+template <bool ROUTED, bool SAVE, bool FP8>
 static int launch_gate_up_pp_shape(const GateUpArgs& a, int64_t packed_rows, hipStream_t stream) {
-    constexpr int BM = ShapePP<TMW>::BM;
+    constexpr int TMW = 4, BM = ShapePP<TMW>::BM;
     const dim3 grid((unsigned)((a.M + BM - 1) / BM), (unsigned)((packed_rows - a.n_base) / 256));
     using Lay = std::conditional_t<FP8, PPLayoutF8<TMW>, PPLayoutK<TMW>>;
     constexpr int kEpi = BM * (128 * 2 + 16);                // the SwiGLU tile, over the stages
     constexpr int kLds = 2 * Lay::kStage > kEpi ? 2 * Lay::kStage : kEpi;
-    auto kern = k_gate_up_pp<ROUTED, TMW, SAVE, FP8>;
+    auto kern = k_gate_up_pp<ROUTED, SAVE, FP8>;
     const int st = ensure_lds(kern, kLds);
     if (st) return st;
     if (grid.x == 0 || grid.y == 0) return TRMOE_OK;
@@ -1696,13 +1696,13 @@ static int launch_gate_up_pp(const GateUpArgs& a, int64_t packed_rows, hipStream
     const bool head_routed = ROUTED && a.ids != nullptr && split > 2 * a.shared_feats;
     int st;
     if (head_routed)
-        st = launch_gate_up_pp_shape<ROUTED, 4, SAVE, FP8>(a, split, stream);
+        st = launch_gate_up_pp_shape<ROUTED, SAVE, FP8>(a, split, stream);
     else if (a.row_scale == nullptr)
         st = launch_gate_up_pps<SAVE, FP8>(a, split, stream);
     else if constexpr (!FP8 && !SAVE)
         st = launch_gate_up_pps<false, false, true>(a, split, stream);
     else
-        st = launch_gate_up_pp_shape<false, 4, SAVE, FP8>(a, split, stream);
+        st = launch_gate_up_pp_shape<false, SAVE, FP8>(a, split, stream);
     if (st || tail == 0) return st;
     GateUpArgs t = a;
     t.n_base = split;
