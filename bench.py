@@ -462,7 +462,7 @@ def c4_e2e(torch, dev, steps: int = 128, reps: int = 3):
         "decode_tokens_per_s": 8 / (step_ms * 1e-3),
         "decode_mlp_ms_per_step": mlp_step_ms,
         "decode_mlp_share": mlp_step_ms / step_ms,
-        "attention": "torch SDPA (flash causal prefill, memory-efficient masked decode)",
+        "attention": "hand-written HIP (causal flash prefill, split decode)",
     }
 
 
