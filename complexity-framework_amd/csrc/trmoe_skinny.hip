@@ -408,15 +408,16 @@ __global__ __launch_bounds__(64 * NW) void k_down_skinny(DownArgs a, float* part
     // the last split of the column tile sums them all, in split order: a
     // round trip to memory instead of a launch (4.6 us at 64 tokens)
     if (!last_arrival(a.counters + ct, splits)) return;
+    const int64_t plane = split_index(1, a.M, a.N, 0, 0);
     for (int qi = threadIdx.x; qi < (int)a.M * kCols; qi += NT) {
         const int row = qi / kCols, col = (int)n0 + qi % kCols;
         if (col >= a.N) continue;
+        const float* p = part + split_index(0, a.M, a.N, row, col);
         float s = 0.f;
         for (int sp = 0; sp < splits; sp += 4) {
             float t[4];
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-                t[j] = load_dev(part + split_index(sp + j < splits ? sp + j : splits - 1, a.M, a.N, row, col));
+            for (int j = 0; j < 4; ++j) t[j] = load_dev(p + (sp + j < splits ? sp + j : splits - 1) * plane);
 #pragma unroll
             for (int j = 0; j < 4; ++j) s += sp + j < splits ? t[j] : 0.f;
         }
@@ -437,17 +438,18 @@ __global__ __launch_bounds__(256) void k_down_reduce(DownArgs a, const float* pa
     const int idx = (int)blockIdx.x * 256 + (int)threadIdx.x;
     if (idx >= (int)a.M * nv) return;
     const int row = idx / nv, c0 = (idx - row * nv) * V;
-    auto at = [&](int sp) { return part + split_index(sp, a.M, a.N, row, c0); };
+    const int64_t plane = split_index(1, a.M, a.N, 0, 0);
+    const float* p = part + split_index(0, a.M, a.N, row, c0);
     using VT = typename std::conditional<V == 4, f32x4, float>::type;
     VT acc{};
     int sp = 0;
     for (; sp + 2 <= splits; sp += 2) {   // two partials in flight; the sum keeps split order
-        const VT v0 = *reinterpret_cast<const VT*>(at(sp));
-        const VT v1 = *reinterpret_cast<const VT*>(at(sp + 1));
+        const VT v0 = *reinterpret_cast<const VT*>(p + sp * plane);
+        const VT v1 = *reinterpret_cast<const VT*>(p + (sp + 1) * plane);
         acc += v0;
         acc += v1;
     }
-    for (; sp < splits; ++sp) acc += *reinterpret_cast<const VT*>(at(sp));
+    for (; sp < splits; ++sp) acc += *reinterpret_cast<const VT*>(p + sp * plane);
     if constexpr (V == 4) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) down_finish<T>(a, row, c0 + j, acc[j]);

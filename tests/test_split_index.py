@@ -24,6 +24,7 @@ def test_split_index_past_32_bits(tmp_path):
                          check=True).stdout.split()
     want = [s * m * n + r * n + c for s, m, n, r, c in cases]
     assert max(want) >= 1 << 32 and [int(v) for v in out] == want
-    # both sums go through it: no product of their own
+    # the store and both sums go through it, their steps from split to split included
     src = (ROOT / "complexity-framework_amd/csrc/trmoe_skinny.hip").read_text()
-    assert src.count("split_index(") == 3 and "plane" not in src
+    steps = src.count("const int64_t plane = split_index(1, a.M, a.N, 0, 0);")
+    assert steps == 2 and src.count("split_index(") == 3 + steps and "int plane" not in src
