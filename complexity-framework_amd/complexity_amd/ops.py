@@ -30,7 +30,7 @@ SKINNY_MAX_TOKENS = 128      # token counts the decode-shape kernels take
 # bf16 layers above this many tokens run on tiles, as prompts do: the decode-shape
 # kernels keep a wave's activations in registers, and at 65..128 tokens there is
 # room for half the waves only (16 layers of the 200M model in one graph: 65
-# tokens 414 -> 358 us, 102 448 -> 372, 128 466 -> 400)
+# tokens 413 -> 358 us, 80 422 -> 375, 102 445 -> 365, 128 461 -> 396)
 DECODE_BF16_TOKENS = 64
 EXPERT_GATE_UP_ALIGN = 128   # rows = 2 * round_up(W, 64)
 DOWN_ALIGN = 256             # rows = round_up(H, 256)

@@ -184,8 +184,12 @@ __global__ __launch_bounds__(64 * kQkvWaves) void k_decode_qkv(DecodeAttnArgs a)
 // else to hide latency behind: the first K/V rows are requested before the
 // position is known, and reductions stay on the vector ALU.  Against all heads
 // in every wave and one 128-position split: 14.2 us at 213 positions before.
-// 16 waves: 256 positions per workgroup cost one batch of loads, and up to that
-// length nothing crosses workgroups (10.6 us with 4 waves and four splits).
+// 16 waves and 256 positions a workgroup, against 4 waves and 64 positions: a
+// quarter of the partials to merge, which pays in long caches and costs in
+// short ones.  us, 14 heads on 2, 4 waves -> 16: one
+// sequence at position 213 of a cache of 256 9.2 -> 10.2, of 1024 10.3 -> 13.0, at
+// 1500 of 4096 17.9 -> 13.7, at 4000 of 4096 18.5 -> 13.3; 8 at 2100 of 2176 16.6 ->
+// 14.1; 16 at 4000 of 4096 24.0 -> 19.7.
 constexpr int kAttnWaves = 16;
 constexpr int kUnroll = 4;
 constexpr int kMaxSplits = 64;
@@ -486,8 +490,9 @@ __global__ __launch_bounds__(256, 2) void k_prefill_attn(PrefillAttnArgs a) {
 #pragma unroll
             for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[n][i]);
         mx = fmaxf(mx, __shfl_xor(mx, 32));
-        // the reference point moves only when the maximum has grown by 2^8: the
-        // weights stay below that in fp32, and the sums need no rescaling
+        // the reference point moves only when the maximum has grown by 2^8 (the
+        // conditional rescaling published with FlashAttention-4): the weights
+        // stay below that in fp32, and the sums need no rescaling
         if (__builtin_amdgcn_ballot_w64((mx - m) * c > 8.0f) != 0) {
             const float alpha = __builtin_amdgcn_exp2f((m - mx) * c);
             m = mx;

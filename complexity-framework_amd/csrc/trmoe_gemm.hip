@@ -189,10 +189,6 @@ __device__ __forceinline__ void gate_up_save(const GateUpArgs& a, const f32x16 (
     }
 }
 
-// ROUTED: the tile may hold dense-routed expert features (route gather and
-// per-token expert weights compiled in); the shared-feature launches leave
-// that code out.  SAVE: also write the raw gate|up outputs to a.gu (training
-// forwards), passed the launch's packed row count as gridDim-independent bound.
 // Tile of a ring launch of at most about one round, grid (row tiles, column
 // tiles).  Workgroups go to the 8 XCDs round-robin; XCD x takes a run of
 // consecutive tiles, down the columns of the longer side's split, so that its
@@ -213,6 +209,10 @@ __device__ __forceinline__ void ring_tile(uint32_t& mt, uint32_t& nt) {
     }
 }
 
+// gate|up + SwiGLU, one tile per workgroup.  ROUTED: the tile may hold
+// dense-routed expert features (route gather and per-token expert weights
+// compiled in); the shared-feature launches leave that code out.  SAVE: also
+// write the raw gate|up outputs to a.gu (training forwards).
 template <class Kind, bool FP8, class Shape, bool GROUPED = false, bool ROUTED = false, bool SAVE = false>
 __global__ __launch_bounds__(Shape::NT) void k_gate_up_swiglu(GateUpArgs a) {
     using T = typename Kind::T;

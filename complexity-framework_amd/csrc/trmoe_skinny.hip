@@ -14,7 +14,9 @@
 //   k_down_skinny      split-K: workgroup (8, 16 or 32 output columns, K chunk)
 //                      writes an fp32 partial [split][M][N] to the caller's
 //                      workspace
-//   k_down_reduce      sums the partials in split order (deterministic),
+//   k_down_reduce      sums the partials in split order (deterministic; calls
+//                      with split counters leave that to the last workgroup of
+//                      each column tile),
 //                      applies the row scales, the routed un-permute and the
 //                      residual, and stores the output
 #include "trmoe_common.h"
