@@ -4,8 +4,10 @@ what it refuses, can be looked at without a device."""
 
 import copy
 import ctypes
+import gc
 import io
 import pickle
+import weakref
 from types import SimpleNamespace
 
 import pytest
@@ -142,6 +144,21 @@ def test_changes_between_steps_are_seen(model, change):
     got = (dims.cache_length, dims.norm_eps, dims.qk_eps, dims.attn_scale)
     assert got == pytest.approx((model.k_cache[0].shape[2], b.input_layernorm.eps, b.self_attn.q_norm.eps,
                                  b.self_attn.scale))
+
+
+def test_a_decoder_let_go_after_a_step_is_gone(model):
+    m = copy.copy(model)
+    m.__dict__ = dict(model.__dict__)
+    m.decode_step(IDS[:, 0])
+    assert m._step_plan is not None and model._step_plan is None
+    gone = weakref.ref(m._step_plan)   # lives as long as the decoder's attributes
+    gc.collect()
+    gc.disable()
+    try:
+        del m
+        assert gone() is None   # no cycle that only the collector would find
+    finally:
+        gc.enable()
 
 
 def test_unequal_caches_take_the_blocks(model):
