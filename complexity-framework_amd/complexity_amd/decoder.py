@@ -240,19 +240,24 @@ def _pinned(block: nn.Module) -> bool:
     return getattr(config, "backend", None) is TRHashBackend.PYTORCH
 
 
+def _other_autocast() -> bool:
+    """Autocast to another type than the kernels': the projections come out in it."""
+    return torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") is not torch.bfloat16
+
+
 class _StepPlan:
     """The layers of a decode step as one native call takes them
     (``trmoe_decoder_step``): the pointers of every block's weights, packs and
     caches, with what they were read from.  ``current`` looks at all of it
     again before each step: module, parameter and cache objects, in-place
-    versions, storage, norm and attention constants, packs, routing.  Without
-    the plan a step spends about 100 us per layer in Python, against 30 us of
-    kernels."""
+    versions, storage, norm and attention constants, packs, routing, and what
+    ``_hip_attention`` asks of a decoder.  Without the plan a step spends about
+    100 us per layer in Python, against 30 us of kernels."""
 
-    def __init__(self, cfg: "TRGQAConfig"):
+    def __init__(self, cfg: "TRGQAConfig", device: torch.device):
         # nothing here refers back to the decoder: one that is let go gives its
         # memory back at once
-        self.cfg = cfg
+        self.cfg, self.device = cfg, device
         self.dims = ops.N.DecoderDims()
         self.layers = None
         self.engines = []   # (engine, config, strategy, E, W, pack entry, route table)
@@ -260,6 +265,8 @@ class _StepPlan:
         self.tensors = []   # (owner's dict, name, tensor, version, pointer)
         self.values = []    # (object's dict, name, value)
         self.caches = []    # (k or v, layer, tensor, pointer, shape)
+        self.stands = []    # (module that a kernel stands in for, its class, weight, shape)
+        self.attns = []
         self.keep = []      # what the pointers point into
 
     def _watch(self, owner: nn.Module, name: str) -> nn.Module:
@@ -282,18 +289,33 @@ class _StepPlan:
         self.caches.append((name == "k_cache", layer, t, t.data_ptr(), t.shape))
         return t
 
+    def _stand_in(self, mod: nn.Module) -> torch.Tensor:
+        t = self._weight(mod, "weight")
+        self.stands.append((mod, type(mod), t, t.shape))
+        return t
+
     @classmethod
     def build(cls, dec: "TRGQADecoder", device: torch.device) -> Optional["_StepPlan"]:
         """None when a block needs the general path: a replaced MLP half,
-        adapted or e4m3 weights, grouped experts, layers that differ in shape."""
+        adapted or e4m3 weights, grouped experts, layers that differ in shape.
+        For decoders that ``_hip_attention`` takes."""
+        with ops.decode_copies_together():
+            return cls._build(dec, device)
+
+    @classmethod
+    def _build(cls, dec: "TRGQADecoder", device: torch.device) -> Optional["_StepPlan"]:
         if dec.mlp_fn is not None or len(dec.k_cache) != len(dec.layers) or len(dec.v_cache) != len(dec.layers):
             return None
         cfg, rows, shapes = dec.cfg, [], set()
-        plan = cls(cfg)
+        plan = cls(cfg, device)
         plan._watch(dec, "layers")
+        first = dec.k_cache[0] if dec.k_cache else None
+        if first is not None and (first.ndim != 4 or first.shape[1::2] != (cfg.num_kv_heads, cfg.head_dim)):
+            return None
         for i, (name, block) in enumerate(dec.layers._modules.items()):
             plan.members.append((dec.layers._modules, name, block))
             attn, mlp = plan._watch(block, "self_attn"), plan._watch(block, "mlp")
+            plan.attns.append(attn)
             norm_in, norm_post = plan._watch(block, "input_layernorm"), plan._watch(block, "post_attention_layernorm")
             if not _plain(norm_post, RMSNorm, cfg.hidden_size) or type(mlp) is not TRHashEngine or mlp._fp8:
                 return None
@@ -323,9 +345,8 @@ class _StepPlan:
                         plan._value(attn.k_norm, "eps"), plan._value(attn, "scale")))
             caches = plan._cache(dec, "k_cache", i), plan._cache(dec, "v_cache", i)
             for t in caches:
-                if (t.dtype is not torch.bfloat16 or t.device != dec.k_cache[0].device or not t.is_contiguous()
-                        or t.ndim != 4 or t.shape != dec.k_cache[0].shape
-                        or t.shape[1:] != (cfg.num_kv_heads, t.shape[2], cfg.head_dim)):
+                if (t.dtype is not torch.bfloat16 or t.device != first.device or t.shape != first.shape
+                        or not t.is_contiguous()):
                     return None
             for n in ("k_proj", "q_proj", "v_proj"):
                 if "weight" not in plan._watch(attn, n)._parameters:
@@ -337,9 +358,8 @@ class _StepPlan:
             if None in frags:
                 return None   # a graph records, and nothing has built them before
             gu, dn = frags[0][0], frags[1][0]
-            ptrs = (plan._weight(norm_in, "weight"), kqv, plan._weight(plan._watch(attn, "q_norm"), "weight"),
-                    plan._weight(plan._watch(attn, "k_norm"), "weight"),
-                    plan._weight(plan._watch(attn, "o_proj"), "weight"), *caches, gu, dn, table)
+            ptrs = (plan._stand_in(norm_in), kqv, *(plan._stand_in(plan._watch(attn, n))
+                                                   for n in ("q_norm", "k_norm", "o_proj")), *caches, gu, dn, table)
             if any(t.data_ptr() % 16 for t in ptrs) or kqv.dtype is not torch.bfloat16:
                 return None
             plan.keep.append(ptrs)
@@ -362,8 +382,9 @@ class _StepPlan:
         plan.layers = (ops.N.DecoderLayer * len(rows))(*rows)
         return plan
 
-    def current(self, dec: "TRGQADecoder") -> bool:
-        if dec.mlp_fn is not None or len(dec.layers) != len(self.engines) or dec.cfg is not self.cfg:
+    def current(self, dec: "TRGQADecoder", device: torch.device) -> bool:
+        if (dec.mlp_fn is not None or len(dec.layers) != len(self.engines) or device != self.device
+                or dec.cfg is not self.cfg or dec.embed_tokens.weight.dtype is not torch.bfloat16 or _other_autocast()):
             return False
         for eng, cfg, strategy, E, W, entry, table in self.engines:
             if (eng._packed_norm is not entry or eng.config is not cfg or eng.routed_strategy != strategy
@@ -376,8 +397,21 @@ class _StepPlan:
         for is_k, i, t, p, shape in self.caches:
             if (k if is_k else v)[i] is not t or t.data_ptr() != p or t.shape != shape:
                 return False
-        return (all(d.get(n) is m for d, n, m in self.members) and all(d.get(n) == x for d, n, x in self.values)
-                and all(d.get(n) is t and t._version == v and t.data_ptr() == p for d, n, t, v, p in self.tensors))
+        bf16 = torch.bfloat16
+        for mod, cls, t, shape in self.stands:
+            if (type(mod) is not cls or mod._forward_hooks or mod._forward_pre_hooks or t.dtype is not bf16
+                    or t.shape != shape or not t.is_contiguous() or mod._parameters.get("bias") is not None):
+                return False
+        for attn in self.attns:
+            if type(attn) is not GQAttention:
+                return False
+        for d, n, m in self.members:
+            if d.get(n) is not m:
+                return False
+        for d, n, t, v, p in self.tensors:
+            if d.get(n) is not t or t._version != v or t.data_ptr() != p:
+                return False
+        return all(d.get(n) == x for d, n, x in self.values)
 
 
 # Replaces a block's MLP half (tests compare against a decoder whose MLPs run
@@ -460,8 +494,8 @@ class TRGQADecoder(nn.Module):
         if (device.type != "cuda" or self.embed_tokens.weight.dtype is not torch.bfloat16
                 or ops.attention_unsupported(cfg.hidden_size, cfg.num_heads, cfg.num_kv_heads, cfg.head_dim)):
             return False
-        if torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") is not torch.bfloat16:
-            return False   # the projections come out in another dtype
+        if _other_autocast():
+            return False
         for block in self.layers:
             m = block._modules
             attn = m["self_attn"]
@@ -556,7 +590,9 @@ class TRGQADecoder(nn.Module):
         L = self.k_cache[0].shape[2]
         dt = self.embed_tokens.weight.dtype
         pos = self._pos
-        if B <= ops.DECODE_ATTN_MAX_BATCH and self._hip_attention(ids.device):
+        if self._step_plan is not None and not self._step_plan.current(self, ids.device):
+            self._step_plan = None
+        if B <= ops.DECODE_ATTN_MAX_BATCH and (self._step_plan is not None or self._hip_attention(ids.device)):
             return self._decode_body_hip(ids, pos, L)
         cos_t, sin_t = self._rope_tables(L, ids.device, dt)
         cos = cos_t.index_select(0, pos)           # [1, D]
@@ -581,7 +617,7 @@ class TRGQADecoder(nn.Module):
         cos, sin = self._rope_tables32(L, ids.device)
         tok = ids.view(B, 1)
         h = self.embed_tokens(tok).view(B, -1)
-        if self._step_plan is None or not self._step_plan.current(self):
+        if self._step_plan is None:
             self._step_plan = _StepPlan.build(self, ids.device)
         if self._step_plan is not None and h.is_contiguous():
             ids = tok.view(B).to(torch.int64).contiguous()

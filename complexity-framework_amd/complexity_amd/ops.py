@@ -11,6 +11,7 @@ exception is raised.
 
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import functools
 import threading
@@ -979,6 +980,25 @@ def choose_strategy(shared_width: int, num_experts: int, expert_width: int, top_
 
 
 _COPY_LOCK = threading.Lock()
+_COPY_BATCH = threading.local()
+
+
+@contextlib.contextmanager
+def decode_copies_together():
+    """Decode copies that this thread builds inside are waited for once, at the
+    end, and only then found by other calls."""
+    if getattr(_COPY_BATCH, "built", None) is not None:
+        yield
+        return
+    _COPY_BATCH.built = built = []   # (stream, keep, copy)
+    try:
+        yield
+    finally:
+        _COPY_BATCH.built = None
+        for stream in {s for s, _, _ in built}:
+            stream.synchronize()
+        for _, keep, got in built:
+            keep(got)
 
 
 def _decode_copy(weight: torch.Tensor, have, build, keep):
@@ -994,9 +1014,12 @@ def _decode_copy(weight: torch.Tensor, have, build, keep):
     with _COPY_LOCK:
         got = have()
         if got is None:
-            got = build()
-            torch.cuda.current_stream(weight.device).synchronize()
-            keep(got)
+            got, stream = build(), torch.cuda.current_stream(weight.device)
+            if getattr(_COPY_BATCH, "built", None) is not None:
+                _COPY_BATCH.built.append((stream, keep, got))
+            else:
+                stream.synchronize()
+                keep(got)
     return got
 
 

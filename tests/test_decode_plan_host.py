@@ -4,6 +4,7 @@ what it refuses, can be looked at without a device."""
 
 import copy
 import ctypes
+import dataclasses
 import gc
 import io
 import pickle
@@ -146,6 +147,18 @@ def test_changes_between_steps_are_seen(model, change):
                                  b.self_attn.scale))
 
 
+class _OtherLinear(torch.nn.Linear):
+    pass
+
+
+class _OtherAttention(dec.GQAttention):
+    pass
+
+
+def _attn(m):
+    return m.layers[1].self_attn
+
+
 def test_a_decoder_let_go_after_a_step_is_gone(model):
     m = copy.copy(model)
     m.__dict__ = dict(model.__dict__)
@@ -159,6 +172,55 @@ def test_a_decoder_let_go_after_a_step_is_gone(model):
         assert gone() is None   # no cycle that only the collector would find
     finally:
         gc.enable()
+
+
+def test_another_configuration_is_seen(model, monkeypatch):
+    model.decode_step(IDS[:, 0])
+    monkeypatch.setattr(TRGQADecoder, "_hip_attention", _ask)
+    model.cfg = dataclasses.replace(CFG, vocab_size=32)
+    with pytest.raises(_Asked):
+        model.decode_step(IDS[:, 1])
+
+
+class _Asked(Exception):
+    pass
+
+
+def _ask(self, device):
+    raise _Asked
+
+
+@pytest.mark.parametrize("change", [
+    lambda m: _attn(m).q_norm.register_forward_hook(lambda *a: None),
+    lambda m: m.layers[0].input_layernorm.register_forward_pre_hook(lambda *a: None),
+    lambda m: setattr(_attn(m).o_proj, "bias", torch.nn.Parameter(torch.zeros(64, dtype=torch.bfloat16))),
+    lambda m: setattr(_attn(m).o_proj, "__class__", _OtherLinear),
+    lambda m: setattr(_attn(m), "__class__", _OtherAttention),
+    lambda m: setattr(_attn(m).o_proj.weight, "data", _attn(m).o_proj.weight.data.view(128, 64).t()),
+    lambda m: setattr(_attn(m).k_norm.weight, "data", _attn(m).k_norm.weight.data[:32]),
+    lambda m: m.embed_tokens.float(),
+    lambda m: setattr(m._step_plan, "device", torch.device("meta")),
+], ids=["hook", "pre_hook", "bias", "class", "attention_class", "strided", "narrowed", "embedding", "device"])
+def test_a_plan_stands_for_what_the_kernels_take(model, monkeypatch, change):
+    """A current plan is taken without asking ``_hip_attention`` again, which
+    is asked as soon as anything that it looks at has changed."""
+    model.decode_step(IDS[:, 0])
+    monkeypatch.setattr(TRGQADecoder, "_hip_attention", _ask)
+    model.decode_step(IDS[:, 1])
+    assert _names(model) == ["step"] * 2
+    change(model)
+    with pytest.raises(_Asked):
+        model.decode_step(IDS[:, 2])
+    assert _names(model) == ["step"] * 2 and model._step_plan is None
+
+
+def test_autocast_drops_the_plan(model, monkeypatch):
+    model.decode_step(IDS[:, 0])
+    monkeypatch.setattr(TRGQADecoder, "_hip_attention", _ask)
+    monkeypatch.setattr(torch, "is_autocast_enabled", lambda device: True)
+    monkeypatch.setattr(torch, "get_autocast_dtype", lambda device: torch.float16)
+    with pytest.raises(_Asked):
+        model.decode_step(IDS[:, 1])
 
 
 def test_unequal_caches_take_the_blocks(model):

@@ -117,3 +117,29 @@ def test_a_copy_is_built_once_by_several_threads(stream, monkeypatch):
     [t.start() for t in ts]
     [t.join() for t in ts]
     assert len(made) == 1 and all(g is made[0] for g in got)
+
+
+def test_copies_built_together_are_waited_for_once(stream):
+    a, b = _dense(), _dense()
+    with ops.decode_copies_together():
+        got = [p.fragments(n, H) for p in (a, b) for n in ("dense_gate_up", "dense_down")]
+        assert stream.did == ["pack"] * 4 and a.frag == b.frag == {}   # no other call finds them yet
+        with ops.decode_copies_together():
+            pass
+        assert a.frag == {}
+    assert stream.did == ["pack"] * 4 + ["synchronize"]
+    assert got == [p.frag[n] for p in (a, b) for n in ("dense_gate_up", "dense_down")]
+    with ops.decode_copies_together():
+        assert a.fragments("dense_down", H) is got[1]
+    assert len(stream.did) == 5
+
+
+def test_copies_of_a_failed_batch_are_kept_complete(stream):
+    p = _dense()
+    with pytest.raises(KeyError):
+        with ops.decode_copies_together():
+            p.fragments("dense_down", H)
+            raise KeyError
+    assert stream.did == ["pack", "synchronize"] and list(p.frag) == ["dense_down"]
+    p.fragments("dense_gate_up", H)   # alone again
+    assert stream.did == ["pack", "synchronize"] * 2
