@@ -414,12 +414,12 @@ __global__ __launch_bounds__(64 * NW) void k_down_skinny(DownArgs a, float* part
     for (int qi = threadIdx.x; qi < (int)a.M * kCols; qi += NT) {
         const int row = qi / kCols, col = (int)n0 + qi % kCols;
         if (col >= a.N) continue;
-        const float* p = part + split_index(0, a.M, a.N, row, col);
+        const uint32_t off = (uint32_t)(row * (int)a.N + col);   // M * N stays below 2^31
         float s = 0.f;
         for (int sp = 0; sp < splits; sp += 4) {
             float t[4];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) t[j] = load_dev(p + (sp + j < splits ? sp + j : splits - 1) * plane);
+            for (int j = 0; j < 4; ++j) t[j] = load_dev(part + (sp + j < splits ? sp + j : splits - 1) * plane + off);
 #pragma unroll
             for (int j = 0; j < 4; ++j) s += sp + j < splits ? t[j] : 0.f;
         }
@@ -441,7 +441,7 @@ __global__ __launch_bounds__(256) void k_down_reduce(DownArgs a, const float* pa
     if (idx >= (int)a.M * nv) return;
     const int row = idx / nv, c0 = (idx - row * nv) * V;
     const int64_t plane = split_index(1, a.M, a.N, 0, 0);
-    const float* p = part + split_index(0, a.M, a.N, row, c0);
+    const float* p = part + row * (int)a.N + c0;
     using VT = typename std::conditional<V == 4, f32x4, float>::type;
     VT acc{};
     int sp = 0;
